@@ -228,8 +228,14 @@ int nhw_create(const nhw_config *cfg, nhw_ctx **out) {
     nhw_destroy(c);
     return NHW_ENOMEM;
   }
+  // the zero fills of the allocations run on the null stream, with which the
+  // context's non-blocking stream is not ordered: they are waited for before
+  // anything is written on that stream (a fill of the scalars landing after
+  // nhw_set_time left dt = 0)
+  auto filled = [] { return hip_check(hipStreamSynchronize(nullptr), "nhw_create"); };
   rc = forcing_setup(c);
   if (!rc) rc = viscous_setup(c);
+  if (!rc) rc = filled();
   if (!rc) rc = turb_seed(c);
   if (rc) {
     nhw_destroy(c);
@@ -242,7 +248,8 @@ int nhw_create(const nhw_config *cfg, nhw_ctx **out) {
       return rc;
     }
   }
-  rc = nhw_set_time(c, 0.0, cfg->dt_ini, 0);
+  rc = filled();
+  if (!rc) rc = nhw_set_time(c, 0.0, cfg->dt_ini, 0);
   if (rc) {
     nhw_destroy(c);
     return rc;
