@@ -250,7 +250,6 @@ constexpr int kMgKMax = 16;      // largest Kglob the multigrid kernels take
 constexpr long kMgCoarseCols = 1024;  // coarsest level: at most this many columns ...
 constexpr int kMgCoarseSide = 64;     // ... and at most this many along either axis (a long,
                                       // narrow grid such as a one-row flume keeps coarsening)
-constexpr long kMgPairCols = 1L << 18;  // levels up to this many columns restrict on lane pairs
 struct MGLevel {
   int M = 0, N = 0, fx = 0, fy = 0;  // fx, fy: coarsening factors to the next level
   double dx = 0.0, dy = 0.0;
@@ -258,10 +257,17 @@ struct MGLevel {
   double *x = nullptr, *b = nullptr, *r = nullptr;  // x, b unused on level 0; r unused
   void *kc = nullptr;  // device table of per-sigma-level constants (LvlK), in the level's type
 };
-// a level restricted on lane pairs (k_resid22_pair): 2x2 coarsening, at most
-// kMgPairCols columns
-inline bool mg_pair_restrict(const MGLevel &lv) {
-  return lv.fx == 2 && lv.fy == 2 && (long)lv.M * lv.N <= kMgPairCols;
+// Column tiles of the multigrid kernels (k_mg_down, k_mg_up): 28 x 12 where a
+// launch has enough columns to fill the chip with them, 12 x 12 below, which
+// spreads a small level over more CUs.  Measured down + up at K = 10, FP64:
+// 16,384 columns 18.8 us in 12 x 12 tiles against 20.7, 65,536 columns 25.5
+// against 22.1, 1,048,576 columns 176 against 153.
+constexpr int kTileX = 28, kTileY = 12, kTileSX = 12, kTileSY = 12;
+constexpr long kMgBigCols = 1L << 15;
+inline bool mg_big_tiles(long columns) { return columns >= kMgBigCols; }
+template <int TX, int TY>
+inline unsigned mg_tiles(const MGLevel &lv) {
+  return (unsigned)(((lv.M + TX - 1) / TX) * ((lv.N + TY - 1) / TY));
 }
 struct MG {
   std::vector<MGLevel> lv;    // FP64 hierarchy (plain form), or FP64 level 0 only (mixed form)
@@ -295,7 +301,7 @@ enum KernelId {
   KID_RK_BLEND, KID_OMEGA_X, KID_OMEGA_Y, KID_OMEGA_COL, KID_DT, KID_MASK, KID_SOURCE,
   KID_ASSEMBLE, KID_SPMV_V, KID_SPMV_T, KID_RESID, KID_PREC_P, KID_PREC_S, KID_LINE_FACTOR,
   KID_KUPDATE, KID_KREDUCE, KID_KMISC, KID_COPY, KID_RHS, KID_MF_V, KID_MF_T, KID_MF_RESID,
-  KID_MG_SETUP, KID_MG_SMOOTH, KID_MG_RESID, KID_MG_COARSE, KID_MG_PROLONG, KID_KVEC, KID_WAVE_BC,
+  KID_MG_SETUP, KID_MG_DOWN, KID_MG_COARSE, KID_MG_UP, KID_KVEC, KID_WAVE_BC,
   KID_SPONGE, KID_DIFFUSION, KID_VISC_SIGMA, KID_VISC_SOLVE, KID_KEPS, KID_COUNT
 };
 

@@ -176,151 +176,63 @@ int mg_setup(nhw_ctx *c, std::vector<MGLevel> &lvs) {
 template int mg_setup<double>(nhw_ctx *, std::vector<MGLevel> &);
 template int mg_setup<float>(nhw_ctx *, std::vector<MGLevel> &);
 
-// one zebra half sweep; algorithmic bytes: b and x of the swept columns, x
-// of the other colour (unless zero), five column fields
-template <class V, int KM>
-static void zebra_k(nhw_ctx *c, const LvlC<V> &L, const G2<V> &G, const V *b, V *x, int color, bool zero,
-                    const int *stop, int kid) {
-  const long nth = (long)((L.M + 1) / 2) * L.N;
-  const double n = (double)L.MN * L.K;
-  Timed t(c, kid, sizeof(V) * ((zero ? 1.0 : 1.5) * n + 5.0 * L.MN));
-  if (zero)
-    hipLaunchKernelGGL((k_zebra<V, KM, true>), dim3(nb(nth)), dim3(kBSm), 0, c->stream, L, G, b, x, color, stop);
-  else
-    hipLaunchKernelGGL((k_zebra<V, KM, false>), dim3(nb(nth)), dim3(kBSm), 0, c->stream, L, G, b, x, color, stop);
-}
-
-template <class V>
-static void smooth(nhw_ctx *c, const LvlC<V> &L, const G2<V> &G, const V *b, V *x, int color, bool zero,
-                   const int *stop, int kid) {
-  if (L.K <= 4) zebra_k<V, 4>(c, L, G, b, x, color, zero, stop, kid);
-  else if (L.K <= 8) zebra_k<V, 8>(c, L, G, b, x, color, zero, stop, kid);
-  else if (L.K <= 12) zebra_k<V, 12>(c, L, G, b, x, color, zero, stop, kid);
-  else zebra_k<V, 16>(c, L, G, b, x, color, zero, stop, kid);
-}
-
 // the coarsest level: coarse_sweeps zebra pairs in one single-workgroup
 // launch; algorithmic bytes: b read and x written per half sweep pair
 template <class V>
 static void coarse(nhw_ctx *c, const LvlC<V> &L, const G2<V> &G, const V *b, V *x, const int *stop) {
   const int sw = c->mg.coarse_sweeps;
-  if (L.MN > kMgCoarseCols) {  // coarsening stopped early: separate sweeps
-    for (int s = 0; s < sw; ++s) {
-      smooth(c, L, G, b, x, 0, s == 0, stop, KID_MG_COARSE);
-      smooth(c, L, G, b, x, 1, false, stop, KID_MG_COARSE);
-    }
-    return;
-  }
   Timed t(c, KID_MG_COARSE, sizeof(V) * (2.0 * L.MN * L.K + 5.0 * L.MN));
-  if (L.K <= 4)
-    hipLaunchKernelGGL((k_coarse<V, 4>), dim3(1), dim3(kCoarseBS), 0, c->stream, L, G, b, x, sw, stop);
-  else if (L.K <= 8)
-    hipLaunchKernelGGL((k_coarse<V, 8>), dim3(1), dim3(kCoarseBS), 0, c->stream, L, G, b, x, sw, stop);
-  else if (L.K <= 12)
-    hipLaunchKernelGGL((k_coarse<V, 12>), dim3(1), dim3(kCoarseBS), 0, c->stream, L, G, b, x, sw, stop);
-  else
-    hipLaunchKernelGGL((k_coarse<V, 16>), dim3(1), dim3(kCoarseBS), 0, c->stream, L, G, b, x, sw, stop);
+  by_rows<kMgKMax>(L.K, [&](auto km) {
+    hipLaunchKernelGGL((k_coarse<V, decltype(km)::value>), dim3(1), dim3(kCoarseBS), 0, c->stream, L, G, b, x, sw,
+                       stop);
+  });
 }
 
-// the 2x2 restriction on lane pairs (k_resid22_pair), with ZSWEEP also the
-// next level's first half sweep
-template <class V, int KM>
-static void resid_pair_k(nhw_ctx *c, const LvlC<V> &L, const G2<V> &G, const V *x, const V *b,
-                         const LvlC<V> &Lc, const G2<V> &Gc, V *bc, V *xc, bool zsweep, const int *stop) {
-  const dim3 grid(nb(2 * Lc.MN));
-  if (zsweep)
-    hipLaunchKernelGGL((k_resid22_pair<V, KM, true>), grid, dim3(kBSm), 0, c->stream, L, G, x, b, Lc, Gc, bc, xc,
-                       stop);
-  else
-    hipLaunchKernelGGL((k_resid22_pair<V, KM, false>), grid, dim3(kBSm), 0, c->stream, L, G, x, b, Lc, Gc, bc, xc,
-                       stop);
+// algorithmic bytes of the two halves of a level's cycle: b, the five column
+// fields and the coarse right side; b, the fields, the coarse solution and x
+template <class V, int KM, int TX, int TY>
+static void down_t(nhw_ctx *c, const LvlC<V> &L, const MGLevel &lv, const MGLevel &q, const V *b, const int *stop) {
+  using T = MgTile<TX, TY>;
+  Timed t(c, KID_MG_DOWN, sizeof(V) * ((double)L.MN * L.K + (double)q.M * q.N * L.K + 5.0 * L.MN));
+  hipLaunchKernelGGL((k_mg_down<V, KM, TX, TY>), dim3(mg_tiles<TX, TY>(lv)), dim3(T::NT), T::lds(L.K, sizeof(V)), c->stream, L, g2<V>(lv),
+                     b, q.M, q.N, lv.fx, lv.fy, (V *)q.b, stop);
 }
-
+template <class V, int KM, int TX, int TY>
+static void up_t(nhw_ctx *c, const LvlC<V> &L, const MGLevel &lv, const MGLevel &q, const V *b, V *x,
+                 const int *stop) {
+  using T = MgTile<TX, TY>;
+  Timed t(c, KID_MG_UP, sizeof(V) * (2.0 * L.MN * L.K + (double)q.M * q.N * L.K + 5.0 * L.MN));
+  hipLaunchKernelGGL((k_mg_up<V, KM, TX, TY>), dim3(mg_tiles<TX, TY>(lv)), dim3(T::NT), T::lds(L.K, sizeof(V)), c->stream, L, g2<V>(lv), b,
+                     q.M, q.N, lv.fx, lv.fy, (const V *)q.x, x, stop);
+}
 // x = V(b): one V(1,1) cycle from a zero guess on level l; the coarsest
-// level (at most kMgCoarseCols columns) gets coarse_sweeps zebra sweeps.
-// With pre_done the first (zero-guess) half sweep has been done by the
-// restriction from the level above.
+// level (at most kMgCoarseCols columns) gets coarse_sweeps zebra sweeps
 template <class V>
-static void vcycle(nhw_ctx *c, const std::vector<MGLevel> &lvs, size_t l, const V *b, V *x, const int *stop,
-                   bool pre_done) {
+static void vcycle(nhw_ctx *c, const std::vector<MGLevel> &lvs, size_t l, const V *b, V *x, const int *stop) {
   const MGLevel &lv = lvs[l];
   const LvlC<V> L = make_lvl<V>(c, lv);
-  const G2<V> G = g2<V>(lv);
-  hipStream_t st = c->stream;
-  const double n = (double)L.MN * L.K;
   if (l + 1 == lvs.size()) {
-    coarse(c, L, G, b, x, stop);
+    coarse(c, L, g2<V>(lv), b, x, stop);
     return;
   }
-  const int kid = KID_MG_SMOOTH;  // one kernel at every level above the coarsest
-  if (!pre_done) smooth(c, L, G, b, x, 0, true, stop, kid);
-  smooth(c, L, G, b, x, 1, false, stop, kid);
   const MGLevel &q = lvs[l + 1];
-  const double nc = (double)q.M * q.N * L.K;
-  // the 2x2 path on lane pairs starts the next level's V-cycle unless that
-  // level is the coarsest (solved by k_coarse).  Up to kMgPairCols fine
-  // columns, where the launches are short, the pairs halve each thread's
-  // walk and the fused half sweep saves a launch; above it (measured at
-  // 1024 x 1024 x 10: 53 us against 38 + 10 us) the single-lane restriction
-  // and a separate half sweep move the bytes faster.
-  const bool even_only = lv.fx == 2 && lv.fy == 2;
-  const bool pair = mg_pair_restrict(lv);
-  const bool zsweep = pair && l + 2 < lvs.size();
-  {
-    // algorithmic bytes: x, b (the even half only on the 2x2 path), the coarse
-    // right side, five fields; with the coarse half sweep also its x and
-    // five coarse fields
-    Timed t(c, KID_MG_RESID, sizeof(V) * ((even_only ? 1.5 : 2.0) * n + nc + 5.0 * L.MN +
-                                          (zsweep ? 0.5 * nc + 5.0 * q.M * q.N : 0.0)));
-    const dim3 grid(nb((long)q.M * q.N));
-    if (pair) {
-      const LvlC<V> Lc = make_lvl<V>(c, q);
-      const G2<V> Gc = g2<V>(q);
-      if (L.K <= 4)
-        resid_pair_k<V, 4>(c, L, G, (const V *)x, b, Lc, Gc, (V *)q.b, (V *)q.x, zsweep, stop);
-      else if (L.K <= 8)
-        resid_pair_k<V, 8>(c, L, G, (const V *)x, b, Lc, Gc, (V *)q.b, (V *)q.x, zsweep, stop);
-      else if (L.K <= 12)
-        resid_pair_k<V, 12>(c, L, G, (const V *)x, b, Lc, Gc, (V *)q.b, (V *)q.x, zsweep, stop);
-      else
-        resid_pair_k<V, 16>(c, L, G, (const V *)x, b, Lc, Gc, (V *)q.b, (V *)q.x, zsweep, stop);
-    } else if (even_only) {
-      const dim3 g22(nb((long)q.M * q.N));
-      if (L.K <= 4)
-        hipLaunchKernelGGL((k_resid_restrict22<V, 4>), g22, dim3(kBSm), 0, st, L, G, (const V *)x, b, q.M, q.N,
-                           (V *)q.b, stop);
-      else if (L.K <= 8)
-        hipLaunchKernelGGL((k_resid_restrict22<V, 8>), g22, dim3(kBSm), 0, st, L, G, (const V *)x, b, q.M, q.N,
-                           (V *)q.b, stop);
-      else if (L.K <= 12)
-        hipLaunchKernelGGL((k_resid_restrict22<V, 12>), g22, dim3(kBSm), 0, st, L, G, (const V *)x, b, q.M, q.N,
-                           (V *)q.b, stop);
-      else
-        hipLaunchKernelGGL((k_resid_restrict22<V, 16>), g22, dim3(kBSm), 0, st, L, G, (const V *)x, b, q.M, q.N,
-                           (V *)q.b, stop);
-    } else if (L.K <= 4)
-      hipLaunchKernelGGL((k_resid_restrict<V, 4>), grid, dim3(kBSm), 0, st, L, G, (const V *)x, b, q.M, q.N, lv.fx,
-                         lv.fy, (V *)q.b, stop);
-    else if (L.K <= 8)
-      hipLaunchKernelGGL((k_resid_restrict<V, 8>), grid, dim3(kBSm), 0, st, L, G, (const V *)x, b, q.M, q.N, lv.fx,
-                         lv.fy, (V *)q.b, stop);
-    else
-      hipLaunchKernelGGL((k_resid_restrict<V, 16>), grid, dim3(kBSm), 0, st, L, G, (const V *)x, b, q.M, q.N,
-                         lv.fx, lv.fy, (V *)q.b, stop);
-  }
-  vcycle<V>(c, lvs, l + 1, (const V *)q.b, (V *)q.x, stop, zsweep);
-  {
-    Timed t(c, KID_MG_PROLONG, sizeof(V) * (n + nc));
-    hipLaunchKernelGGL(k_prolong_add<V>, dim3(nb((long)((lv.M + 1) / 2) * lv.N)), dim3(kBSm), 0, st, lv.M, lv.N,
-                       q.M, q.N, L.K, lv.fx, lv.fy, (const V *)q.x, x, stop);
-  }
-  smooth(c, L, G, b, x, 1, false, stop, kid);
-  smooth(c, L, G, b, x, 0, false, stop, kid);
+  const bool big = mg_big_tiles((long)lv.M * lv.N);
+  by_rows<kMgKMax>(L.K, [&](auto km) {
+    constexpr int KM = decltype(km)::value;
+    if (big) down_t<V, KM, kTileX, kTileY>(c, L, lv, q, b, stop);
+    else down_t<V, KM, kTileSX, kTileSY>(c, L, lv, q, b, stop);
+  });
+  vcycle<V>(c, lvs, l + 1, (const V *)q.b, (V *)q.x, stop);
+  by_rows<kMgKMax>(L.K, [&](auto km) {
+    constexpr int KM = decltype(km)::value;
+    if (big) up_t<V, KM, kTileX, kTileY>(c, L, lv, q, b, x, stop);
+    else up_t<V, KM, kTileSX, kTileSY>(c, L, lv, q, b, x, stop);
+  });
 }
 
 template <class V>
 void mg_apply(nhw_ctx *c, const std::vector<MGLevel> &lvs, const V *b, V *x, const int *stop) {
-  vcycle<V>(c, lvs, 0, b, x, stop, false);
+  vcycle<V>(c, lvs, 0, b, x, stop);
 }
 template void mg_apply<double>(nhw_ctx *, const std::vector<MGLevel> &, const double *, double *, const int *);
 template void mg_apply<float>(nhw_ctx *, const std::vector<MGLevel> &, const float *, float *, const int *);

@@ -11,13 +11,16 @@ namespace nhw {
 constexpr int kBSm = 256;
 
 // calls f(std::integral_constant<int, KM>) with the smallest row bucket KM in
-// {4, 8, ..., KMX} that holds K rows: kernels shared by members of different
-// K unroll only as far as each member needs (K is uniform per workgroup)
+// {4, 6, 8, 10, 12, 16} up to KMX that holds K rows: the column kernels keep a
+// column's rows in registers and unroll over the bucket, so a bucket that
+// fits saves the work on rows that are not there (K = 10 in 12 rows: 10 % of
+// k_mg_down and k_mg_up).  K is uniform per workgroup.
 template <int KMX, class F>
-__device__ __forceinline__ void by_rows(int K, F &&f) {
+__host__ __device__ __forceinline__ void by_rows(int K, F &&f) {
   if constexpr (KMX > 4) {
-    if (K <= KMX - 4) {
-      by_rows<KMX - 4>(K, f);
+    constexpr int below = KMX == 16 ? 12 : KMX - 2;
+    if (K <= below) {
+      by_rows<below>(K, f);
       return;
     }
   }
@@ -180,6 +183,22 @@ __device__ __forceinline__ ColC<V> col_consts(const G2<V> &G, const LvlC<V> &L, 
   q.FAy = (o - kym) * Aym - (o - kyp) * Ayp; q.FBy = (o - kym) * Bym - (o - kyp) * Byp;
   q.c0b = L.cxy - ((o - kxm) + (o - kxp)) * L.idx2 - ((o - kym) + (o - kyp)) * L.idy2;
   q.hxm = -kxm * L.idx2; q.hxp = -kxp * L.idx2; q.hym = -kym * L.idy2; q.hyp = -kyp * L.idy2;
+  return q;
+}
+
+// the constants of a column whose other columns are taken as zero: its own
+// fields and the folded sides' sums, whose neighbour is a zero halo entry
+template <class V>
+__device__ __forceinline__ ColC<V> col_consts_centre(const G2<V> &G, const LvlC<V> &L, int i, int j) {
+  const unsigned c = (unsigned)(i + 1) + (unsigned)G.ld * (unsigned)(j + 1);
+  ColC<V> q{};
+  q.axc = ldo(G.ax, c); q.bxc = ldo(G.bx, c); q.ayc = ldo(G.ay, c); q.byc = ldo(G.by, c);
+  const V rd = ldo(G.rd, c);
+  q.rd2 = rd * rd;
+  const V w = V(i == 0), e = V(i == L.M - 1), s = V(j == 0), n = V(j == L.N - 1);
+  q.FAx = (w - e) * q.axc; q.FBx = (w - e) * q.bxc;
+  q.FAy = (s - n) * q.ayc; q.FBy = (s - n) * q.byc;
+  q.c0b = L.cxy - (w + e) * L.idx2 - (s + n) * L.idy2;
   return q;
 }
 
@@ -450,31 +469,35 @@ __device__ __forceinline__ void thomas_fwd(const ZRow<V> &z, V r, V &cp, V &dp) 
   dp = fma(-z.c12, dp, r) * inv;
 }
 
-// z-line Gauss-Seidel update of column (i,j): solves its vertical tridiagonal
-// with the couplings to the other columns moved to the right side; with ZERO
-// the other columns are taken as zero.  Forward elimination runs as the rows
-// are formed (only the modified super-diagonal and right side are kept), then
-// back substitution stores the column.
-// back substitution of a column's eliminated tridiagonal into x at plane
-// offset off
+// back substitution of a column's eliminated tridiagonal, in registers: r
+// holds the eliminated right side on entry and the solution on return
+// (entries k >= K are not meaningful)
 template <class V, int KM>
-__device__ __forceinline__ void col_back(const LvlC<V> &L, const V (&cp)[KM], const V (&r)[KM], V *__restrict__ x,
-                                         unsigned off) {
+__device__ __forceinline__ void col_back(const LvlC<V> &L, const V (&cp)[KM], V (&r)[KM]) {
   const int K1 = L.K - 1;
   V xn = V(0);
 #pragma unroll
   for (int k = KM - 1; k >= 0; --k) {
     xn = k >= K1 ? r[k] : fma(-cp[k], xn, r[k]);
-    if (k < L.K) sto(plane(x, L, k), off, xn);
+    r[k] = xn;
   }
 }
 
-// the zero-guess solve of a column (the other columns taken as zero) with
-// its constants q and right side r in registers; r is overwritten, the
-// solution stored at plane offset off
+// a column's rows into x at plane offset off
 template <class V, int KM>
-__device__ __forceinline__ void zero_solve(const LvlC<V> &L, const ColC<V> &q, V (&r)[KM], V *__restrict__ x,
-                                           unsigned off) {
+__device__ __forceinline__ void store_rows(const LvlC<V> &L, const V (&r)[KM], V *__restrict__ x, unsigned off) {
+#pragma unroll
+  for (int k = 0; k < KM; ++k)
+    if (k < L.K) sto(plane(x, L, k), off, r[k]);
+}
+
+// z-line Gauss-Seidel update of a column, in registers: line_rows solves its
+// vertical tridiagonal with the couplings to its neighbours' values in x
+// moved to the right side r, zero_rows takes the other columns as zero.
+// Forward elimination runs as the rows are formed (only the modified
+// super-diagonal and right side are kept); r is overwritten by the solution.
+template <class V, int KM>
+__device__ __forceinline__ void zero_rows(const LvlC<V> &L, const ColC<V> &q, V (&r)[KM]) {
   V cp[KM];
   V cprev = V(0), dprev = V(0);
   const Pl<V> none{};
@@ -484,62 +507,28 @@ __device__ __forceinline__ void zero_solve(const LvlC<V> &L, const ColC<V> &q, V
     cp[k] = cprev;
     r[k] = dprev;
   }
-  col_back<V, KM>(L, cp, r, x, off);
+  col_back<V, KM>(L, cp, r);
 }
 
-// the Gauss-Seidel solve of a column against its neighbours' current values
-// in x; r is overwritten
+// plane stride of the neighbour values is Lx.MN (Lx differs from L only
+// there, for values staged in LDS)
 template <class V, int KM>
-__device__ __forceinline__ void line_solve(const LvlC<V> &L, const ColC<V> &q, const Nb &o, V (&r)[KM],
-                                           V *__restrict__ x) {
+__device__ __forceinline__ void line_rows(const LvlC<V> &Lx, const ColC<V> &q, const Nb &o, V (&r)[KM],
+                                          const V *__restrict__ x) {
   V cp[KM];
   V cprev = V(0), dprev = V(0);
   // the column's own values are the unknowns: only its neighbours are read
-  walk_col<V, KM>(L, q, o, x, [&](int k, const ZRow<V> &z, const Pl<V> &, const Pl<V> &, const Pl<V> &) {
+  walk_col<V, KM>(Lx, q, o, x, [&](int k, const ZRow<V> &z, const Pl<V> &, const Pl<V> &, const Pl<V> &) {
     thomas_fwd(z, r[k] - z.s, cprev, dprev);
     cp[k] = cprev;
     r[k] = dprev;
   });
-  col_back<V, KM>(L, cp, r, x, o.c);
-}
-
-// the zero-guess solve of column (i,j) with its right side r in registers
-template <class V, int KM>
-__device__ __forceinline__ void zero_col_solve(const LvlC<V> &L, const G2<V> &G, int i, int j, V (&r)[KM],
-                                               V *__restrict__ x) {
-  zero_solve<V, KM>(L, col_consts(G, L, i, j), r, x, (unsigned)zcol(i, j, L.M));
-}
-
-template <class V, int KM, bool ZERO>
-__device__ __forceinline__ void zebra_col(const LvlC<V> &L, const G2<V> &G, const V *__restrict__ b,
-                                          V *__restrict__ x, int i, int j) {
-  const Nb o = nbrs(L, i, j);
-  V r[KM];
-  load_rows<V, KM>(b, o.c, L, r);
-  if (ZERO) zero_solve<V, KM>(L, col_consts(G, L, i, j), r, x, o.c);
-  else line_solve<V, KM>(L, col_consts(G, L, i, j), o, r, x);
-}
-
-// zebra half sweep over the columns of one colour ((i+j) parity); columns of
-// one colour share no stencil entry, so they update in parallel
-template <class V, int KM, bool ZERO>
-__global__ __launch_bounds__(kBSm) void k_zebra(LvlC<V> L, G2<V> G, const V *__restrict__ b, V *__restrict__ x,
-                                                int color, const int *stop) {
-  if (stop[0]) return;
-  const int half = (L.M + 1) / 2;
-  long t = (long)xcd_block() * kBSm + threadIdx.x;
-  if (t >= (long)half * L.N) return;
-  const int j = (int)(t / half);
-  const int i = 2 * (int)(t % half) + ((j + color) & 1);
-  if (i >= L.M) return;
-  zebra_col<V, KM, ZERO>(L, G, b, x, i, j);
+  col_back<V, KM>(Lx, cp, r);
 }
 
 // The coarsest level (at most kMgCoarseCols columns) solved approximately
 // inside one workgroup: `sweeps` zebra pairs from a zero guess with x kept in
-// LDS between half sweeps, so the whole solve is one launch.  The arithmetic
-// is that of the zebra kernels: the result equals `sweeps` pairs of k_zebra
-// launches.
+// LDS between half sweeps, so the whole solve is one launch.
 // Each thread owns at most one column of each colour, whose offsets,
 // constants and right side it forms once, before the sweeps.
 constexpr int kCoarseBS = 512;
@@ -578,8 +567,9 @@ __device__ __forceinline__ void coarse_solve(const LvlC<V> &L, const G2<V> &G, c
         V r[KM];
 #pragma unroll
         for (int k = 0; k < KM; ++k) r[k] = rb[colour][k];
-        if (sw == 0 && colour == 0) zero_solve<V, KM>(L, q[colour], r, xs, o[colour].c);
-        else line_solve<V, KM>(L, q[colour], o[colour], r, xs);
+        if (sw == 0 && colour == 0) zero_rows<V, KM>(L, q[colour], r);
+        else line_rows<V, KM>(L, q[colour], o[colour], r, xs);
+        store_rows<V, KM>(L, r, xs, o[colour].c);
       }
       __syncthreads();
     }
@@ -593,136 +583,6 @@ __global__ __launch_bounds__(kCoarseBS) void k_coarse(LvlC<V> L, G2<V> G, const 
   if (stop[0]) return;
   __shared__ V xs[KM * kMgCoarseCols];
   coarse_solve<V, KM>(L, G, b, x, sweeps, xs);
-}
-
-// residual of a level restricted to the next coarser level's right side in
-// one pass: one thread per coarse column (I,J) walks its fx*fy fine columns
-// bottom to top, forms b - A x there and stores the block means
-// (block-average restriction) for every sigma level
-template <class V, int KM>
-__global__ __launch_bounds__(kBSm) void k_resid_restrict(LvlC<V> L, G2<V> G, const V *__restrict__ x,
-                                                         const V *__restrict__ b, int Mc, int Nc, int fx, int fy,
-                                                         V *__restrict__ bc, const int *stop) {
-  if (stop[0]) return;
-  long cc = (long)xcd_block() * kBSm + threadIdx.x;
-  const long MNc = (long)Mc * Nc;
-  if (cc >= MNc) return;
-  const int I = (int)(cc % Mc), J = (int)(cc / Mc);
-  V s[KM];
-#pragma unroll
-  for (int k = 0; k < KM; ++k) s[k] = V(0);
-  int cnt = 0;
-  for (int bb = 0; bb < fy; ++bb)
-    for (int a = 0; a < fx; ++a) {
-      const int i = I * fx + a, j = J * fy + bb;
-      if (i >= L.M || j >= L.N) continue;
-      const long col = (long)i + (long)L.M * j;
-      const ColC<V> q = col_consts(G, L, i, j);
-      const Nb o = nbrs(L, i, j);
-      V bv[KM];
-      load_rows<V, KM>(b, o.c, L, bv);
-      walk_col<V, KM>(L, q, o, x, [&](int k, const ZRow<V> &z, const Pl<V> &pv, const Pl<V> &cu, const Pl<V> &nx) {
-        s[k] += bv[k] - zrow_apply(z, pv, cu, nx);
-      });
-      ++cnt;
-    }
-  const V w = V(1) / (V)cnt;
-  const long zc = zcol(I, J, Mc);
-#pragma unroll
-  for (int k = 0; k < KM; ++k)
-    if (k < L.K) bc[zc + (long)k * MNc] = s[k] * w;
-}
-
-// The same for 2x2 coarsening right after the pre-smoothing, whose last
-// half sweep solved the odd columns ((i+j) odd) exactly: their residual is
-// zero, so only the two even columns (2I,2J) and (2I+1,2J+1) of coarse cell
-// (I,J) are formed.  One thread per coarse cell; the even columns of rows 2J
-// and 2J+1 sit at plane offsets 2J*M + I and (2J+1)*M + I in the zebra
-// layout, so neighbouring threads read neighbouring values.
-template <class V, int KM>
-__device__ __forceinline__ void resid22_body(const LvlC<V> &L, const G2<V> &G, const V *__restrict__ x,
-                                             const V *__restrict__ b, int Mc, int Nc, V *__restrict__ bc, long t) {
-  if (t >= (long)Mc * Nc) return;
-  const int I = (int)(t % Mc), J = (int)(t / Mc);
-  const int i0 = 2 * I, j0 = 2 * J;
-  const bool ix = i0 + 1 < L.M, jy = j0 + 1 < L.N;
-  const int cnt = 1 + ix + jy + (ix && jy);  // fine cells of the block
-  V s[KM];
-#pragma unroll
-  for (int k = 0; k < KM; ++k) s[k] = V(0);
-  for (int e = 0; e < (ix && jy ? 2 : 1); ++e) {
-    const int i = i0 + e, j = j0 + e;
-    const ColC<V> q = col_consts(G, L, i, j);
-    const Nb o = nbrs(L, i, j);
-    V bv[KM];
-    load_rows<V, KM>(b, o.c, L, bv);
-    walk_col<V, KM>(L, q, o, x, [&](int k, const ZRow<V> &z, const Pl<V> &pv, const Pl<V> &cu, const Pl<V> &nx) {
-      s[k] += bv[k] - zrow_apply(z, pv, cu, nx);
-    });
-  }
-  const long MNc = (long)Mc * Nc, zc = zcol(I, J, Mc);
-#pragma unroll
-  for (int k = 0; k < KM; ++k)
-    if (k < L.K) bc[zc + (long)k * MNc] = s[k] / (V)cnt;
-}
-
-template <class V, int KM>
-__global__ __launch_bounds__(kBSm) void k_resid_restrict22(LvlC<V> L, G2<V> G, const V *__restrict__ x,
-                                                           const V *__restrict__ b, int Mc, int Nc,
-                                                           V *__restrict__ bc, const int *stop) {
-  if (stop[0]) return;
-  resid22_body<V, KM>(L, G, x, b, Mc, Nc, bc, (long)xcd_block() * kBSm + threadIdx.x);
-}
-
-// resid22_body with the two fine columns of a coarse cell on neighbouring
-// lanes (lane pair t, t^1), whose partial sums meet through a shuffle: the
-// sum is formed as (0 + r0) + r1, the order of the single-lane loop, so the
-// coarse right side is bit-identical.  With ZSWEEP the lane pair then
-// starts the coarse level's V-cycle: the zero-guess half sweep over its
-// colour-0 columns needs nothing but each column's own right side, which is
-// in registers here, so those columns are solved (zero_col_solve) and the
-// coarse level skips its first half sweep.
-template <class V, int KM, bool ZSWEEP>
-__device__ __forceinline__ void resid22_pair_body(const LvlC<V> &L, const G2<V> &G, const V *__restrict__ x,
-                                                  const V *__restrict__ b, const LvlC<V> &Lc, const G2<V> &Gc,
-                                                  V *__restrict__ bc, V *__restrict__ xc, long t) {
-  const long cc = t >> 1;
-  const int e = (int)(t & 1);
-  if (cc >= Lc.MN) return;  // both lanes of a pair leave together
-  const int I = (int)(cc % Lc.M), J = (int)(cc / Lc.M);
-  const int i0 = 2 * I, j0 = 2 * J;
-  const bool ix = i0 + 1 < L.M, jy = j0 + 1 < L.N;
-  const int cnt = 1 + ix + jy + (ix && jy);  // fine cells of the block
-  const bool live = e == 0 || (ix && jy);    // a lane without a column walks (i0, j0) and adds zero
-  const int i = live ? i0 + e : i0, j = live ? j0 + e : j0;
-  V a[KM];
-  {
-    const ColC<V> q = col_consts(G, L, i, j);
-    const Nb o = nbrs(L, i, j);
-    V bv[KM];
-    load_rows<V, KM>(b, o.c, L, bv);
-    walk_col<V, KM>(L, q, o, x, [&](int k, const ZRow<V> &z, const Pl<V> &pv, const Pl<V> &cu, const Pl<V> &nx) {
-      const V r = bv[k] - zrow_apply(z, pv, cu, nx);
-      a[k] = e == 0 ? V(0) + r : (live ? r : V(0));
-    });
-  }
-  V s[KM];
-#pragma unroll
-  for (int k = 0; k < KM; ++k) s[k] = (a[k] + __shfl_xor(a[k], 1, 64)) / (V)cnt;
-  if (e != 0) return;
-  const unsigned zc = (unsigned)zcol(I, J, Lc.M);
-#pragma unroll
-  for (int k = 0; k < KM; ++k)
-    if (k < L.K) sto(plane(bc, Lc, k), zc, s[k]);
-  if (ZSWEEP && ((I + J) & 1) == 0) zero_col_solve<V, KM>(Lc, Gc, I, J, s, xc);
-}
-
-template <class V, int KM, bool ZSWEEP>
-__global__ __launch_bounds__(kBSm) void k_resid22_pair(LvlC<V> L, G2<V> G, const V *__restrict__ x,
-                                                       const V *__restrict__ b, LvlC<V> Lc, G2<V> Gc,
-                                                       V *__restrict__ bc, V *__restrict__ xc, const int *stop) {
-  if (stop[0]) return;
-  resid22_pair_body<V, KM, ZSWEEP>(L, G, x, b, Lc, Gc, bc, xc, (long)xcd_block() * kBSm + threadIdx.x);
 }
 
 // bilinear (cell-centred) prolongation weights and coarse plane offsets
@@ -754,36 +614,258 @@ __device__ __forceinline__ Pro<V> pro_at(int Mc, int Nc, int fx, int fy, int i, 
   return w;
 }
 
-// xf += P xc on the fine columns with (i+j) even.  The post-smoothing that
-// follows sweeps the odd columns first, which reads only even neighbours,
-// and then overwrites the even ones: the odd columns' corrections are never
-// read, so they are not formed.  One thread per even column (the first half
-// of each zebra row), walking its sigma levels.
+// ---------------------------------------------------------------------------
+// the two halves of a V-cycle on one level, a tile of columns per workgroup
+// ---------------------------------------------------------------------------
+// A zebra half sweep reads one colour and writes the other, so a V(1,1)
+// cycle done sweep by sweep streams the level's vectors through HBM six
+// times.  Here each workgroup takes a tile of TX x TY columns and recomputes
+// the halo its half sweeps need, so nothing but the level's right side b, the
+// coarse vectors and the final x moves:
+//
+//  k_mg_down: even columns from a zero guess (halo 2), odd columns against
+//    them (halo 1), then the residual of the tile's even columns averaged
+//    onto the coarse right side (the odd columns' residual is zero: they were
+//    just solved exactly).
+//  k_mg_up: the even columns' zero-guess solution formed again (cheaper than
+//    a store and a load of half a vector) plus the interpolated coarse
+//    correction (halo 2), odd columns against them (halo 1), even columns
+//    again.  The odd columns of the pre-smoothing are never read after the
+//    restriction (a half sweep solves for them from even values only), so
+//    they are not kept, and the result needs no copy of x.
+//
+// Each colour's values pass between the half sweeps through LDS.
+//
+// Bound on large levels by the FP64 instruction rate and the three waves a
+// SIMD that 150 VGPRs leave, on small ones by the elimination's chain of
+// dependent operations.  Measured, FP64, a level's whole cycle: 1024 x 1024 x
+// 10 162 us (sweep by sweep 195), 512 x 512 54 (68), 64 x 64 22 in two
+// launches (34 in six); a V-cycle of the 1024 x 1024 x 10 hierarchy 304 us
+// (385).
+template <int TX, int TY>
+struct MgTile {
+  static_assert(TX % 2 == 0 && TY % 2 == 0, "tiles start on even columns and whole coarse cells");
+  static constexpr int HW = TX / 2 + 2;       // slots of one colour in a row, halo 2
+  static constexpr int SL = HW * (TY + 4);    // slots of one colour
+  static constexpr int OW = HW - 1;           // odd columns of a row within halo 1
+  static constexpr int ODD = OW * (TY + 2);
+  static constexpr int EV = TX / 2 * TY;      // the tile's own columns of one colour
+  static constexpr int NT = (SL + 63) / 64 * 64;  // threads: one even column each
+  // LDS of both colours' values for K rows
+  static constexpr size_t lds(int K, size_t esize) { return 2 * (size_t)SL * K * esize; }
+};
+
+// column of a tile slot: row r (0 .. TY+3 from y0-2), position p in the row
+struct TCol {
+  int i, j, r, p;
+  bool in;  // inside the level
+};
 template <class V>
-__device__ __forceinline__ void prolong_col(int Mf, int Nf, int Mc, int Nc, int K, int fx, int fy,
-                                            const V *__restrict__ xc, V *__restrict__ xf, long t) {
-  const int half = (Mf + 1) / 2;
-  if (t >= (long)half * Nf) return;
-  const int p = (int)(t % half), j = (int)(t / half);
-  if (p >= (Mf + 1 - (j & 1)) >> 1) return;
-  const int i = 2 * p + (j & 1);
-  const Pro<V> w = pro_at<V>(Mc, Nc, fx, fy, i, j);
-  const long MNc = (long)Mc * Nc, MNf = (long)Mf * Nf;
-  const unsigned f = (unsigned)((long)j * Mf + p);
-  for (int k = 0; k < K; ++k) {
-    const V *xk = xc + MNc * k;
-    V *yk = xf + MNf * k;
-    const V v = w.wy0 * (w.wx0 * ldo(xk, w.c00) + w.wx1 * ldo(xk, w.c10)) +
-                w.wy1 * (w.wx0 * ldo(xk, w.c01) + w.wx1 * ldo(xk, w.c11));
-    sto(yk, f, ldo((const V *)yk, f) + v);
-  }
+__device__ __forceinline__ TCol tile_col(const LvlC<V> &L, int x0, int y0, int r, int p, int colour) {
+  TCol c;
+  c.r = r;
+  c.p = p;
+  c.i = x0 - 2 + 2 * p + ((r + colour) & 1);
+  c.j = y0 - 2 + r;
+  c.in = c.i >= 0 && c.i < L.M && c.j >= 0 && c.j < L.N;
+  return c;
+}
+// LDS slots of a slot's four neighbours, which are of the other colour
+template <int HW>
+__device__ __forceinline__ Nb tile_nbrs(int r, int p, int colour) {
+  Nb o;
+  const int s = r * HW + p, m = s - 1 + ((r + colour) & 1);
+  o.c = s;
+  o.xm = m;
+  o.xp = m + 1;
+  o.ym = s - HW;
+  o.yp = s + HW;
+  return o;
 }
 
+// right-side rows of a tile column, zeros outside the level
+template <class V, int KM>
+__device__ __forceinline__ void tile_rows(const V *__restrict__ b, const LvlC<V> &L, const TCol &c, V (&r)[KM]) {
+#pragma unroll
+  for (int k = 0; k < KM; ++k) r[k] = V(0);
+  if (c.in) load_rows<V, KM>(b, (unsigned)zcol(c.i, c.j, L.M), L, r);
+}
+template <class V, int KM, int SL>
+__device__ __forceinline__ void tile_put(const LvlC<V> &L, const V (&r)[KM], V *xs, int slot) {
+#pragma unroll
+  for (int k = 0; k < KM; ++k)
+    if (k < L.K) xs[k * SL + slot] = r[k];
+}
+
+// zero-guess solve of the thread's even column (tile slot threadIdx.x), in r
+template <class V, int KM>
+__device__ __forceinline__ void tile_even_zero(const LvlC<V> &L, const G2<V> &G, const V *__restrict__ b,
+                                               const TCol &c, V (&r)[KM]) {
+  tile_rows<V, KM>(b, L, c, r);
+  if (c.in) zero_rows<V, KM>(L, col_consts_centre(G, L, c.i, c.j), r);
+}
+
+// odd columns of the tile against the even ones in xe, into xo; solved()
+// sees the solution in r
+template <class V, int KM, int TX, int TY, class F>
+__device__ __forceinline__ void tile_odd(const LvlC<V> &L, const LvlC<V> &Ls, const G2<V> &G, const TCol &c,
+                                         bool live, V (&r)[KM], const V *xe, V *xo, F &&solved) {
+  using T = MgTile<TX, TY>;
+  __syncthreads();
+  if (live && c.in) {
+    line_rows<V, KM>(Ls, col_consts(G, L, c.i, c.j), tile_nbrs<T::HW>(c.r, c.p, 1), r, xe);
+    solved();
+  }
+  if (live) tile_put<V, KM, T::SL>(L, r, xo, c.r * T::HW + c.p);
+  __syncthreads();
+}
+
+// residual b - A x of a tile column from its own values xc and its
+// neighbours' xn, added to s
+template <class V, int KM, int HW>
+__device__ __forceinline__ void tile_resid(const LvlC<V> &L, const LvlC<V> &Ls, const G2<V> &G,
+                                           const V *__restrict__ b, int i, int j, int x0, int y0, int colour,
+                                           const V *xc, const V *xn, V (&s)[KM]) {
+  const int r = j - y0 + 2, p = (i - x0 + 2 - ((r + colour) & 1)) >> 1;
+  const Nb o = tile_nbrs<HW>(r, p, colour);
+  V bv[KM];
+  load_rows<V, KM>(b, (unsigned)zcol(i, j, L.M), L, bv);
+  const int K1 = L.K - 1, SL = (int)Ls.MN;
+  V below = xc[o.c], at = below, above = xc[min(1, K1) * SL + o.c];
+  walk_col<V, KM>(Ls, col_consts(G, L, i, j), o, xn,
+                  [&](int k, const ZRow<V> &z, const Pl<V> &, const Pl<V> &, const Pl<V> &) {
+    s[k] += bv[k] - fma(z.c0, at, fma(z.c5, above, fma(z.c12, below, z.s)));
+    below = at;
+    at = above;
+    above = xc[min(k + 2, K1) * SL + o.c];
+  });
+}
+
+template <class V, int KM, int TX, int TY>
+__device__ __forceinline__ void mg_down_body(const LvlC<V> &L, const G2<V> &G, const V *__restrict__ b, int Mc,
+                                             int Nc, int fx, int fy, V *__restrict__ bc, long tile, V *xs) {
+  using T = MgTile<TX, TY>;
+  const int ntx = (L.M + TX - 1) / TX;
+  const int ty = (int)(tile / ntx), x0 = (int)(tile - (long)ty * ntx) * TX, y0 = ty * TY;
+  const int t = threadIdx.x;
+  LvlC<V> Ls = L;
+  Ls.MN = T::SL;
+  V *xe = xs, *xo = xs + (long)T::SL * L.K;
+  // the odd column's right side is requested before the even columns' work
+  const bool olive = t < T::ODD;
+  const int orow = olive ? 1 + t / T::OW : 1;
+  const TCol oc = tile_col(L, x0, y0, orow, (olive ? t % T::OW : 0) + (orow & 1), 1);
+  V ro[KM];
+  {
+    V re[KM];
+    const TCol ec = tile_col(L, x0, y0, t / T::HW, t % T::HW, 0);
+    tile_even_zero<V, KM>(L, G, b, ec, re);
+    tile_rows<V, KM>(b, L, oc, ro);
+    if (t < T::SL) tile_put<V, KM, T::SL>(L, re, xe, t);
+  }
+  tile_odd<V, KM, TX, TY>(L, Ls, G, oc, olive, ro, xe, xo, [] {});
+  // 2x2 coarse cells: their two even columns on neighbouring lanes, whose
+  // residuals meet through a shuffle.  Cells of a level coarsened along one
+  // axis: both columns on one lane.
+  const bool two = fx == 2 && fy == 2;
+  const int c = two ? t >> 1 : t, e = two ? t & 1 : 0;
+  const int cw = TX / fx, cx = c % cw, cy = c / cw;
+  const int I = x0 / fx + cx, J = y0 / fy + cy, i0 = I * fx, j0 = J * fy;
+  const bool cell = t < T::EV && i0 < L.M && j0 < L.N;
+  V s[KM];
+#pragma unroll
+  for (int k = 0; k < KM; ++k) s[k] = V(0);
+  for (int a = 0; a < (two ? 1 : 2); ++a) {
+    const int i = two ? i0 + e : fx == 2 ? i0 + a : i0, j = two ? j0 + e : fy == 2 ? j0 + a : j0;
+    const int odd = (i + j) & 1;
+    if (cell && i < L.M && j < L.N)
+      tile_resid<V, KM, T::HW>(L, Ls, G, b, i, j, x0, y0, odd, odd ? xo : xe, odd ? xe : xo, s);
+  }
+  const int cnt = (min(i0 + fx, L.M) - i0) * (min(j0 + fy, L.N) - j0);  // fine cells of the block
+  const V w = V(1) / (V)cnt;
+  if (two)
+#pragma unroll
+    for (int k = 0; k < KM; ++k) s[k] += __shfl_xor(s[k], 1, 64);
+  if (!cell || e != 0) return;
+  const long MNc = (long)Mc * Nc;
+  const unsigned zc = (unsigned)zcol(I, J, Mc);
+#pragma unroll
+  for (int k = 0; k < KM; ++k)
+    if (k < L.K) sto(bc + (long)k * MNc, zc, s[k] * w);
+}
+
+template <class V, int KM, int TX, int TY>
+__device__ __forceinline__ void mg_up_body(const LvlC<V> &L, const G2<V> &G, const V *__restrict__ b, int Mc, int Nc,
+                                           int fx, int fy, const V *__restrict__ xc, V *__restrict__ x, long tile,
+                                           V *xs) {
+  using T = MgTile<TX, TY>;
+  const int ntx = (L.M + TX - 1) / TX;
+  const int ty = (int)(tile / ntx), x0 = (int)(tile - (long)ty * ntx) * TX, y0 = ty * TY;
+  const int t = threadIdx.x;
+  LvlC<V> Ls = L;
+  Ls.MN = T::SL;
+  V *xe = xs, *xo = xs + (long)T::SL * L.K;
+  const bool olive = t < T::ODD;
+  const int orow = olive ? 1 + t / T::OW : 1;
+  const TCol oc = tile_col(L, x0, y0, orow, (olive ? t % T::OW : 0) + (orow & 1), 1);
+  V ro[KM];
+  {
+    V re[KM];
+    const TCol ec = tile_col(L, x0, y0, t / T::HW, t % T::HW, 0);
+    tile_even_zero<V, KM>(L, G, b, ec, re);
+    if (ec.in) {
+      const Pro<V> w = pro_at<V>(Mc, Nc, fx, fy, ec.i, ec.j);
+      const long MNc = (long)Mc * Nc;
+      const int K1 = L.K - 1;
+#pragma unroll
+      for (int k = 0; k < KM; ++k) {
+        const V *xk = xc + MNc * min(k, K1);
+        re[k] += w.wy0 * (w.wx0 * ldo(xk, w.c00) + w.wx1 * ldo(xk, w.c10)) +
+                 w.wy1 * (w.wx0 * ldo(xk, w.c01) + w.wx1 * ldo(xk, w.c11));
+      }
+    }
+    tile_rows<V, KM>(b, L, oc, ro);
+    if (t < T::SL) tile_put<V, KM, T::SL>(L, re, xe, t);
+  }
+  // the tile's own columns of either colour are stored; the halo's are
+  // their own tile's to store
+  tile_odd<V, KM, TX, TY>(L, Ls, G, oc, olive, ro, xe, xo, [&] {
+    if (oc.i >= x0 && oc.i < x0 + TX && oc.j >= y0 && oc.j < y0 + TY)
+      store_rows<V, KM>(L, ro, x, (unsigned)zcol(oc.i, oc.j, L.M));
+  });
+  if (t >= T::EV) return;
+  const TCol c = tile_col(L, x0, y0, 2 + t / (TX / 2), 1 + t % (TX / 2), 0);
+  if (!c.in) return;
+  const unsigned zc = (unsigned)zcol(c.i, c.j, L.M);
+  V r[KM];
+  load_rows<V, KM>(b, zc, L, r);
+  line_rows<V, KM>(Ls, col_consts(G, L, c.i, c.j), tile_nbrs<T::HW>(c.r, c.p, 0), r, (const V *)xo);
+  store_rows<V, KM>(L, r, x, zc);
+}
+
+// the workgroup's dynamic LDS
 template <class V>
-__global__ void k_prolong_add(int Mf, int Nf, int Mc, int Nc, int K, int fx, int fy, const V *__restrict__ xc,
-                              V *__restrict__ xf, const int *stop) {
+__device__ __forceinline__ V *tile_lds() {
+  extern __shared__ __align__(16) unsigned char mg_tile_lds[];
+  return (V *)mg_tile_lds;
+}
+
+template <class V, int KM, int TX, int TY>
+__global__ __launch_bounds__((MgTile<TX, TY>::NT)) void k_mg_down(LvlC<V> L, G2<V> G, const V *__restrict__ b, int Mc,
+                                                                int Nc, int fx, int fy, V *__restrict__ bc,
+                                                                const int *stop) {
   if (stop[0]) return;
-  prolong_col<V>(Mf, Nf, Mc, Nc, K, fx, fy, xc, xf, (long)xcd_block() * blockDim.x + threadIdx.x);
+  V *xs = tile_lds<V>();
+  mg_down_body<V, KM, TX, TY>(L, G, b, Mc, Nc, fx, fy, bc, (long)xcd_block(), xs);
+}
+
+template <class V, int KM, int TX, int TY>
+__global__ __launch_bounds__((MgTile<TX, TY>::NT)) void k_mg_up(LvlC<V> L, G2<V> G, const V *__restrict__ b, int Mc,
+                                                              int Nc, int fx, int fy, const V *__restrict__ xc,
+                                                              V *__restrict__ x, const int *stop) {
+  if (stop[0]) return;
+  V *xs = tile_lds<V>();
+  mg_up_body<V, KM, TX, TY>(L, G, b, Mc, Nc, fx, fy, xc, x, (long)xcd_block(), xs);
 }
 
 }  // namespace nhw

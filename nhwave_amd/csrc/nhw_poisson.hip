@@ -981,23 +981,6 @@ __device__ __forceinline__ R *lvl_x(const BScn<R> &S, int l, int vout) {
   return l == 0 ? bvec(S, vout) : S.lx[l];
 }
 
-template <class R, int KM, bool ZERO>
-__global__ __launch_bounds__(256) void kb_zebra(BTab<R> T, int l, int color, int vin, int vout) {
-  const BPos b = bfind(T);
-  const BScn<R> &S = T.scn[b.s];
-  if (S.flag[0]) return;
-  const LvlC<R> &L = S.L[l];
-  const int half = (L.M + 1) / 2;
-  const long t = b.b * blockDim.x + threadIdx.x;
-  if (t >= (long)half * L.N) return;
-  const int j = (int)(t / half);
-  const int i = 2 * (int)(t % half) + ((j + color) & 1);
-  if (i >= L.M) return;
-  by_rows<KM>(L.K, [&](auto km) {
-    zebra_col<R, decltype(km)::value, ZERO>(L, S.G[l], lvl_b(S, l, vin), lvl_x(S, l, vout), i, j);
-  });
-}
-
 // the coarsest level of each member in one workgroup (coarse_solve)
 template <class R, int KM>
 __global__ __launch_bounds__(kCoarseBS) void kb_coarse(BTab<R> T, int l, int vin, int vout, int sweeps) {
@@ -1010,87 +993,30 @@ __global__ __launch_bounds__(kCoarseBS) void kb_coarse(BTab<R> T, int l, int vin
   });
 }
 
-// fused residual + 2x2 restriction of level l into the right side of l+1
-// (resid22_body: one thread per coarse cell)
-template <class R, int KM>
-__global__ __launch_bounds__(256) void kb_resid_restrict22(BTab<R> T, int l, int vin, int vout) {
+// the two halves of a level's V-cycle, one tile of a member's columns per
+// workgroup (mg_down_body, mg_up_body)
+template <class R, int KM, int TX, int TY>
+__global__ __launch_bounds__((MgTile<TX, TY>::NT)) void kb_mg_down(BTab<R> T, int l, int vin) {
   const BPos bp = bfind(T);
   const BScn<R> &S = T.scn[bp.s];
   if (S.flag[0]) return;
-  const LvlC<R> &L = S.L[l];
-  by_rows<KM>(L.K, [&](auto km) {
-    resid22_body<R, decltype(km)::value>(L, S.G[l], lvl_x(S, l, vout), lvl_b(S, l, vin), S.L[l + 1].M,
-                                         S.L[l + 1].N, S.lb[l + 1], bp.b * blockDim.x + threadIdx.x);
+  R *xs = tile_lds<R>();
+  by_rows<KM>(S.L[l].K, [&](auto km) {
+    mg_down_body<R, decltype(km)::value, TX, TY>(S.L[l], S.G[l], lvl_b(S, l, vin), S.L[l + 1].M, S.L[l + 1].N,
+                                                 S.lfx[l], S.lfy[l], S.lb[l + 1], bp.b, xs);
   });
 }
 
-// the same on lane pairs (resid22_pair_body), with ZSWEEP starting level
-// l+1's V-cycle
-template <class R, int KM, bool ZSWEEP>
-__global__ __launch_bounds__(256) void kb_resid22_pair(BTab<R> T, int l, int vin, int vout) {
+template <class R, int KM, int TX, int TY>
+__global__ __launch_bounds__((MgTile<TX, TY>::NT)) void kb_mg_up(BTab<R> T, int l, int vin, int vout) {
   const BPos bp = bfind(T);
   const BScn<R> &S = T.scn[bp.s];
   if (S.flag[0]) return;
-  const LvlC<R> &L = S.L[l];
-  by_rows<KM>(L.K, [&](auto km) {
-    resid22_pair_body<R, decltype(km)::value, ZSWEEP>(L, S.G[l], lvl_x(S, l, vout), lvl_b(S, l, vin), S.L[l + 1],
-                                                       S.G[l + 1], S.lb[l + 1], S.lx[l + 1],
-                                                       bp.b * blockDim.x + threadIdx.x);
+  R *xs = tile_lds<R>();
+  by_rows<KM>(S.L[l].K, [&](auto km) {
+    mg_up_body<R, decltype(km)::value, TX, TY>(S.L[l], S.G[l], lvl_b(S, l, vin), S.L[l + 1].M, S.L[l + 1].N, S.lfx[l],
+                                               S.lfy[l], (const R *)S.lx[l + 1], lvl_x(S, l, vout), bp.b, xs);
   });
-}
-
-// the same for levels not coarsened 2x2: one thread per coarse column
-template <class R, int KM>
-__global__ __launch_bounds__(256) void kb_resid_restrict(BTab<R> T, int l, int vin, int vout) {
-  const BPos bp = bfind(T);
-  const BScn<R> &S = T.scn[bp.s];
-  if (S.flag[0]) return;
-  const LvlC<R> &L = S.L[l];
-  const G2<R> &G = S.G[l];
-  const R *x = lvl_x(S, l, vout);
-  const R *b = lvl_b(S, l, vin);
-  const int Mc = S.L[l + 1].M, Nc = S.L[l + 1].N, fx = S.lfx[l], fy = S.lfy[l];
-  const long cc = bp.b * blockDim.x + threadIdx.x;
-  const long MNc = (long)Mc * Nc;
-  if (cc >= MNc) return;
-  const int I = (int)(cc % Mc), J = (int)(cc / Mc);
-  by_rows<KM>(L.K, [&](auto km) {
-    constexpr int KR = decltype(km)::value;
-    R s[KR];
-#pragma unroll
-    for (int k = 0; k < KR; ++k) s[k] = R(0);
-    int cnt = 0;
-    for (int bb = 0; bb < fy; ++bb)
-      for (int a = 0; a < fx; ++a) {
-        const int i = I * fx + a, j = J * fy + bb;
-        if (i >= L.M || j >= L.N) continue;
-        const ColC<R> q = col_consts(G, L, i, j);
-        const Nb o = nbrs(L, i, j);
-        R bv[KR];
-        load_rows<R, KR>(b, o.c, L, bv);
-        walk_col<R, KR>(L, q, o, x, [&](int k, const ZRow<R> &z, const Pl<R> &pv, const Pl<R> &cu, const Pl<R> &nx) {
-          s[k] += bv[k] - zrow_apply(z, pv, cu, nx);
-        });
-        ++cnt;
-      }
-    R *bc = S.lb[l + 1];
-    const long zc = zcol(I, J, Mc);
-#pragma unroll
-    for (int k = 0; k < KR; ++k)
-      if (k < L.K) bc[zc + (long)k * MNc] = s[k] / (R)cnt;
-  });
-}
-
-// xf += P xc on the even (zebra colour 0) columns of level l (see
-// k_prolong_add)
-template <class R>
-__global__ __launch_bounds__(256) void kb_prolong(BTab<R> T, int l, int vout) {
-  const BPos bp = bfind(T);
-  const BScn<R> &S = T.scn[bp.s];
-  if (S.flag[0]) return;
-  const LvlC<R> &L = S.L[l];
-  prolong_col<R>(L.M, L.N, S.L[l + 1].M, S.L[l + 1].N, L.K, S.lfx[l], S.lfy[l], S.lx[l + 1], lvl_x(S, l, vout),
-                 bp.b * blockDim.x + threadIdx.x);
 }
 
 template <class R>
@@ -1146,48 +1072,35 @@ static BTab<R> pbtab(Batch *B, const BShape &S) {
 }
 
 // launch of a batched kernel instantiated at R (the batch's storage type)
-#define PBL(kid, bytes, kern, shape, ...)                                                             \
+#define PBL(kid, bytes, kern, shape, ...) PBLS(kid, bytes, kern, shape, 0, ##__VA_ARGS__)
+// with `lds` bytes of dynamic LDS a workgroup
+#define PBLS(kid, bytes, kern, shape, lds, ...)                                                        \
   do {                                                                                                 \
     const BShape &S_ = (shape);                                                                        \
     if (S_.nblk > 0) {                                                                                 \
       Timed _t(B->lead, kid, bytes);                                                                   \
-      hipLaunchKernelGGL(HIP_KERNEL_NAME(kern), dim3(S_.nblk), dim3(S_.bs), 0, B->lead->stream,        \
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(kern), dim3(S_.nblk), dim3(S_.bs), lds, B->lead->stream,      \
                          pbtab<R>(B, S_), ##__VA_ARGS__);                                              \
     }                                                                                                  \
   } while (0)
 
 static bool has_shape(Batch *B, const std::string &k) { return B->shapes.count(k) > 0; }
 
-template <class R, int KM>
-static void bzebra(Batch *B, const std::string &key, int l, int color, bool zero, int vin, int vout) {
-  if (!has_shape(B, key)) return;
-  const int kid = KID_MG_SMOOTH;  // one kernel at every level above the coarsest
-  if (zero) PBL(kid, 0.0, (kb_zebra<R, KM, true>), bshape(B, key), l, color, vin, vout);
-  else PBL(kid, 0.0, (kb_zebra<R, KM, false>), bshape(B, key), l, color, vin, vout);
-}
-
 // batched V(1,1) cycle on level l: members whose coarsest level is l sweep
 // there; the others go down
 template <class R, int KM>
 static void bvcycle(Batch *B, int l, int vin, int vout) {
-  const std::string co = "k:co" + std::to_string(l), zb = "k:zb" + std::to_string(l);
+  const std::string L = std::to_string(l), co = "k:co" + L, tb = "k:tb" + L, ts = "k:ts" + L;
   if (has_shape(B, co))
     PBL(KID_MG_COARSE, 0.0, (kb_coarse<R, KM>), bshape(B, co), l, vin, vout, B->lead->mg.coarse_sweeps);
-  if (!has_shape(B, zb)) return;
-  const std::string L = std::to_string(l);
-  // the zero-guess half sweep of the members whose restriction from level
-  // l-1 has not done it
-  bzebra<R, KM>(B, "k:zz" + L, l, 0, true, vin, vout);
-  bzebra<R, KM>(B, zb, l, 1, false, vin, vout);
-  const std::string rr = "k:rr" + L, rg = "k:rg" + L, rp = "k:rp" + L, rz = "k:rz" + L;
-  if (has_shape(B, rr)) PBL(KID_MG_RESID, 0.0, (kb_resid_restrict22<R, KM>), bshape(B, rr), l, vin, vout);
-  if (has_shape(B, rp)) PBL(KID_MG_RESID, 0.0, (kb_resid22_pair<R, KM, false>), bshape(B, rp), l, vin, vout);
-  if (has_shape(B, rz)) PBL(KID_MG_RESID, 0.0, (kb_resid22_pair<R, KM, true>), bshape(B, rz), l, vin, vout);
-  if (has_shape(B, rg)) PBL(KID_MG_RESID, 0.0, (kb_resid_restrict<R, KM>), bshape(B, rg), l, vin, vout);
+  if (!has_shape(B, tb) && !has_shape(B, ts)) return;
+  const size_t lb = MgTile<kTileX, kTileY>::lds(B->kmax, sizeof(R));
+  const size_t ls = MgTile<kTileSX, kTileSY>::lds(B->kmax, sizeof(R));
+  PBLS(KID_MG_DOWN, 0.0, (kb_mg_down<R, KM, kTileX, kTileY>), bshape(B, tb), lb, l, vin);
+  PBLS(KID_MG_DOWN, 0.0, (kb_mg_down<R, KM, kTileSX, kTileSY>), bshape(B, ts), ls, l, vin);
   bvcycle<R, KM>(B, l + 1, 0, 0);
-  PBL(KID_MG_PROLONG, 0.0, kb_prolong<R>, bshape(B, "k:pr" + std::to_string(l)), l, vout);
-  bzebra<R, KM>(B, zb, l, 1, false, vin, vout);
-  bzebra<R, KM>(B, zb, l, 0, false, vin, vout);
+  PBLS(KID_MG_UP, 0.0, (kb_mg_up<R, KM, kTileX, kTileY>), bshape(B, tb), lb, l, vin, vout);
+  PBLS(KID_MG_UP, 0.0, (kb_mg_up<R, KM, kTileSX, kTileSY>), bshape(B, ts), ls, l, vin, vout);
 }
 
 // reads every member's Krylov flag; returns how many are still running
@@ -1326,17 +1239,13 @@ static int batch_poisson_t(Batch *B) {
   return 0;
 }
 
-int batch_poisson(Batch *B) {
-  if (B->mixed) {
-    if (B->kmax <= 4) return batch_poisson_t<float, 4>(B);
-    if (B->kmax <= 8) return batch_poisson_t<float, 8>(B);
-    if (B->kmax <= 12) return batch_poisson_t<float, 12>(B);
-    return batch_poisson_t<float, 16>(B);
-  }
-  if (B->kmax <= 4) return batch_poisson_t<double, 4>(B);
-  if (B->kmax <= 8) return batch_poisson_t<double, 8>(B);
-  if (B->kmax <= 12) return batch_poisson_t<double, 12>(B);
-  return batch_poisson_t<double, 16>(B);
+template <class R>
+static int batch_poisson_r(Batch *B) {
+  if (B->kmax <= 4) return batch_poisson_t<R, 4>(B);
+  if (B->kmax <= 8) return batch_poisson_t<R, 8>(B);
+  if (B->kmax <= 12) return batch_poisson_t<R, 12>(B);
+  return batch_poisson_t<R, 16>(B);
 }
+int batch_poisson(Batch *B) { return B->mixed ? batch_poisson_r<float>(B) : batch_poisson_r<double>(B); }
 
 }  // namespace nhw

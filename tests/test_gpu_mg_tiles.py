@@ -1,0 +1,51 @@
+"""The multigrid cycle's column tiles (28 x 12 in launches of at least 32768
+columns, 12 x 12 below) at sizes around their edges: two steps with the
+multigrid solver against the line solver, which shares none of the cycle,
+alone (small tiles) and in a batch whose other member brings the launch over
+the threshold (large tiles).
+
+Both solvers leave |b - A x| <= 1e-12 |b|; the pressure's error is that times
+the condition of the system, below 1e4 on these grids (dx of the order of the
+depth, at most 57 columns across), and the velocities take dt/rho of its
+gradient.  Hence 1e-7 on P and 1e-8 on the rest, relative to each field's
+largest value."""
+import numpy as np
+import pytest
+
+from nhwave_amd import capi
+from nhwave_amd import scenario as S
+from nhwave_amd.batch import Batch
+from nhwave_amd.model import Model
+
+pytestmark = pytest.mark.gpu
+FIELDS = ("Eta", "U", "V", "W", "P")
+
+
+def case(m, n, k):
+    return S.random_scenario(7, mglob=m, nglob=n, kglob=k, steps=2, dry=False, tol=1e-12)
+
+
+def interior(f):
+    return {q: v[(slice(2, -2),) * v.ndim] for q, v in f.items()}
+
+
+@pytest.mark.parametrize("m,n,k", [(12, 12, 3), (13, 11, 2), (28, 12, 10), (29, 13, 9), (27, 25, 16), (57, 24, 12),
+                                   (100, 3, 5), (70, 1, 4), (3, 400, 7), (83, 41, 6)])
+def test_tiles_against_the_line_solver(gpu, m, n, k):
+    s = case(m, n, k)
+    with Model(s, solver=capi.NHW_SOLVER_LINE) as a:
+        a.step(2)
+        ref = interior(a.download(*FIELDS))
+    with Model(s) as a:
+        a.step(2)
+        assert a.stats().not_converged == 0
+        alone = interior(a.download(*FIELDS))
+    big = S.bumps_beach(n=192, m=180, kglob=3, dx=10.0, nbumps=4, beach_width=400.0, tol=1e-8)
+    with Batch([s, big], autotune=False) as b:
+        b.step(2)
+        assert b.members[0].stats().not_converged == 0
+        together = interior(b.members[0].download(*FIELDS))
+    for q in FIELDS:
+        top = max(float(np.abs(ref[q]).max()), 1e-300)
+        for got in (alone, together):
+            assert float(np.abs(got[q] - ref[q]).max()) / top < (1e-7 if q == "P" else 1e-8), q
