@@ -155,8 +155,7 @@ int blaunch_source_terms(Batch *B);
 int blaunch_fluxes(Batch *B);
 int blaunch_eval_explicit(Batch *B, int istep);
 int blaunch_get_uvw(Batch *B);
-int blaunch_projection(Batch *B);
-int blaunch_rk_blend(Batch *B, int istep);
+int blaunch_end_stage(Batch *B, int istep);
 int blaunch_get_omega(Batch *B);
 int blaunch_wave_bc(Batch *B);   // boundary forcing (nhw_forcing.hip)
 int blaunch_sponge(Batch *B);

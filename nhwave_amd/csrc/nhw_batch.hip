@@ -189,7 +189,7 @@ static int batch_build(Batch *B) {
   B->shapes.clear();
   B->ibuf_h.clear();
   B->kbuf_h.clear();
-  std::vector<long> fx, fy, fz, c2, c3, a2, a3, one;
+  std::vector<long> fx, fy, fz, c2, c3, a2, a3, one, ex, lg;
   for (nhw_ctx *c : B->m) {
     const Geo &g = c->g;
     fx.push_back(flux_x_threads(g));
@@ -197,6 +197,8 @@ static int batch_build(Batch *B) {
     fz.push_back((long)g.M * g.N);
     c2.push_back((long)g.M * g.N);
     c3.push_back(g.neq());
+    ex.push_back((long)g.M * g.N * (c->p.viscous ? 1 : 1 + g.K));  // mass columns, momentum cells
+    lg.push_back((long)g.M * g.N * level_groups(g));
     a2.push_back(g.n2());
     a3.push_back(g.n3());
     one.push_back(1);
@@ -208,21 +210,25 @@ static int batch_build(Batch *B) {
     bshape_add(B, "fy" + s, fy, all, bs);
     bshape_add(B, "fz" + s, fz, all, bs);
     bshape_add(B, "c2" + s, c2, all, bs);
+    bshape_add(B, "lg" + s, lg, all, bs);
   }
   bshape_add(B, "c3/256", c3, all, 256);
+  bshape_add(B, "ex/256", ex, all, 256);
   bshape_add(B, "a2/256", a2, all, 256);
   bshape_add(B, "a3/256", a3, all, 256);
   bshape_add(B, "one", one, all, 256, true);
-  // boundary forcing over the members that have it
-  std::vector<long> wb, sp;
-  std::vector<int> wbi, spi;
+  // boundary forcing and the viscous branch over the members that have it
+  std::vector<long> wb, sp, vs;
+  std::vector<int> wbi, spi, vsi;
   for (int u = 0; u < ns; ++u) {
     const nhw_ctx *c = B->m[u];
+    if (c->p.viscous) { vs.push_back((long)c->g.M * c->g.N); vsi.push_back(u); }
     if (west_wavemaker(c->p.wave.kind)) { wb.push_back(c->g.Nloc); wbi.push_back(u); }
     if (c->p.wave.sponge_on) { sp.push_back(c->g.n2()); spi.push_back(u); }
   }
   bshape_add(B, "wb/64", wb, wbi, 64);
   bshape_add(B, "sp/256", sp, spi, 256);
+  bshape_add(B, "vs/256", vs, vsi, 256);
   if (B->non_hydro) {
     int maxlev = 0;
     for (nhw_ctx *c : B->m) maxlev = std::max(maxlev, (int)(B->mixed ? c->mg.lvf : c->mg.lv).size());
@@ -368,9 +374,7 @@ static int stage_pre(Batch *B, int st) {
 }
 static int stage_post(Batch *B, int st) {
   int rc;
-  if (B->non_hydro && (rc = blaunch_projection(B))) return rc;
-  if ((rc = blaunch_rk_blend(B, st))) return rc;
-  if ((rc = blaunch_get_uvw(B))) return rc;
+  if ((rc = blaunch_end_stage(B, st))) return rc;
   if ((rc = blaunch_get_omega(B))) return rc;
   if ((rc = blaunch_sponge(B))) return rc;
   return own_launches(B, is_viscous, eval_turb);

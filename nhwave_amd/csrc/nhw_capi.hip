@@ -551,10 +551,8 @@ int nhw_eval_duvw(nhw_ctx *c, int32_t istep) {
   if (c->cfg.non_hydro) {
     if ((rc = launch_get_uvw(c))) return rc;
     if ((rc = poisson_solve(c))) return rc;
-    if ((rc = launch_projection(c))) return rc;
   }
-  if ((rc = launch_rk_blend(c, istep))) return rc;
-  if ((rc = launch_get_uvw(c))) return rc;
+  if ((rc = launch_end_stage(c, istep))) return rc;
   return launch_get_omega(c);
 }
 
@@ -564,9 +562,7 @@ int nhw_step(nhw_ctx *c, int32_t nsteps) {
   for (int s = 0; s < nsteps; ++s) {
     if ((rc = launch_estimate_dt(c))) return rc;
     if ((rc = launch_wave_bc(c))) return rc;
-    if ((rc = launch_update_mask(c))) return rc;
-    if ((rc = launch_update_wind(c))) return rc;
-    if ((rc = launch_update_vars(c))) return rc;
+    if ((rc = launch_begin_step(c))) return rc;
     for (int st = 1; st <= c->cfg.time_order; ++st) {
       if ((rc = launch_source_terms(c))) return rc;
       if ((rc = launch_fluxes(c))) return rc;

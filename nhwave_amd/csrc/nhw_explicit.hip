@@ -10,6 +10,7 @@
 // fused: each face thread reconstructs its two states from the cell fields,
 // applies the wet-dry overrides, wave speeds, HLL and flux_bc in registers,
 // and writes only the four final face fluxes.
+#include <algorithm>
 #include <utility>
 #include <vector>
 
@@ -152,8 +153,14 @@ __device__ __forceinline__ bool wave_speeds_r(int ml, int mr, double pl, double 
 template <class R>
 __device__ __forceinline__ void flux_x_body(const Geo &g, const Par &p, const DevT<R> &d, long t, int arg) {
   const int wpr = (g.M + 1 + kXFaces - 1) / kXFaces;  // wavefronts per row
-  const long w = t >> 6;
-  if (w >= (long)wpr * g.N) return;  // whole wavefronts leave together
+  // arg: parts the levels are split into (0: one); a part's wavefronts follow
+  // those of the part before
+  const int parts = max(arg, 1);
+  const long rows = (long)wpr * g.N, wave = t >> 6;
+  if (wave >= rows * parts) return;  // whole wavefronts leave together
+  const int part = (int)(wave / rows);
+  const long w = wave - part * rows;
+  const int ka = g.Kbeg + part * g.K / parts, kb = g.Kbeg + (part + 1) * g.K / parts;
   const int lane = (int)(t & 63);
   const int j = g.Jbeg + (int)(w / wpr);
   const int i = g.Ibeg - 2 + (int)(w % wpr) * kXFaces + lane;  // the lane's cell, and its west face
@@ -188,14 +195,14 @@ __device__ __forceinline__ void flux_x_body(const Geo &g, const Par &p, const De
   const bool mutR = (i <= g.Iend) && mr == 1 && mrr != 0 && ml == 0; // case 2 of cell i
   if (mutL) h0 = d.Hc[c2m1];
   else if (mutR) h0 = d.Hc[c20];
-  if (face && (mutL || mutR)) d.Hfx0[g.x2(i, j)] = h0;
+  if (face && part == 0 && (mutL || mutR)) d.Hfx0[g.x2(i, j)] = h0;
   if (leftOv) { etaL = em1; DL = d.D[c2m1]; }
   if (rightOv) { etaR = e0; DR = d.D[c20]; }
   const double PL = pres(etaL, h0), PR = pres(etaR, h0);
   const double pl = sqrt(kGrav * fabs(DL)), pr = sqrt(kGrav * fabs(DR));
 
   const R dxR = (R)dx, hdxR = (R)hdx;
-  for (int k = g.Kbeg; k <= g.Kend; ++k) {
+  for (int k = ka; k < kb; ++k) {
     const long c0 = g.c3(ic, j, k);
     auto recon = [&](const R *F, R &qL, R &qR) {
       const R c = F[c0];
@@ -259,12 +266,13 @@ __device__ __forceinline__ void flux_x_body(const Geo &g, const Par &p, const De
 // step's loads are contiguous rows.
 template <class R>
 __device__ __forceinline__ void flux_y_body(const Geo &g, const Par &p, const DevT<R> &d, long t, int arg) {
-  if (t >= flux_y_threads(g)) return;
+  const int faces = arg > 0 ? arg : kYFaces;  // faces a thread walks
+  if (t >= flux_y_threads(g, faces)) return;
   const int i = g.Ibeg + (int)(t % g.M);
   const long r = t / g.M;
   const int k = g.Kbeg + (int)(r % g.K);
-  const int jf0 = g.Jbeg + (int)(r / g.K) * kYFaces;
-  const int jf1 = min(jf0 + kYFaces - 1, g.Jend1);
+  const int jf0 = g.Jbeg + (int)(r / g.K) * faces;
+  const int jf1 = min(jf0 + faces - 1, g.Jend1);
   const double dy = g.dy, hdy = 0.5 * dy, MinDep = p.min_dep;
   const R dyR = (R)dy, hdyR = (R)hdy;
   const long sj = g.Mloc;
@@ -405,22 +413,33 @@ __device__ __forceinline__ void flux_y_body(const Geo &g, const Par &p, const De
 // loaded once, with the arithmetic of z_slope.
 template <class R>
 __device__ __forceinline__ void flux_z_body(const Geo &g, const Par &p, const DevT<R> &d, long t, int arg) {
-  if (t >= (long)g.M * g.N) return;
-  const int i = g.Ibeg + (int)(t % g.M), j = g.Jbeg + (int)(t / g.M);
+  // arg: parts a column's faces are split into (0: one); a part starts with
+  // the slope of the cell below its first face
+  const int parts = max(arg, 1);
+  const long cols = (long)g.M * g.N;
+  if (t >= cols * parts) return;
+  const int part = (int)(t / cols);
+  const int tc = (int)(t - part * cols);
+  const int i = g.Ibeg + tc % g.M, j = g.Jbeg + tc / g.M;
   const long sk = (long)g.Mloc * g.Nloc;
-  const long q0 = g.c3(i, j, g.Kbeg);
-  d.Fz[q0] = 0.0; d.Gz[q0] = 0.0; d.Hz[q0] = 0.0;
-  const long qt = q0 + (long)g.K * sk;  // the surface face Kend1
-  d.Fz[qt] = 0.0; d.Gz[qt] = 0.0; d.Hz[qt] = 0.0;
-  if (g.K < 2) return;
+  const long qb = g.c3(i, j, g.Kbeg);
+  if (part == 0) { d.Fz[qb] = 0.0; d.Gz[qb] = 0.0; d.Hz[qb] = 0.0; }
+  if (part == parts - 1) {
+    const long qt = qb + (long)g.K * sk;  // the surface face Kend1
+    d.Fz[qt] = 0.0; d.Gz[qt] = 0.0; d.Hz[qt] = 0.0;
+  }
+  // inner faces Kbeg+1 .. Kend, split evenly
+  const int nf = g.K - 1, ka = g.Kbeg + 1 + part * nf / parts, kb = g.Kbeg + 1 + (part + 1) * nf / parts;
+  if (ka >= kb) return;
   const double *sigc = d.sigc - 1, *dsig = d.dsig - 1;
   const R *const Fl[3] = {d.U, d.V, d.W};
   R *const Out[3] = {d.Fz, d.Gz, d.Hz};
   // per field: the forward difference quotient of the cell below the face,
   // the face's left state and the value of the cell above it
   R t1b[3], zl[3], ca[3];
+  const long q0 = qb + (long)(ka - 1 - g.Kbeg) * sk;
   {
-    const int k = g.Kbeg;  // the bottom cell: its slope gives the left state of face Kbeg+1
+    const int k = ka - 1;  // the cell below: its slope gives the left state of face ka
     const R hm = (R)(sigc[k] - sigc[k - 1]), hp = (R)(sigc[k + 1] - sigc[k]);
     const R hd = (R)(0.5 * dsig[k]);
 #pragma unroll
@@ -433,8 +452,8 @@ __device__ __forceinline__ void flux_z_body(const Geo &g, const Par &p, const De
       ca[n] = c;
     }
   }
-  for (int k = g.Kbeg + 1; k <= g.Kend; ++k) {
-    const long q = q0 + (long)(k - g.Kbeg) * sk;
+  for (int k = ka; k < kb; ++k) {
+    const long q = q0 + (long)(k - ka + 1) * sk;
     const R om = d.Omega[q];
     const R hp = (R)(sigc[k + 1] - sigc[k]);
     const R hd0 = (R)(0.5 * dsig[k]);
@@ -471,13 +490,52 @@ __device__ __forceinline__ int mir(int i, int beg, int end) {
 }
 
 // eval_duvw explicit part, src/nhwave.F:611-634, 637-688, 841-845,
-// 1004-1008, 1163-1182: one thread per interior column.  Mass update, D floor,
-// wall ghosts of D (wl_bc, :5119-5262), Eta = D - Hc, momentum update.
+// 1004-1008, 1163-1182.  Of each row of columns, one slice of threads takes a
+// column each: mass update, D floor, wall ghosts of D (wl_bc, :5119-5262),
+// Eta = D - Hc.  The other slices take a cell each, a level a slice: momentum
+// update (left to k_visc_solve in viscous runs).  Neither part reads what the
+// other writes; a thread per column for both walked the levels twice, its
+// loads waiting on one another.  The slices of a row follow one another, so
+// that the sigma faces a cell shares with the one above and the y faces it
+// shares with the next row are still in the L2 (257 x 33 x 5: 9.5 us, now 6;
+// 333 x 217 x 7: 20.6, now 15.8; 2048 x 2048 x 8 in float: 604, now 581, of
+// which its arrays take 430 at 5 TB/s; 1024 x 1024 x 10: 340, as before).
+__host__ __device__ __forceinline__ long explicit_threads(const Geo &g, const Par &p) {
+  return (long)g.M * g.N * (p.viscous ? 1 : 1 + g.K);
+}
+template <class R>
+__device__ __forceinline__ void momentum_cell(const Geo &g, const Par &p, const DevT<R> &d, int i, int j, int k) {
+  const long c = g.c2(i, j), q = g.c3(i, j, k);
+  if (d.Mask[c] == 0) {
+    d.DU[q] = 0.0; d.DV[q] = 0.0; d.DW[q] = 0.0;
+    return;
+  }
+  const double dt = d.scal[0], dx = g.dx, dy = g.dy;
+  const double fcor = p.fcor, SX = d.SourceX[c], SY = d.SourceY[c];
+  const double du = d.DU[q], dv = d.DV[q], dw = d.DW[q];
+  const double rdz = 1.0 / (d.dsig - 1)[k];
+  const long fx0 = g.x3(i, j, k), fy0 = g.y3(i, j, k);
+  const long fz0 = q, fz1 = q + (long)g.Mloc * g.Nloc;
+  double R2 = -1.0 / dx * (d.Fx[fx0 + 1] - d.Fx[fx0]) - 1.0 / dy * (d.Fy[fy0 + g.Mloc] - d.Fy[fy0]) -
+              rdz * (d.Fz[fz1] - d.Fz[fz0]) + fcor * dv + 0.0 + SX + 0.0 + 0.0 + 0.0;
+  double R3 = -1.0 / dx * (d.Gx[fx0 + 1] - d.Gx[fx0]) - 1.0 / dy * (d.Gy[fy0 + g.Mloc] - d.Gy[fy0]) -
+              rdz * (d.Gz[fz1] - d.Gz[fz0]) - fcor * du + 0.0 + SY + 0.0 + 0.0 + 0.0;
+  double R4 = -1.0 / dx * (d.Hx[fx0 + 1] - d.Hx[fx0]) - 1.0 / dy * (d.Hy[fy0 + g.Mloc] - d.Hy[fy0]) -
+              rdz * (d.Hz[fz1] - d.Hz[fz0]) + 0.0 + 0.0;
+  d.DU[q] = du + dt * R2;
+  d.DV[q] = dv + dt * R3;
+  d.DW[q] = dw + dt * R4;
+}
+
 template <class R>
 __device__ __forceinline__ void eval_explicit_body(const Geo &g, const Par &p, const DevT<R> &d, long t, int arg) {
   const double A = p.alpha[arg - 1], B = p.beta[arg - 1];
-  if (t >= (long)g.M * g.N) return;
-  const int i = g.Ibeg + (int)(t % g.M), j = g.Jbeg + (int)(t / g.M);
+  const int slices = p.viscous ? 1 : 1 + g.K;
+  const int i = g.Ibeg + (int)(t % g.M);
+  const long r = t / g.M;
+  const int s = (int)(r % slices), j = g.Jbeg + (int)(r / slices);
+  if (j > g.Jend) return;
+  if (s > 0) return momentum_cell(g, p, d, i, j, g.Kbeg + s - 1);
   const long c = g.c2(i, j);
   const double dt = d.scal[0], dx = g.dx, dy = g.dy;
   const double *dsig = d.dsig - 1;
@@ -485,6 +543,7 @@ __device__ __forceinline__ void eval_explicit_body(const Geo &g, const Par &p, c
   double Dn = d.D[c];
   double R1 = 0.0;
   if (m != 0) {
+#pragma unroll 4
     for (int k = g.Kbeg; k <= g.Kend; ++k)
       R1 = R1 - 1.0 / dx * (d.Ex[g.x3(i + 1, j, k)] - d.Ex[g.x3(i, j, k)]) * dsig[k] -
            1.0 / dy * (d.Ey[g.y3(i, j + 1, k)] - d.Ey[g.y3(i, j, k)]) * dsig[k];
@@ -527,29 +586,6 @@ __device__ __forceinline__ void eval_explicit_body(const Geo &g, const Par &p, c
       d.D[cc] = xv[a];
       d.Eta[cc] = xv[a] - d.Hc[cc];
     }
-  // momentum (the viscous branch solves it implicitly in k_visc_solve)
-  if (p.viscous) return;
-  const double fcor = p.fcor, SX = d.SourceX[c], SY = d.SourceY[c];
-  for (int k = g.Kbeg; k <= g.Kend; ++k) {
-    const long q = g.c3(i, j, k);
-    if (m == 0) {
-      d.DU[q] = 0.0; d.DV[q] = 0.0; d.DW[q] = 0.0;
-      continue;
-    }
-    const double du = d.DU[q], dv = d.DV[q], dw = d.DW[q];
-    const double rdz = 1.0 / dsig[k];
-    const long fx0 = g.x3(i, j, k), fy0 = g.y3(i, j, k);
-    const long fz0 = q, fz1 = q + (long)g.Mloc * g.Nloc;
-    double R2 = -1.0 / dx * (d.Fx[fx0 + 1] - d.Fx[fx0]) - 1.0 / dy * (d.Fy[fy0 + g.Mloc] - d.Fy[fy0]) -
-                rdz * (d.Fz[fz1] - d.Fz[fz0]) + fcor * dv + 0.0 + SX + 0.0 + 0.0 + 0.0;
-    double R3 = -1.0 / dx * (d.Gx[fx0 + 1] - d.Gx[fx0]) - 1.0 / dy * (d.Gy[fy0 + g.Mloc] - d.Gy[fy0]) -
-                rdz * (d.Gz[fz1] - d.Gz[fz0]) - fcor * du + 0.0 + SY + 0.0 + 0.0 + 0.0;
-    double R4 = -1.0 / dx * (d.Hx[fx0 + 1] - d.Hx[fx0]) - 1.0 / dy * (d.Hy[fy0 + g.Mloc] - d.Hy[fy0]) -
-                rdz * (d.Hz[fz1] - d.Hz[fz0]) + 0.0 + 0.0;
-    d.DU[q] = du + dt * R2;
-    d.DV[q] = dv + dt * R3;
-    d.DW[q] = dw + dt * R4;
-  }
 }
 
 // DelxEta/DelyEta at interior cells, src/nhwave.F:630-631
@@ -565,9 +601,11 @@ __device__ __forceinline__ void eta_slopes_body(const Geo &g, const Par &p, cons
 
 // ----------------------------------------------------------------------------
 // get_UVW + vel_bc, src/nhwave.F:1651-1683, 4416-5066 (lateral BC 1/2,
-// Bc_Z0 = 1).  Pass A: U = DU/D, lateral wall ghosts, and the surface/bottom
-// z-face states with the kinematic BCs (KBC_surface/KBC_bottom).  Pass B:
-// limited x/y slopes of those face states and the vertical ghost cells.
+// Bc_Z0 = 1), with the projection and the SSP-RK blend that precede it at the
+// end of a stage.  Pass A: the momenta, U = DU/D, lateral wall ghosts, and the
+// surface/bottom z-face states with the kinematic BCs (KBC_surface/
+// KBC_bottom).  Pass B: limited x/y slopes of those face states and the
+// vertical ghost cells.
 // ----------------------------------------------------------------------------
 // vel_bc's wall friction boundary (BC 5, :4486-4501, :4583-4598,
 // :4676-4691, :4737-4752): Cdrag = Cd0 (Ibot = 1) or 1/(1/Kappa log(30 h/2/
@@ -586,24 +624,134 @@ __device__ __forceinline__ double wall_phi(const Par &p, const DevT<R> &d, doubl
   return phi < 2.0 ? phi : 2.0;
 }
 
+// What a velocity pass does to its cells (flags in `arg`, RK stage from bit
+// 8): the momenta's projection (projection_corrector) and SSP-RK blend, U =
+// DU/D, and the surface slopes DelxEta/DelyEta.
+enum { UVW_DIVIDE = 1, UVW_BLEND = 2, UVW_PROJECT = 4, UVW_SLOPES = 8 };
+
+// projection_corrector, src/nhwave.F:487-536, of one wet cell (DelxSc/DelySc
+// of sigma_transform, :6505-6541, formed in place).  lo, hi: the pressures on
+// the sigma faces below and above it: of the column, then its west, east,
+// south and north neighbours.
 template <class R>
+__device__ __forceinline__ void project_cell(const Geo &g, const DevT<R> &d, long c, int k, const double (&lo)[5],
+                                             const double (&hi)[5], R &du, R &dv, R &dw) {
+  const double dx = g.dx, dy = g.dy, dt = d.scal[0];
+  const double *dsig = d.dsig - 1, *sigc = d.sigc - 1;
+  const double dxp = 0.5 * ((lo[2] - lo[1]) / (2. * dx) + (hi[2] - hi[1]) / (2. * dx));
+  const double dyp = 0.5 * ((lo[4] - lo[3]) / (2. * dy) + (hi[4] - hi[3]) / (2. * dy));
+  const double dzp = (hi[0] - lo[0]) / dsig[k];
+  const double Dd = d.D[c];
+  const double dxsc = (1.0 - sigc[k]) / Dd * d.DelxH[c] - sigc[k] / Dd * d.DelxEta[c];
+  const double dysc = (1.0 - sigc[k]) / Dd * d.DelyH[c] - sigc[k] / Dd * d.DelyEta[c];
+  du = du - Dd * dt / kRho0 * (dxp + dzp * dxsc);
+  dv = dv - Dd * dt / kRho0 * (dyp + dzp * dysc);
+  dw = dw - dt / kRho0 * dzp;
+}
+// ... the pressures of the sigma face at q
+__device__ __forceinline__ void face_pressures(const Geo &g, const double *P, long q, double (&f)[5]) {
+  f[0] = P[q];
+  f[1] = P[q - 1]; f[2] = P[q + 1];
+  f[3] = P[q - g.Mloc]; f[4] = P[q + g.Mloc];
+}
+
+// SSP-RK blend + dry zeroing + Froude cap, src/nhwave.F:1227-1261, of one cell
+// with the step's momenta DU0, DV0, DW0; fu: the capped momentum.  The square
+// root waits for a sum of squares that can reach fu (rounding included).
+template <class R>
+__device__ __forceinline__ void blend_cell(const Par &p, int stage, int m, double fu, R DU0, R DV0, R DW0, R &DU,
+                                           R &DV, R &DW) {
+  const double A = p.alpha[stage - 1], B = p.beta[stage - 1];
+  double du = A * DU0 + B * DU;
+  double dv = A * DV0 + B * DV;
+  double dw = A * DW0 + B * DW;
+  if (m == 0) { du = 0.0; dv = 0.0; dw = 0.0; }
+  if (p.froude_on && m > 0) {
+    const double s = du * du + dv * dv + dw * dw;
+    if (s > fu * fu * (1.0 - 1e-14) && sqrt(s) > fu) {
+      const double ang = atan2(dv, du);
+      du = fu * cos(ang);
+      dv = fu * sin(ang);
+      dw = 0.0;
+    }
+  }
+  DU = (R)du; DV = (R)dv; DW = (R)dw;
+}
+
+// One thread takes a group of sigma levels of a column (level_groups): their
+// momenta (projection and blend in place), U = DU/D and the lateral ghosts of
+// those levels; the groups at the surface and at the bottom also form the
+// face states there, from values still in registers.  Projection, blend,
+// division and ghosts were a launch each, every one streaming the momenta
+// again, the last of them a thread per column (1024 x 1024 x 10: 182 + 137 +
+// 195 us, now 324; 333 x 217 x 7: 38 + 8, now 15).  Every load is issued before the first value is used: a
+// wait for memory, not the rate of the loads, is what a thread spends its
+// time on.  Rows go one by one with the groups of a row next to one another,
+// so that the pressures of neighbouring rows and levels are in the L2.
+//
+// MODE is the flags of a pass over walls that mirror (BC 1, 2); the general
+// form, MODE 0, takes them from `arg`, has inflow and friction sides too and
+// groups of three levels, which cost it a third of its wavefronts (registers).
+template <class R, int MODE>
 __device__ __forceinline__ void uvw_a_body(const Geo &g, const Par &p, const DevT<R> &d, long t, int arg) {
-  const int divide = arg;
-  if (t >= (long)g.M * g.N) return;
-  const int i = g.Ibeg + (int)(t % g.M), j = g.Jbeg + (int)(t / g.M);
+  constexpr int NL = MODE ? 2 : 3;
+  const int what = MODE ? MODE : arg;
+  const bool divide = what & UVW_DIVIDE, blend = what & UVW_BLEND, project = what & UVW_PROJECT;
+  const int stage = arg >> 8, ng = level_groups(g);
+  const int i = g.Ibeg + (int)(t % g.M);
+  const long r = t / g.M;
+  const int grp = (int)(r % ng), j = g.Jbeg + (int)(r / ng);
+  if (j > g.Jend) return;
+  const bool odd = g.K & 1, three = !MODE && g.K == 3;
+  const int ka = g.Kbeg + 2 * grp - (odd && grp > 1), nk = three ? 3 : odd && grp == 1 ? 1 : 2;
   const long c = g.c2(i, j);
   const double Dd = d.D[c];
   const long sk = (long)g.Mloc * g.Nloc;
-  const long q0 = g.c3(i, j, g.Kbeg);
-  if (divide)
-    for (int k = g.Kbeg; k <= g.Kend; ++k) {
-      const long q = q0 + (k - g.Kbeg) * sk;
-      d.U[q] = d.DU[q] / Dd;
-      d.V[q] = d.DV[q] / Dd;
-      d.W[q] = d.DW[q] / Dd;
+  const long qa = g.c3(i, j, ka);
+  double dxe = 0.0, dye = 0.0;
+  if (grp == ng - 1) {
+    if (arg & UVW_SLOPES) {  // src/nhwave.F:630-631
+      const int m = d.Mask[c];
+      dxe = tvd_slope(d.Eta[c - 1], d.Eta[c], d.Eta[c + 1], g.dx, m);
+      dye = tvd_slope(d.Eta[c - g.Mloc], d.Eta[c], d.Eta[c + g.Mloc], g.dy, m);
+      d.DelxEta[c] = dxe;
+      d.DelyEta[c] = dye;
+    } else {
+      dxe = d.DelxEta[c];
+      dye = d.DelyEta[c];
     }
+  }
+  R u[NL], v[NL], w[NL], du[NL], dv[NL], dw[NL];
+  {
+    const int m = blend || project ? d.Mask[c] : 1;
+    const double fu = blend ? sqrt(kGrav * Dd) * p.froude_cap * Dd : 0.0;
+    R u0[NL], v0[NL], w0[NL];
+    double P[NL + 1][5];
+    if (project) face_pressures(g, d.P, qa, P[0]);
+#pragma unroll
+    for (int n = 0; n < NL; ++n) {
+      const long q = qa + min(n, nk - 1) * sk;
+      if (project) face_pressures(g, d.P, q + sk, P[n + 1]);
+      du[n] = d.DU[q]; dv[n] = d.DV[q]; dw[n] = d.DW[q];
+      if (blend) { u0[n] = d.DU0[q]; v0[n] = d.DV0[q]; w0[n] = d.DW0[q]; }
+      if (!divide) { u[n] = d.U[q]; v[n] = d.V[q]; w[n] = d.W[q]; }
+    }
+#pragma unroll
+    for (int n = 0; n < NL; ++n) {
+      if (n >= nk) break;
+      const long q = qa + n * sk;
+      if (project && m != 0) project_cell(g, d, c, ka + n, P[n], P[n + 1], du[n], dv[n], dw[n]);
+      if (blend) blend_cell(p, stage, m, fu, u0[n], v0[n], w0[n], du[n], dv[n], dw[n]);
+      if (project || blend) { d.DU[q] = du[n]; d.DV[q] = dv[n]; d.DW[q] = dw[n]; }
+      if (divide) {
+        u[n] = (R)(du[n] / Dd); v[n] = (R)(dv[n] / Dd); w[n] = (R)(dw[n] / Dd);
+        d.U[q] = u[n]; d.V[q] = v[n]; d.W[q] = w[n];
+      }
+    }
+  }
   // the velocity of interior cell q of column cq as this pass leaves it (a
-  // neighbour's own thread may be writing it: formed again, the same way)
+  // neighbour's own thread may be writing it: formed again, the same way; a
+  // pass that also projects or blends has no wall friction sides)
   auto vel = [&](const R *F, const R *DF, long q, long cq) -> double {
     return divide ? (double)(R)((double)DF[q] / d.D[cq]) : (double)F[q];
   };
@@ -611,71 +759,68 @@ __device__ __forceinline__ void uvw_a_body(const Geo &g, const Par &p, const Dev
   // normal one mirrored; their D U take D(n, j) (x sides) or D(i, n) (y
   // sides), n = 1, 2 the ghost's distance from the wall, as the reference
   // writes them
-  auto wall5 = [&](long gq, long s, double ph, double dg, bool xside) {
-    d.U[gq] = xside ? -d.U[s] : (R)((1.0 - ph) * (double)d.U[s]);
-    d.V[gq] = xside ? (R)((1.0 - ph) * (double)d.V[s]) : -d.V[s];
-    d.W[gq] = (R)((1.0 - ph) * (double)d.W[s]);
-    d.DU[gq] = (R)(dg * (double)d.U[gq]);
-    d.DV[gq] = (R)(dg * (double)d.V[gq]);
-    d.DW[gq] = (R)(dg * (double)d.W[gq]);
+  auto wall5 = [&](long gq, int n, double ph, double dg, bool xside) {
+    const R gu = xside ? -u[n] : (R)((1.0 - ph) * (double)u[n]);
+    const R gv = xside ? (R)((1.0 - ph) * (double)v[n]) : -v[n];
+    const R gw = (R)((1.0 - ph) * (double)w[n]);
+    d.U[gq] = gu; d.V[gq] = gv; d.W[gq] = gw;
+    d.DU[gq] = (R)(dg * (double)gu);
+    d.DV[gq] = (R)(dg * (double)gv);
+    d.DW[gq] = (R)(dg * (double)gw);
   };
   // lateral ghosts, :4440-4761 (inflow at the west, :4468-4476)
   auto xghost = [&](int gi, int bc) {
-    if (bc == 3 && gi > g.Iend) return;  // FLUX_LR's open east boundary: k_east_ghosts
-    if (bc == 5) {
-      const int ib = gi < g.Ibeg ? g.Ibeg : g.Iend, n = gi < g.Ibeg ? g.Ibeg - gi : gi - g.Iend;
-      const long cb = g.c2(ib, j);
-      const double dg = d.D[g.c2(n, j)];
-      for (int k = g.Kbeg; k <= g.Kend; ++k) {
-        const long b = g.c3(ib, j, k);
-        const double ph = wall_phi(p, d, g.dx, vel(d.V, d.DV, b, cb), vel(d.W, d.DW, b, cb), b);
-        wall5(g.c3(gi, j, k), q0 + (k - g.Kbeg) * sk, ph, dg, true);
-      }
-      return;
-    }
+    if (!MODE && bc == 3 && gi > g.Iend) return;  // FLUX_LR's open east boundary: k_east_ghosts
     const bool ns = bc == 2;
-    for (int k = g.Kbeg; k <= g.Kend; ++k) {
-      const long s = q0 + (k - g.Kbeg) * sk, gq = g.c3(gi, j, k);
-      if (bc == 3) {
+#pragma unroll
+    for (int n = 0; n < NL; ++n) {
+      if (n >= nk) break;
+      const int k = ka + n;
+      const long gq = g.c3(gi, j, k);
+      if (!MODE && bc == 5) {
+        const int ib = gi < g.Ibeg ? g.Ibeg : g.Iend, far = gi < g.Ibeg ? g.Ibeg - gi : gi - g.Iend;
+        const long cb = g.c2(ib, j), b = g.c3(ib, j, k);
+        const double ph = wall_phi(p, d, g.dx, vel(d.V, d.DV, b, cb), vel(d.W, d.DW, b, cb), b);
+        wall5(gq, n, ph, d.D[g.c2(far, j)], true);
+      } else if (!MODE && bc == 3) {
         const long b = inflow_idx(g, j, k);
         const double din = d.Din0[j - 1], uin = d.Uin0[b], vin = d.Vin0[b], win = d.Win0[b];
-        d.U[gq] = (R)(2.0 * uin - (double)d.U[s]);
-        d.V[gq] = (R)(2.0 * vin - (double)d.V[s]);
-        d.W[gq] = (R)(2.0 * win - (double)d.W[s]);
-        d.DU[gq] = (R)(2.0 * din * uin - (double)d.DU[s]);
-        d.DV[gq] = (R)(2.0 * din * vin - (double)d.DV[s]);
-        d.DW[gq] = (R)(2.0 * din * win - (double)d.DW[s]);
-        continue;
+        d.U[gq] = (R)(2.0 * uin - (double)u[n]);
+        d.V[gq] = (R)(2.0 * vin - (double)v[n]);
+        d.W[gq] = (R)(2.0 * win - (double)w[n]);
+        d.DU[gq] = (R)(2.0 * din * uin - (double)du[n]);
+        d.DV[gq] = (R)(2.0 * din * vin - (double)dv[n]);
+        d.DW[gq] = (R)(2.0 * din * win - (double)dw[n]);
+      } else {
+        d.U[gq] = -u[n];
+        d.V[gq] = ns ? -v[n] : v[n];
+        d.W[gq] = ns ? -w[n] : w[n];
+        d.DU[gq] = -du[n];
+        d.DV[gq] = ns ? -dv[n] : dv[n];
+        d.DW[gq] = ns ? -dw[n] : dw[n];
       }
-      d.U[gq] = -d.U[s];
-      d.V[gq] = ns ? -d.V[s] : d.V[s];
-      d.W[gq] = ns ? -d.W[s] : d.W[s];
-      d.DU[gq] = -d.DU[s];
-      d.DV[gq] = ns ? -d.DV[s] : d.DV[s];
-      d.DW[gq] = ns ? -d.DW[s] : d.DW[s];
     }
   };
   auto yghost = [&](int gj, int bc) {
-    if (bc == 5) {
-      const int jb = gj < g.Jbeg ? g.Jbeg : g.Jend, n = gj < g.Jbeg ? g.Jbeg - gj : gj - g.Jend;
-      const long cb = g.c2(i, jb);
-      const double dg = d.D[g.c2(i, n)];
-      for (int k = g.Kbeg; k <= g.Kend; ++k) {
-        const long b = g.c3(i, jb, k);
-        const double ph = wall_phi(p, d, g.dy, vel(d.U, d.DU, b, cb), vel(d.W, d.DW, b, cb), b);
-        wall5(g.c3(i, gj, k), q0 + (k - g.Kbeg) * sk, ph, dg, false);
-      }
-      return;
-    }
     const bool ns = bc == 2;
-    for (int k = g.Kbeg; k <= g.Kend; ++k) {
-      const long s = q0 + (k - g.Kbeg) * sk, gq = g.c3(i, gj, k);
-      d.U[gq] = ns ? -d.U[s] : d.U[s];
-      d.V[gq] = -d.V[s];
-      d.W[gq] = ns ? -d.W[s] : d.W[s];
-      d.DU[gq] = ns ? -d.DU[s] : d.DU[s];
-      d.DV[gq] = -d.DV[s];
-      d.DW[gq] = ns ? -d.DW[s] : d.DW[s];
+#pragma unroll
+    for (int n = 0; n < NL; ++n) {
+      if (n >= nk) break;
+      const int k = ka + n;
+      const long gq = g.c3(i, gj, k);
+      if (!MODE && bc == 5) {
+        const int jb = gj < g.Jbeg ? g.Jbeg : g.Jend, far = gj < g.Jbeg ? g.Jbeg - gj : gj - g.Jend;
+        const long cb = g.c2(i, jb), b = g.c3(i, jb, k);
+        const double ph = wall_phi(p, d, g.dy, vel(d.U, d.DU, b, cb), vel(d.W, d.DW, b, cb), b);
+        wall5(gq, n, ph, d.D[g.c2(i, far)], false);
+      } else {
+        d.U[gq] = ns ? -u[n] : u[n];
+        d.V[gq] = -v[n];
+        d.W[gq] = ns ? -w[n] : w[n];
+        d.DU[gq] = ns ? -du[n] : du[n];
+        d.DV[gq] = -dv[n];
+        d.DW[gq] = ns ? -dw[n] : dw[n];
+      }
     }
   };
   if (i <= g.Ibeg + 1) xghost(2 * g.Ibeg - 1 - i, p.bc_x0);
@@ -685,28 +830,33 @@ __device__ __forceinline__ void uvw_a_body(const Geo &g, const Par &p, const Dev
   // surface/bottom face states, :4778-4785 (delzFun_3D + construct_3D_z +
   // KBC); the vertical ghosts read here are those of the previous vel_bc
   const double *sigc = d.sigc - 1, *dsig = d.dsig - 1;
-  const int Kb = g.Kbeg, Ke = g.Kend;
-  const long qb = q0, qe = q0 + (long)(Ke - Kb) * sk;
-  const double hpt = sigc[Ke + 1] - sigc[Ke], hmt = sigc[Ke] - sigc[Ke - 1];
-  const double hpb = sigc[Kb + 1] - sigc[Kb], hmb = sigc[Kb] - sigc[Kb - 1];
-  auto top = [&](const R *F) {
-    double a = F[qe - sk], b = F[qe], e = F[qe + sk];
-    return b + 0.5 * dsig[Ke] * z_slope(a, b, e, hpt, hmt);
-  };
-  auto bot = [&](const R *F) {
-    double a = F[qb - sk], b = F[qb], e = F[qb + sk];
-    return b - 0.5 * dsig[Kb] * z_slope(a, b, e, hpb, hmb);
-  };
-  const double uzl = top(d.U), vzl = top(d.V);
-  // KBC_bottom (:5104-5112): a no-slip bottom (Bc_Z0 = 2) zeroes the
-  // horizontal bottom-face states
-  const double uzr = p.bc_z0 == 2 ? 0.0 : bot(d.U), vzr = p.bc_z0 == 2 ? 0.0 : bot(d.V);
-  const double dt = d.scal[0];
-  const double wzl = (d.Eta[c] - d.Eta0[c]) / dt + d.DelxEta[c] * uzl + d.DelyEta[c] * vzl;
-  const double deltH = 0.0;  // DeltH: fixed bathymetry
-  const double wzr = -deltH - d.DelxH[c] * uzr - d.DelyH[c] * vzr;
-  d.ztU[c] = uzl; d.ztV[c] = vzl; d.ztW[c] = wzl;
-  d.zbU[c] = uzr; d.zbV[c] = vzr; d.zbW[c] = wzr;
+  if (grp == ng - 1) {
+    const int Ke = g.Kend;
+    const long qe = g.c3(i, j, Ke);
+    const double hpt = sigc[Ke + 1] - sigc[Ke], hmt = sigc[Ke] - sigc[Ke - 1];
+    auto top = [&](const R (&f)[NL], const R *F) {
+      const double a = three ? f[1] : f[0], b = three ? f[NL - 1] : f[1], e = F[qe + sk];
+      return b + 0.5 * dsig[Ke] * z_slope(a, b, e, hpt, hmt);
+    };
+    const double uzl = top(u, d.U), vzl = top(v, d.V);
+    const double dt = d.scal[0];
+    const double wzl = (d.Eta[c] - d.Eta0[c]) / dt + dxe * uzl + dye * vzl;
+    d.ztU[c] = uzl; d.ztV[c] = vzl; d.ztW[c] = wzl;
+  }
+  if (grp == 0) {
+    const int Kb = g.Kbeg;
+    const double hpb = sigc[Kb + 1] - sigc[Kb], hmb = sigc[Kb] - sigc[Kb - 1];
+    auto bot = [&](const R (&f)[NL], const R *F) {
+      const double a = F[qa - sk], b = f[0], e = f[1];
+      return b - 0.5 * dsig[Kb] * z_slope(a, b, e, hpb, hmb);
+    };
+    // KBC_bottom (:5104-5112): a no-slip bottom (Bc_Z0 = 2) zeroes the
+    // horizontal bottom-face states
+    const double uzr = p.bc_z0 == 2 ? 0.0 : bot(u, d.U), vzr = p.bc_z0 == 2 ? 0.0 : bot(v, d.V);
+    const double deltH = 0.0;  // DeltH: fixed bathymetry
+    const double wzr = -deltH - d.DelxH[c] * uzr - d.DelyH[c] * vzr;
+    d.zbU[c] = uzr; d.zbV[c] = vzr; d.zbW[c] = wzr;
+  }
 }
 
 template <class R>
@@ -836,60 +986,27 @@ __device__ __forceinline__ void uvw_b_body(const Geo &g, const Par &p, const Dev
   (void)sk;
 }
 
-// projection_corrector, src/nhwave.F:487-536 (DelxSc/DelySc of
-// sigma_transform, :6505-6541, formed in place)
+// projection and blend alone, a thread per cell, before the velocity pass of
+// a scenario with wall friction sides (whose ghosts read a neighbouring
+// column's final momenta)
 template <class R>
-__device__ __forceinline__ void projection_body(const Geo &g, const Par &p, const DevT<R> &d, long t, int arg) {
+__device__ __forceinline__ void momenta_body(const Geo &g, const Par &p, const DevT<R> &d, long t, int arg) {
   if (t >= (long)g.M * g.N * g.K) return;
   const int i = g.Ibeg + (int)(t % g.M);
   const long r = t / g.M;
   const int j = g.Jbeg + (int)(r % g.N), k = g.Kbeg + (int)(r / g.N);
-  const long c = g.c2(i, j);
-  if (d.Mask[c] == 0) return;
-  const double dx = g.dx, dy = g.dy, dt = d.scal[0];
-  const double *dsig = d.dsig - 1, *sigc = d.sigc - 1;
-  const long sk = (long)g.Mloc * g.Nloc, sj = g.Mloc;
-  const long q = g.c3(i, j, k);
-  const double *P = d.P;
-  const double dxp = 0.5 * ((P[q + 1] - P[q - 1]) / (2. * dx) + (P[q + sk + 1] - P[q + sk - 1]) / (2. * dx));
-  const double dyp = 0.5 * ((P[q + sj] - P[q - sj]) / (2. * dy) + (P[q + sk + sj] - P[q + sk - sj]) / (2. * dy));
-  const double dzp = (P[q + sk] - P[q]) / dsig[k];
-  const double Dd = d.D[c];
-  const double dxsc = (1.0 - sigc[k]) / Dd * d.DelxH[c] - sigc[k] / Dd * d.DelxEta[c];
-  const double dysc = (1.0 - sigc[k]) / Dd * d.DelyH[c] - sigc[k] / Dd * d.DelyEta[c];
-  d.DU[q] = d.DU[q] - Dd * dt / kRho0 * (dxp + dzp * dxsc);
-  d.DV[q] = d.DV[q] - Dd * dt / kRho0 * (dyp + dzp * dysc);
-  d.DW[q] = d.DW[q] - dt / kRho0 * dzp;
-}
-
-// SSP-RK blend + dry zeroing + Froude cap, src/nhwave.F:1227-1261; one
-// thread per interior column.
-template <class R>
-__device__ __forceinline__ void rk_blend_body(const Geo &g, const Par &p, const DevT<R> &d, long t, int arg) {
-  const double A = p.alpha[arg - 1], B = p.beta[arg - 1];
-  if (t >= (long)g.M * g.N) return;
-  const int i = g.Ibeg + (int)(t % g.M), j = g.Jbeg + (int)(t / g.M);
-  const long c = g.c2(i, j);
+  const long c = g.c2(i, j), q = g.c3(i, j, k);
   const int m = d.Mask[c];
   const double Dd = d.D[c];
-  const double fu = sqrt(kGrav * Dd) * p.froude_cap * Dd;
-  for (int k = g.Kbeg; k <= g.Kend; ++k) {
-    const long q = g.c3(i, j, k);
-    double du = A * d.DU0[q] + B * d.DU[q];
-    double dv = A * d.DV0[q] + B * d.DV[q];
-    double dw = A * d.DW0[q] + B * d.DW[q];
-    if (m == 0) { du = 0.0; dv = 0.0; dw = 0.0; }
-    if (p.froude_on && m > 0) {
-      const double duu = sqrt(du * du + dv * dv + dw * dw);
-      if (duu > fu) {
-        const double ang = atan2(dv, du);
-        du = fu * cos(ang);
-        dv = fu * sin(ang);
-        dw = 0.0;
-      }
-    }
-    d.DU[q] = du; d.DV[q] = dv; d.DW[q] = dw;
+  R du = d.DU[q], dv = d.DV[q], dw = d.DW[q];
+  if ((arg & UVW_PROJECT) && m != 0) {
+    double lo[5], hi[5];
+    face_pressures(g, d.P, q, lo);
+    face_pressures(g, d.P, q + (long)g.Mloc * g.Nloc, hi);
+    project_cell(g, d, c, k, lo, hi, du, dv, dw);
   }
+  blend_cell(p, arg >> 8, m, sqrt(kGrav * Dd) * p.froude_cap * Dd, d.DU0[q], d.DV0[q], d.DW0[q], du, dv, dw);
+  d.DU[q] = du; d.DV[q] = dv; d.DW[q] = dw;
 }
 
 // ----------------------------------------------------------------------------
@@ -905,8 +1022,14 @@ __device__ __forceinline__ void rk_blend_body(const Geo &g, const Par &p, const 
 template <class R>
 __device__ __forceinline__ void omega_x_body(const Geo &g, const Par &p, const DevT<R> &d, long t, int arg) {
   const int wpr = (g.M + 1 + kXFaces - 1) / kXFaces;
-  const long w = t >> 6;
-  if (w >= (long)wpr * g.N) return;  // whole wavefronts leave together
+  // arg: parts the levels are split into (0: one); a part's wavefronts follow
+  // those of the part before
+  const int parts = max(arg, 1);
+  const long rows = (long)wpr * g.N, wave = t >> 6;
+  if (wave >= rows * parts) return;  // whole wavefronts leave together
+  const int part = (int)(wave / rows);
+  const long w = wave - part * rows;
+  const int ka = g.Kbeg + part * g.K / parts, kb = g.Kbeg + (part + 1) * g.K / parts;
   const int lane = (int)(t & 63);
   const int j = g.Jbeg + (int)(w / wpr);
   const int i = g.Ibeg - 2 + (int)(w % wpr) * kXFaces + lane;
@@ -930,11 +1053,11 @@ __device__ __forceinline__ void omega_x_body(const Geo &g, const Par &p, const D
   if (leftOv) { etaL = em1; DL = d.D[c2m1]; }
   if (rightOv) { etaR = e0; DR = d.D[c20]; }
   const double pl = sqrt(kGrav * fabs(DL)), pr = sqrt(kGrav * fabs(DR));
-  if (face) {
+  if (face && part == 0) {
     d.EtaxL[g.x2(i, j)] = etaL;
     d.EtaxR[g.x2(i, j)] = etaR;
   }
-  for (int k = g.Kbeg; k <= g.Kend; ++k) {
+  for (int k = ka; k < kb; ++k) {
     const long c0 = g.c3(ic, j, k);
     auto recon = [&](const R *F, double &qL, double &qR) {
       const double c = F[c0];
@@ -960,12 +1083,13 @@ __device__ __forceinline__ void omega_x_body(const Geo &g, const Par &p, const D
 
 template <class R>
 __device__ __forceinline__ void omega_y_body(const Geo &g, const Par &p, const DevT<R> &d, long t, int arg) {
-  if (t >= flux_y_threads(g)) return;
+  const int faces = arg > 0 ? arg : kYFaces;  // faces a thread walks
+  if (t >= flux_y_threads(g, faces)) return;
   const int i = g.Ibeg + (int)(t % g.M);
   const long r = t / g.M;
   const int k = g.Kbeg + (int)(r % g.K);
-  const int jf0 = g.Jbeg + (int)(r / g.K) * kYFaces;
-  const int jf1 = min(jf0 + kYFaces - 1, g.Jend1);
+  const int jf0 = g.Jbeg + (int)(r / g.K) * faces;
+  const int jf1 = min(jf0 + faces - 1, g.Jend1);
   const double dy = g.dy, hdy = 0.5 * dy, MinDep = p.min_dep;
   const long sj = g.Mloc;
   const R *const Fl[2] = {d.V, d.DV};
@@ -1210,6 +1334,27 @@ __device__ __forceinline__ void wind_body(const Geo &g, const Par &p, const DevT
   d.Wsy[c] = (double)0.001293f * cds * wv * wds;
 }
 
+// the end of update_mask (pass B), update_wind and update_vars in one pass
+// over all cells: one launch where the step had two and five copies, which at
+// small grids cost a launch each
+template <class R>
+__device__ __forceinline__ void begin_body(const Geo &g, const Par &p, const DevT<R> &d, long t, int arg) {
+  if (t < g.n3()) {
+    d.DU0[t] = d.DU[t];
+    d.DV0[t] = d.DV[t];
+    d.DW0[t] = d.DW[t];
+  }
+  if (t >= g.n2()) return;
+  const int i = 1 + (int)(t % g.Mloc), j = 1 + (int)(t / g.Mloc);
+  if (i >= g.Ibeg && i <= g.Iend && j >= g.Jbeg && j <= g.Jend) {
+    const long c = (i - g.Ibeg) + (long)g.M * (j - g.Jbeg);
+    mask_b_body<R>(g, p, d, c, 0);
+    wind_body<R>(g, p, d, c, 0);
+  }
+  d.D0[t] = d.D[t];
+  d.Eta0[t] = d.Eta[t];
+}
+
 // initial, src/initialize.F:3118-3153: mask, dry Eta, over all cells
 __global__ void k_init_mask(Geo g, Par p, Dev d) {
   long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1282,8 +1427,10 @@ __global__ void k_p_from_x(Geo g, const double *__restrict__ x, Dev d, int zl) {
 // XCD = 1: the single-scenario kernel takes its blocks in XCD-aware order, so
 // the neighbouring rows and planes its stencil reads are mostly worked by the
 // same XCD and found in its L2.  Measured per kernel at 1024x1024x10: it pays
-// for projection (176 -> 109 us) and the Omega column sweep (65 -> 55 us) and
-// costs the sigma-face fluxes (190 -> 225 us); the others are unchanged.
+// for the projection (momenta; 176 -> 109 us) and the Omega column sweep (65 ->
+// 55 us) and costs the sigma-face fluxes (190 -> 225 us), the y sweeps (99 ->
+// 104 and 240 -> 246 us) and the velocity pass (318 -> 330 us); the others are
+// unchanged.
 #define NHW_KERNELS(NAME, XCD)                                                                  \
   template <class R>                                                                            \
   __global__ __launch_bounds__(256) void k_##NAME(Geo g, Par p, DevT<R> d, int arg) {          \
@@ -1300,18 +1447,40 @@ NHW_KERNELS(flux_x, 0)
 NHW_KERNELS(flux_y, 0)
 NHW_KERNELS(flux_z, 0)
 NHW_KERNELS(source_terms, 0)
-NHW_KERNELS(eval_explicit, 0)
+NHW_KERNELS(eval_explicit, 1)
 NHW_KERNELS(eta_slopes, 0)
-NHW_KERNELS(uvw_a, 0)
+template <class R, int MODE>
+__global__ __launch_bounds__(256) void k_uvw_a(Geo g, Par p, DevT<R> d, int arg) {
+  uvw_a_body<R, MODE>(g, p, d, (long)blockIdx.x * blockDim.x + threadIdx.x, arg);
+}
+template <class R, int MODE>
+__global__ __launch_bounds__(256) void kb_uvw_a(BTab<R> T, int arg) {
+  const BPos b = bfind(T);
+  const BScn<R> &S = T.scn[b.s];
+  uvw_a_body<R, MODE>(S.g, S.p, S.d, b.b * blockDim.x + threadIdx.x, arg);
+}
+// calls `run` with the mode (as an integral constant) of flags `f`; `plain`:
+// the scenario takes a mode of its own
+static bool uvw_plain(const nhw_ctx *c) { return mirror_walls(c->p) && c->g.K != 3; }
+template <class Run>
+static void uvw_mode(int f, bool plain, Run run) {
+  using std::integral_constant;
+  constexpr int D = UVW_DIVIDE, DB = D | UVW_BLEND, DBP = DB | UVW_PROJECT;
+  const int what = f & DBP;
+  if (plain && what == D) run(integral_constant<int, D>());
+  else if (plain && what == DB) run(integral_constant<int, DB>());
+  else if (plain && what == DBP) run(integral_constant<int, DBP>());
+  else run(integral_constant<int, 0>());
+}
 NHW_KERNELS(uvw_b, 0)
-NHW_KERNELS(projection, 1)
-NHW_KERNELS(rk_blend, 0)
+NHW_KERNELS(momenta, 1)
 NHW_KERNELS(omega_x, 0)
 NHW_KERNELS(omega_y, 0)
 NHW_KERNELS(omega_col, 1)
 NHW_KERNELS(mask_a, 0)
 NHW_KERNELS(mask_b, 0)
 NHW_KERNELS(wind, 0)
+NHW_KERNELS(begin, 0)
 #undef NHW_KERNELS
 
 // ----------------------------------------------------------------------------
@@ -1341,12 +1510,23 @@ NHW_KERNELS(wind, 0)
 
 static int post(const char *what) { return hip_check(hipGetLastError(), what); }
 
+static void launch_uvw_a(nhw_ctx *c, int flags) {
+  const Geo &g = c->g;
+  const long n = (long)g.M * g.N * level_groups(g);
+  uvw_mode(flags, uvw_plain(c), [&](auto mode) {
+    if (c->mixed)
+      LAUNCH(KID_UVW_A, (k_uvw_a<float, decltype(mode)::value>), n, g, c->p, view<float>(c->d), flags);
+    else
+      LAUNCH(KID_UVW_A, (k_uvw_a<double, decltype(mode)::value>), n, g, c->p, c->d, flags);
+  });
+}
+
 int launch_initial(nhw_ctx *c) {
   const Geo &g = c->g;
   LAUNCH(KID_MASK, k_init_mask, g.n2(), g, c->p, c->d);
   LAUNCH(KID_MASK, k_init_eta_ghost, g.n2(), g, c->d);
   LAUNCH(KID_MASK, k_init_eta0_d, g.n2(), g, c->p, c->d);
-  LAUNCH_R(KID_UVW_A, k_uvw_a, (long)g.M * g.N, g, c->p, dv, 0);
+  launch_uvw_a(c, 0);
   if (int rc = launch_east_ghosts(c)) return rc;
   LAUNCH_R(KID_UVW_B, k_uvw_b, (long)g.M * g.N, g, c->p, dv, 0);
   LAUNCH_R(KID_RK_BLEND, k_init_du, g.n3(), g, dv);
@@ -1355,7 +1535,7 @@ int launch_initial(nhw_ctx *c) {
 
 int launch_estimate_dt(nhw_ctx *c) {
   const Geo &g = c->g;
-  const int nblk = 1024;
+  const int nblk = (int)std::min<long>(1024, nblocks(g.neq(), 256));
   {
     Timed t(c, KID_DT);
     if (c->mixed)
@@ -1463,27 +1643,57 @@ int launch_source_terms(nhw_ctx *c) {
   return post("source_terms");
 }
 
+// update_mask, update_wind and update_vars of the driver's step
+int launch_begin_step(nhw_ctx *c) {
+  const Geo &g = c->g;
+  int rc = launch_flux_lr_history(c);
+  if (rc) return rc;
+  LAUNCH_R(KID_MASK, k_mask_a, g.n2(), g, c->p, dv, 0);
+  LAUNCH_R(KID_KMISC, k_begin, g.n3(), g, c->p, dv, 0);
+  rc = post("begin step");
+  std::swap(c->d.Mask, c->d.MaskNew);
+  return rc;
+}
+
 int launch_fluxes(nhw_ctx *c) {
   const Geo &g = c->g;
-  LAUNCH_R(KID_FLUX_X, k_flux_x, flux_x_threads(g), g, c->p, dv, 0);
-  LAUNCH_R(KID_FLUX_Y, k_flux_y, flux_y_threads(g), g, c->p, dv, 0);
-  LAUNCH_R(KID_FLUX_Z, k_flux_z, (long)g.M * g.N, g, c->p, dv, 0);
+  const int px = level_parts(g, flux_x_threads(g)), fy = row_faces(g), pz = level_parts(g, (long)g.M * g.N);
+  LAUNCH_R(KID_FLUX_X, k_flux_x, flux_x_threads(g, px), g, c->p, dv, px);
+  LAUNCH_R(KID_FLUX_Y, k_flux_y, flux_y_threads(g, fy), g, c->p, dv, fy);
+  LAUNCH_R(KID_FLUX_Z, k_flux_z, (long)g.M * g.N * pz, g, c->p, dv, pz);
   return post("fluxes");
 }
 
 int launch_eval_explicit(nhw_ctx *c, int istep) {
   const Geo &g = c->g;
-  LAUNCH_R(KID_EXPLICIT, k_eval_explicit, (long)g.M * g.N, g, c->p, dv, istep);
-  LAUNCH_R(KID_SOURCE, k_eta_slopes, (long)g.M * g.N, g, c->p, dv, 0);
+  LAUNCH_R(KID_EXPLICIT, k_eval_explicit, explicit_threads(g, c->p), g, c->p, dv, istep);
+  // the viscous solves read the slopes before the velocity pass, which forms
+  // them otherwise
+  if (c->p.viscous) LAUNCH_R(KID_SOURCE, k_eta_slopes, (long)g.M * g.N, g, c->p, dv, 0);
   return post("eval_duvw");
 }
 
-int launch_get_uvw(nhw_ctx *c) {
+static int uvw_pass(nhw_ctx *c, int flags) {
   const Geo &g = c->g;
-  LAUNCH_R(KID_UVW_A, k_uvw_a, (long)g.M * g.N, g, c->p, dv, 1);
+  launch_uvw_a(c, flags);
   if (int rc = launch_east_ghosts(c)) return rc;
   LAUNCH_R(KID_UVW_B, k_uvw_b, (long)g.M * g.N, g, c->p, dv, 0);
   return post("get_UVW");
+}
+// get_UVW before the pressure solve, with the surface slopes of the new Eta
+int launch_get_uvw(nhw_ctx *c) { return uvw_pass(c, UVW_DIVIDE | (c->p.viscous ? 0 : UVW_SLOPES)); }
+
+// the end of a stage: projection (non-hydrostatic), SSP-RK blend, get_UVW
+int launch_end_stage(nhw_ctx *c, int istep) {
+  const Geo &g = c->g;
+  const Par &p = c->p;
+  const int mom = UVW_BLEND | (p.non_hydro ? UVW_PROJECT : 0) | istep << 8;
+  const int slopes = !p.non_hydro && !p.viscous ? UVW_SLOPES : 0;
+  if (wall_friction(p)) {
+    LAUNCH_R(KID_PROJECTION, k_momenta, g.neq(), g, p, dv, mom);
+    return uvw_pass(c, UVW_DIVIDE | slopes);
+  }
+  return uvw_pass(c, UVW_DIVIDE | slopes | mom);
 }
 
 int launch_p_from_x(nhw_ctx *c, const double *x) {
@@ -1492,22 +1702,11 @@ int launch_p_from_x(nhw_ctx *c, const double *x) {
   return post("poisson P");
 }
 
-int launch_projection(nhw_ctx *c) {
-  const Geo &g = c->g;
-  LAUNCH_R(KID_PROJECTION, k_projection, g.neq(), g, c->p, dv, 0);
-  return post("projection_corrector");
-}
-
-int launch_rk_blend(nhw_ctx *c, int istep) {
-  const Geo &g = c->g;
-  LAUNCH_R(KID_RK_BLEND, k_rk_blend, (long)g.M * g.N, g, c->p, dv, istep);
-  return post("rk blend");
-}
-
 int launch_get_omega(nhw_ctx *c) {
   const Geo &g = c->g;
-  LAUNCH_R(KID_OMEGA_X, k_omega_x, flux_x_threads(g), g, c->p, dv, 0);
-  LAUNCH_R(KID_OMEGA_Y, k_omega_y, flux_y_threads(g), g, c->p, dv, 0);
+  const int px = level_parts(g, flux_x_threads(g)), fy = row_faces(g);
+  LAUNCH_R(KID_OMEGA_X, k_omega_x, flux_x_threads(g, px), g, c->p, dv, px);
+  LAUNCH_R(KID_OMEGA_Y, k_omega_y, flux_y_threads(g, fy), g, c->p, dv, fy);
   LAUNCH_R(KID_OMEGA_COL, k_omega_col, (long)g.M * g.N, g, c->p, dv, 0);
   return post("get_Omega");
 }
@@ -1701,25 +1900,43 @@ int blaunch_fluxes(Batch *B) {
 }
 
 int blaunch_eval_explicit(Batch *B, int istep) {
-  BLAUNCH(KID_EXPLICIT, kb_eval_explicit, bshape(B, "c2/256"), istep);
-  BLAUNCH(KID_SOURCE, kb_eta_slopes, bshape(B, "c2/256"), 0);
+  BLAUNCH(KID_EXPLICIT, kb_eval_explicit, bshape(B, "ex/256"), istep);
+  BLAUNCH(KID_SOURCE, kb_eta_slopes, bshape(B, "vs/256"), 0);
   return bpost("batch eval_duvw");
 }
 
-int blaunch_get_uvw(Batch *B) {
-  BLAUNCH(KID_UVW_A, kb_uvw_a, tuned(B, "c2", BT_UVW_A), 1);
+static void blaunch_uvw_a(Batch *B, int flags) {
+  const BShape &S = tuned(B, "lg", BT_UVW_A);
+  bool plain = true;
+  for (nhw_ctx *c : B->m) plain = plain && uvw_plain(c);
+  Timed t(B->lead, KID_UVW_A, bbytes(B, KID_UVW_A));
+  uvw_mode(flags, plain, [&](auto mode) {
+    if (B->mixed)
+      hipLaunchKernelGGL((kb_uvw_a<float, decltype(mode)::value>), dim3(S.nblk), dim3(S.bs), 0, B->lead->stream,
+                         btab<float>(B, S), flags);
+    else
+      hipLaunchKernelGGL((kb_uvw_a<double, decltype(mode)::value>), dim3(S.nblk), dim3(S.bs), 0, B->lead->stream,
+                         btab<double>(B, S), flags);
+  });
+}
+static int buvw_pass(Batch *B, int flags) {
+  blaunch_uvw_a(B, flags);
   BLAUNCH(KID_UVW_B, kb_uvw_b, tuned(B, "c2", BT_UVW_B), 0);
   return bpost("batch get_UVW");
 }
-
-int blaunch_projection(Batch *B) {
-  BLAUNCH(KID_PROJECTION, kb_projection, bshape(B, "c3/256"), 0);
-  return bpost("batch projection_corrector");
-}
-
-int blaunch_rk_blend(Batch *B, int istep) {
-  BLAUNCH(KID_RK_BLEND, kb_rk_blend, bshape(B, "c2/256"), istep);
-  return bpost("batch rk blend");
+// as launch_get_uvw and launch_end_stage; the slopes a viscous member has
+// already formed come out the same again
+int blaunch_get_uvw(Batch *B) { return buvw_pass(B, UVW_DIVIDE | UVW_SLOPES); }
+int blaunch_end_stage(Batch *B, int istep) {
+  const int mom = UVW_BLEND | (B->non_hydro ? UVW_PROJECT : 0) | istep << 8;
+  const int slopes = B->non_hydro ? 0 : UVW_SLOPES;
+  bool friction = false;
+  for (nhw_ctx *c : B->m) friction = friction || wall_friction(c->p);
+  if (friction) {
+    BLAUNCH(KID_PROJECTION, kb_momenta, bshape(B, "c3/256"), mom);
+    return buvw_pass(B, UVW_DIVIDE | slopes);
+  }
+  return buvw_pass(B, UVW_DIVIDE | slopes | mom);
 }
 
 int blaunch_get_omega(Batch *B) {
@@ -1803,7 +2020,7 @@ int batch_autotune(Batch *B) {
           case BT_FLUX_Z: BLAUNCH(KID_FLUX_Z, kb_flux_z, tuned(B, "fz", kind), 0); break;
           case BT_OMEGA_X: BLAUNCH(KID_OMEGA_X, kb_omega_x, tuned(B, "fx", kind), 0); break;
           case BT_OMEGA_Y: BLAUNCH(KID_OMEGA_Y, kb_omega_y, tuned(B, "fy", kind), 0); break;
-          case BT_UVW_A: BLAUNCH(KID_UVW_A, kb_uvw_a, tuned(B, "c2", kind), 1); break;
+          case BT_UVW_A: blaunch_uvw_a(B, UVW_DIVIDE); break;
           default: BLAUNCH(KID_UVW_B, kb_uvw_b, tuned(B, "c2", kind), 0); break;
         }
         (void)hipEventRecord(e1, st);

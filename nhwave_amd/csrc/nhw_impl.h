@@ -83,18 +83,41 @@ struct Geo {
   __host__ __device__ long neq() const { return (long)M * N * K; }
 };
 
-// Thread counts of the x- and y-face flux kernels: the x kernel gives each
-// row of faces wavefronts of 64 lanes covering kXFaces faces each (each lane
-// walks the sigma levels); the y kernel gives each (i, k) threads walking
-// kYFaces faces of increasing j.
+// Thread counts of the face and column sweeps.  The x-face kernels give each
+// row of faces wavefronts of 64 lanes covering kXFaces faces each, and the
+// sigma levels in `parts` parts; the y-face kernels give each (i, k) threads
+// walking `faces` faces of increasing j; the sigma-face kernel gives each
+// column `parts` threads.
 constexpr int kXFaces = 62;
 constexpr int kYFaces = 16;
-__host__ __device__ __forceinline__ long flux_x_threads(const Geo &g) {
-  return (long)((g.M + 1 + kXFaces - 1) / kXFaces) * g.N * 64;
+__host__ __device__ __forceinline__ long flux_x_threads(const Geo &g, int parts = 1) {
+  return (long)((g.M + 1 + kXFaces - 1) / kXFaces) * g.N * 64 * parts;
 }
-__host__ __device__ __forceinline__ long flux_y_threads(const Geo &g) {
-  return (long)g.M * g.K * ((g.N + 1 + kYFaces - 1) / kYFaces);
+__host__ __device__ __forceinline__ long flux_y_threads(const Geo &g, int faces = kYFaces) {
+  return (long)g.M * g.K * ((g.N + 1 + faces - 1) / faces);
 }
+// How a sweep is split on one scenario.  A walk over levels or rows loads
+// each value once and forms each slope once, but on a small grid too few
+// threads walk: a thread's chain of loads then sets the time.  The walks are
+// cut until the launch has kFillThreads threads (two waves a SIMD) or one step
+// is left of them; on larger grids the whole walk is the faster one.  x faces,
+// y faces, sigma faces at 257 x 33 x 5: 18, 36 and 8.3 us whole, 7, 8 and 5
+// cut to one step; at 333 x 217 x 7: 28, 36 and 12.7 whole, 20, 24 and 9.7 cut.
+constexpr long kFillThreads = 131072;
+inline int level_parts(const Geo &g, long threads) {
+  const long want = (kFillThreads + threads - 1) / threads;
+  return (int)(want < 1 ? 1 : want > g.K ? g.K : want);
+}
+inline int row_faces(const Geo &g) {
+  int f = kYFaces;
+  while (f > 1 && flux_y_threads(g, f) < kFillThreads) f /= 2;
+  return f;
+}
+// Groups of sigma levels of one column that a thread of the velocity kernel
+// takes: two levels each, so that the two levels a surface or bottom face
+// state reads are one thread's.  With an odd number of levels the second
+// group has one; three levels are one group.
+__host__ __device__ __forceinline__ int level_groups(const Geo &g) { return g.K == 3 ? 1 : (g.K + 1) / 2; }
 
 // inflow and outflow boundaries (BC 3): offset of (j,k) in the (Nloc,Kloc)
 // arrays Uin/Vin/Win_X0 (west) and Uin/Vin/Win_Xn, Uin_Xni (east)
@@ -148,6 +171,17 @@ struct Par {
   double alpha[3], beta[3];
   Wave wave;
 };
+
+// some side has the wall friction boundary (BC 5)
+inline bool wall_friction(const Par &p) {
+  return p.bc_x0 == 5 || p.bc_xn == 5 || p.bc_y0 == 5 || p.bc_yn == 5;
+}
+
+// every side mirrors: free or no slip (BC 1, 2)
+inline bool mirror_walls(const Par &p) {
+  auto mirrors = [](int bc) { return bc == 1 || bc == 2; };
+  return mirrors(p.bc_x0) && mirrors(p.bc_xn) && mirrors(p.bc_y0) && mirrors(p.bc_yn);
+}
 
 // Device pointers of the resident state.  R is the storage type of the 3-D
 // velocity/momentum fields, their stage copies, the face fluxes and Omega:
@@ -382,8 +416,8 @@ int launch_source_terms(nhw_ctx *c);
 int launch_fluxes(nhw_ctx *c);
 int launch_eval_explicit(nhw_ctx *c, int istep);
 int launch_get_uvw(nhw_ctx *c);
-int launch_projection(nhw_ctx *c);
-int launch_rk_blend(nhw_ctx *c, int istep);
+int launch_end_stage(nhw_ctx *c, int istep);
+int launch_begin_step(nhw_ctx *c);
 int launch_get_omega(nhw_ctx *c);
 // boundary forcing (nhw_forcing.hip)
 int forcing_setup(nhw_ctx *c);   // constants and device tables; after the grid
