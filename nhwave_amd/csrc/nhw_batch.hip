@@ -60,20 +60,20 @@ void bshape_add(Batch *B, const std::string &key, const std::vector<long> &items
 // the Krylov and multigrid launch shapes over members `mem` (key prefix pre)
 static void solver_shapes(Batch *B, const std::vector<int> &mem, const std::string &pre, int table) {
   std::vector<long> c2, c3, one;
-  int maxlev = 0;
   for (int u : mem) {
     const Geo &g = B->m[u]->g;
     c2.push_back((long)g.M * g.N);
     c3.push_back(g.neq());
     one.push_back(1);
-    maxlev = std::max(maxlev, (int)(B->mixed ? B->m[u]->mg.lvf : B->m[u]->mg.lv).size());
   }
   bshape_add(B, pre + "c3/256", c3, mem, 256, false, table);
   bshape_add(B, pre + "c2/256", c2, mem, 256, false, table);
   bshape_add(B, pre + "one", one, mem, 256, true, table);
+  // every member's coarsest level, whichever it is: one workgroup (kb_coarse)
+  bshape_add(B, pre + "co", one, mem, kCoarseBS, true, table);
   for (int l = 0; l < kBMaxLev; ++l) {
-    std::vector<long> co, ti, gc;
-    std::vector<int> ico, iti;
+    std::vector<long> ti, gc;
+    std::vector<int> iti;
     long columns = 0;  // of the level's tile launches, all members
     for (int u : mem) {
       const std::vector<MGLevel> &h = B->mixed ? B->m[u]->mg.lvf : B->m[u]->mg.lv;
@@ -82,25 +82,17 @@ static void solver_shapes(Batch *B, const std::vector<int> &mem, const std::stri
     const bool big = mg_big_tiles(columns);
     for (int u : mem) {
       const std::vector<MGLevel> &h = B->mixed ? B->m[u]->mg.lvf : B->m[u]->mg.lv;
-      const int nl = (int)h.size();
-      if (nl <= l) continue;
-      if (nl == l + 1) {  // coarsest: one workgroup (kb_coarse)
-        co.push_back(1);
-        ico.push_back(u);
-        continue;
-      }
+      if ((int)h.size() <= l + 1) continue;
       // one workgroup per tile (kb_mg_down, kb_mg_up)
       ti.push_back(big ? mg_tiles<kTileX, kTileY>(h[l]) : mg_tiles<kTileSX, kTileSY>(h[l]));
       gc.push_back((long)h[l + 1].M * h[l + 1].N);
       iti.push_back(u);
     }
     const std::string L = std::to_string(l);
-    bshape_add(B, pre + "co" + L, co, ico, kCoarseBS, true, table);
     if (big) bshape_add(B, pre + "tb" + L, ti, iti, MgTile<kTileX, kTileY>::NT, true, table);
     else bshape_add(B, pre + "ts" + L, ti, iti, MgTile<kTileSX, kTileSY>::NT, true, table);
     bshape_add(B, pre + "gc" + L, gc, iti, 256, false, table);
   }
-  (void)maxlev;
 }
 
 // device pointers of the shapes of one table after its upload

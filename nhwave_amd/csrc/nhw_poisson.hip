@@ -981,12 +981,17 @@ __device__ __forceinline__ R *lvl_x(const BScn<R> &S, int l, int vout) {
   return l == 0 ? bvec(S, vout) : S.lx[l];
 }
 
-// the coarsest level of each member in one workgroup (coarse_solve)
+// the coarsest level of each member, whichever it is, in one workgroup
+// (coarse_solve).  A launch for each level that is some member's coarsest
+// took as long as this one, one after the other: 11 us each, up to three of
+// them a cycle (24 members of 32 to 96 cells a side and 3 to 6 levels: six
+// steps 82 ms, now 67).
 template <class R, int KM>
-__global__ __launch_bounds__(kCoarseBS) void kb_coarse(BTab<R> T, int l, int vin, int vout, int sweeps) {
+__global__ __launch_bounds__(kCoarseBS) void kb_coarse(BTab<R> T, int vin, int vout, int sweeps) {
   const BPos b = bfind(T);
   const BScn<R> &S = T.scn[b.s];
   if (S.flag[0]) return;
+  const int l = S.nlev - 1;
   __shared__ R xs[KM * kMgCoarseCols];
   by_rows<KM>(S.L[l].K, [&](auto km) {
     coarse_solve<R, decltype(km)::value>(S.L[l], S.G[l], lvl_b(S, l, vin), lvl_x(S, l, vout), sweeps, xs);
@@ -1086,21 +1091,25 @@ static BTab<R> pbtab(Batch *B, const BShape &S) {
 
 static bool has_shape(Batch *B, const std::string &k) { return B->shapes.count(k) > 0; }
 
-// batched V(1,1) cycle on level l: members whose coarsest level is l sweep
-// there; the others go down
+// batched V(1,1) cycle: the members that have a coarser level go down from
+// each level, all members sweep on their coarsest, and up again
 template <class R, int KM>
-static void bvcycle(Batch *B, int l, int vin, int vout) {
-  const std::string L = std::to_string(l), co = "k:co" + L, tb = "k:tb" + L, ts = "k:ts" + L;
-  if (has_shape(B, co))
-    PBL(KID_MG_COARSE, 0.0, (kb_coarse<R, KM>), bshape(B, co), l, vin, vout, B->lead->mg.coarse_sweeps);
-  if (!has_shape(B, tb) && !has_shape(B, ts)) return;
+static void bvcycle(Batch *B, int vin, int vout) {
   const size_t lb = MgTile<kTileX, kTileY>::lds(B->kmax, sizeof(R));
   const size_t ls = MgTile<kTileSX, kTileSY>::lds(B->kmax, sizeof(R));
-  PBLS(KID_MG_DOWN, 0.0, (kb_mg_down<R, KM, kTileX, kTileY>), bshape(B, tb), lb, l, vin);
-  PBLS(KID_MG_DOWN, 0.0, (kb_mg_down<R, KM, kTileSX, kTileSY>), bshape(B, ts), ls, l, vin);
-  bvcycle<R, KM>(B, l + 1, 0, 0);
-  PBLS(KID_MG_UP, 0.0, (kb_mg_up<R, KM, kTileX, kTileY>), bshape(B, tb), lb, l, vin, vout);
-  PBLS(KID_MG_UP, 0.0, (kb_mg_up<R, KM, kTileSX, kTileSY>), bshape(B, ts), ls, l, vin, vout);
+  int l = 0;
+  for (;; ++l) {
+    const std::string L = std::to_string(l), tb = "k:tb" + L, ts = "k:ts" + L;
+    if (!has_shape(B, tb) && !has_shape(B, ts)) break;
+    PBLS(KID_MG_DOWN, 0.0, (kb_mg_down<R, KM, kTileX, kTileY>), bshape(B, tb), lb, l, vin);
+    PBLS(KID_MG_DOWN, 0.0, (kb_mg_down<R, KM, kTileSX, kTileSY>), bshape(B, ts), ls, l, vin);
+  }
+  PBL(KID_MG_COARSE, 0.0, (kb_coarse<R, KM>), bshape(B, "k:co"), vin, vout, B->lead->mg.coarse_sweeps);
+  while (l-- > 0) {
+    const std::string L = std::to_string(l), tb = "k:tb" + L, ts = "k:ts" + L;
+    PBLS(KID_MG_UP, 0.0, (kb_mg_up<R, KM, kTileX, kTileY>), bshape(B, tb), lb, l, vin, vout);
+    PBLS(KID_MG_UP, 0.0, (kb_mg_up<R, KM, kTileSX, kTileSY>), bshape(B, ts), ls, l, vin, vout);
+  }
 }
 
 // reads every member's Krylov flag; returns how many are still running
@@ -1140,11 +1149,11 @@ static int bbicgstab(Batch *B, const std::vector<int> &round, int *iters_out) {
     for (int q = 0; q < chunk; ++q) {
       const BShape &rows = bshape(B, "k:c3/256"), &cols = bshape(B, "k:c2/256"), &one = bshape(B, "k:one");
       PBL(KID_KVEC, 0.0, kb_pvec<R>, rows);
-      bvcycle<R, KM>(B, 0, BV_P, BV_PH);
+      bvcycle<R, KM>(B, BV_P, BV_PH);
       PBL(KID_MF_V, 0.0, (kb_mf_apply<R, 1>), cols, BV_PH, BV_V, BV_RH, part);
       PBL(KID_KREDUCE, 0.0, kb_fin<R>, one, cols.off, (const double *)part, 1);
       PBL(KID_KVEC, 0.0, kb_svec<R>, rows);
-      bvcycle<R, KM>(B, 0, BV_S, BV_SH);
+      bvcycle<R, KM>(B, BV_S, BV_SH);
       PBL(KID_MF_T, 0.0, (kb_mf_apply<R, 2>), cols, BV_SH, BV_T, BV_S, part);
       PBL(KID_KREDUCE, 0.0, kb_fin<R>, one, cols.off, (const double *)part, 2);
       PBL(KID_KUPDATE, 0.0, kb_update<R>, rows, part);
