@@ -181,7 +181,9 @@ static int batch_build(Batch *B) {
   B->shapes.clear();
   B->ibuf_h.clear();
   B->kbuf_h.clear();
-  std::vector<long> fx, fy, fz, c2, c3, a2, a3, one, ex, lg;
+  std::vector<long> fx, fy, fz, c2, c3, a2, a3, one, ex, lg[2];
+  std::vector<int> lgi[2];  // plain members of the velocity pass, the others
+  int at = 0;
   for (nhw_ctx *c : B->m) {
     const Geo &g = c->g;
     fx.push_back(flux_x_threads(g));
@@ -190,7 +192,9 @@ static int batch_build(Batch *B) {
     c2.push_back((long)g.M * g.N);
     c3.push_back(g.neq());
     ex.push_back((long)g.M * g.N * (c->p.viscous ? 1 : 1 + g.K));  // mass columns, momentum cells
-    lg.push_back((long)g.M * g.N * level_groups(g));
+    const int form = uvw_plain(g, c->p) ? 0 : 1;
+    lg[form].push_back((long)g.M * g.N * level_groups(g));
+    lgi[form].push_back(at++);
     a2.push_back(g.n2());
     a3.push_back(g.n3());
     one.push_back(1);
@@ -202,7 +206,8 @@ static int batch_build(Batch *B) {
     bshape_add(B, "fy" + s, fy, all, bs);
     bshape_add(B, "fz" + s, fz, all, bs);
     bshape_add(B, "c2" + s, c2, all, bs);
-    bshape_add(B, "lg" + s, lg, all, bs);
+    bshape_add(B, "lg" + s, lg[0], lgi[0], bs);
+    bshape_add(B, "lx" + s, lg[1], lgi[1], bs);
   }
   bshape_add(B, "c3/256", c3, all, 256);
   bshape_add(B, "ex/256", ex, all, 256);

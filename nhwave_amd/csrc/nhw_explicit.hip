@@ -1461,7 +1461,6 @@ __global__ __launch_bounds__(256) void kb_uvw_a(BTab<R> T, int arg) {
 }
 // calls `run` with the mode (as an integral constant) of flags `f`; `plain`:
 // the scenario takes a mode of its own
-static bool uvw_plain(const nhw_ctx *c) { return mirror_walls(c->p) && c->g.K != 3; }
 template <class Run>
 static void uvw_mode(int f, bool plain, Run run) {
   using std::integral_constant;
@@ -1513,7 +1512,7 @@ static int post(const char *what) { return hip_check(hipGetLastError(), what); }
 static void launch_uvw_a(nhw_ctx *c, int flags) {
   const Geo &g = c->g;
   const long n = (long)g.M * g.N * level_groups(g);
-  uvw_mode(flags, uvw_plain(c), [&](auto mode) {
+  uvw_mode(flags, uvw_plain(g, c->p), [&](auto mode) {
     if (c->mixed)
       LAUNCH(KID_UVW_A, (k_uvw_a<float, decltype(mode)::value>), n, g, c->p, view<float>(c->d), flags);
     else
@@ -1905,19 +1904,21 @@ int blaunch_eval_explicit(Batch *B, int istep) {
   return bpost("batch eval_duvw");
 }
 
+// the plain members in their own form, the others in the general one
 static void blaunch_uvw_a(Batch *B, int flags) {
-  const BShape &S = tuned(B, "lg", BT_UVW_A);
-  bool plain = true;
-  for (nhw_ctx *c : B->m) plain = plain && uvw_plain(c);
   Timed t(B->lead, KID_UVW_A, bbytes(B, KID_UVW_A));
-  uvw_mode(flags, plain, [&](auto mode) {
-    if (B->mixed)
-      hipLaunchKernelGGL((kb_uvw_a<float, decltype(mode)::value>), dim3(S.nblk), dim3(S.bs), 0, B->lead->stream,
-                         btab<float>(B, S), flags);
-    else
-      hipLaunchKernelGGL((kb_uvw_a<double, decltype(mode)::value>), dim3(S.nblk), dim3(S.bs), 0, B->lead->stream,
-                         btab<double>(B, S), flags);
-  });
+  for (const bool plain : {true, false}) {
+    const BShape &S = tuned(B, plain ? "lg" : "lx", BT_UVW_A);
+    if (S.nblk == 0) continue;
+    uvw_mode(flags, plain, [&](auto mode) {
+      if (B->mixed)
+        hipLaunchKernelGGL((kb_uvw_a<float, decltype(mode)::value>), dim3(S.nblk), dim3(S.bs), 0, B->lead->stream,
+                           btab<float>(B, S), flags);
+      else
+        hipLaunchKernelGGL((kb_uvw_a<double, decltype(mode)::value>), dim3(S.nblk), dim3(S.bs), 0, B->lead->stream,
+                           btab<double>(B, S), flags);
+    });
+  }
 }
 static int buvw_pass(Batch *B, int flags) {
   blaunch_uvw_a(B, flags);

@@ -183,6 +183,10 @@ inline bool mirror_walls(const Par &p) {
   return mirrors(p.bc_x0) && mirrors(p.bc_xn) && mirrors(p.bc_y0) && mirrors(p.bc_yn);
 }
 
+// the velocity pass has forms of its own (k_uvw_a) for mirroring walls and
+// groups of at most two levels
+inline bool uvw_plain(const Geo &g, const Par &p) { return mirror_walls(p) && g.K != 3; }
+
 // Device pointers of the resident state.  R is the storage type of the 3-D
 // velocity/momentum fields, their stage copies, the face fluxes and Omega:
 // double in the plain form, float in the mixed form.  Depth, Eta and every
