@@ -10,7 +10,7 @@ constexpr int kBS = 256;  // threads per block of the Krylov kernels
 constexpr double kInnerTol = 1e-4;  // relative residual reduction of one FP32 inner solve
 constexpr int kMaxRefine = 20;      // refinement rounds of the mixed form
 
-enum { S_RHO = 0, S_ALPHA, S_OMEGA, S_BETA, S_BB, S_RR, S_RHV, S_TS, S_TT, S_TRUE, S_REF, S_ITOL, S_N };
+enum { S_RHO = 0, S_ALPHA, S_OMEGA, S_BETA, S_BB, S_RR, S_RHV, S_TS, S_TT, S_TRUE, S_REF, S_ITOL, S_RHOP, S_N };
 
 // scalars and flags of one solve.  flag[0]: 0 running, 1 converged,
 // 2 breakdown, 3 ITMAX reached, 4 zero right-hand side; flag[1]: iterations;
@@ -58,6 +58,34 @@ __device__ __forceinline__ double final_sum(const double *part, int m, long b0, 
   return out;
 }
 
+// final_sum of at most kFuseParts partials, the same additions in the same
+// order, by every wavefront on its own: no barrier, and the sum in all of its
+// lanes.  A kernel that needs a scalar of the iteration forms it like this in
+// each of its wavefronts, where a launch of one workgroup had done it.  The
+// constructor only asks for the partials; other loads may follow before sum().
+constexpr int kFuseParts = 512;
+struct WaveSum {
+  double v[2][4];
+  __device__ __forceinline__ WaveSum(const double *part, int m, int nblk) {
+#pragma unroll
+    for (int i = 0; i < kFuseParts / kBS; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int b = (int)(threadIdx.x & 63) + 64 * q + kBS * i;
+        v[i][q] = b < nblk ? part[3 * b + m] : 0.0;
+      }
+  }
+  __device__ __forceinline__ double sum() const {
+    double a[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) a[q] = (0.0 + v[0][q]) + v[1][q];
+    double s = (a[0] + a[2]) + (a[1] + a[3]);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) s += __shfl_down(s, d, 64);
+    return __shfl(s, 0, 64);
+  }
+};
+
 // start of a solve: rr = |r0|^2, bb = |b|^2
 __device__ __forceinline__ void fin0_logic(const KScal &k, double rr, double bb) {
   k.sc[S_RR] = rr; k.sc[S_BB] = bb; k.sc[S_RHO] = rr; k.sc[S_TRUE] = rr;
@@ -74,33 +102,57 @@ __device__ __forceinline__ void fin0_logic(const KScal &k, double rr, double bb)
   else k.flag[0] = 0;
 }
 
+// The logic after the dots of an iteration.  Each returns the scalar that the
+// kernels after it use and whether they run.  Where it is formed by every
+// wavefront of a launch, all come to the same answer and one thread (`write`)
+// records it; it writes nothing the others read but flag[0], which may make a
+// wavefront that starts late leave early: after a stop nothing the launch
+// writes is used, or the launch leaves by the returned `go`.
+
 // alpha = rho / (rh, v)
-__device__ __forceinline__ void fin1_logic(const KScal &k, double rhv) {
-  k.sc[S_RHV] = rhv;
-  if (rhv == 0.0 || !(rhv == rhv)) { k.flag[0] = 2; k.flag[2] = 2; return; }
-  k.sc[S_ALPHA] = k.sc[S_RHO] / rhv;
+__device__ __forceinline__ bool fin1_logic(const KScal &k, double rhv, double &alpha, bool write = true) {
+  if (write) k.sc[S_RHV] = rhv;
+  if (rhv == 0.0 || !(rhv == rhv)) {
+    if (write) { k.flag[0] = 2; k.flag[2] = 2; }
+    return false;
+  }
+  alpha = k.sc[S_RHO] / rhv;
+  if (write) k.sc[S_ALPHA] = alpha;
+  return true;
 }
 
-// omega = (t, s) / (t, t)
-__device__ __forceinline__ void fin2_logic(const KScal &k, double ts, double tt) {
-  k.sc[S_TS] = ts; k.sc[S_TT] = tt;
+// omega = (t, s) / (t, t); keeps rho for fin3_logic, which replaces it
+__device__ __forceinline__ bool fin2_logic(const KScal &k, double ts, double tt, double &omega, bool write = true) {
   // tt == 0 means s == 0: the half step already solves the system
-  k.sc[S_OMEGA] = tt == 0.0 ? 0.0 : ts / tt;
-  if (!(tt == tt)) { k.flag[0] = 2; k.flag[2] = 3; }
+  omega = tt == 0.0 ? 0.0 : ts / tt;
+  const bool go = tt == tt;
+  if (write) {
+    k.sc[S_TS] = ts; k.sc[S_TT] = tt;
+    k.sc[S_OMEGA] = omega;
+    k.sc[S_RHOP] = k.sc[S_RHO];
+    if (!go) { k.flag[0] = 2; k.flag[2] = 3; }
+  }
+  return go;
 }
 
 // convergence test and beta after the update; rhr = (rh, r), rr = |r|^2
-__device__ __forceinline__ void fin3_logic(const KScal &k, double rhr, double rr) {
-  const int it = k.flag[1] + 1;
-  k.flag[1] = it;
-  k.sc[S_RR] = rr;
+__device__ __forceinline__ bool fin3_logic(const KScal &k, double rhr, double rr, double &beta, bool write = true) {
   const double omega = k.sc[S_OMEGA];
-  if (!(rr == rr)) { k.flag[0] = 2; k.flag[2] = 4; return; }
-  if (rr <= (k.inner ? k.sc[S_ITOL] : k.tol2) * k.sc[S_REF]) { k.flag[0] = 1; return; }
-  if (it >= k.itmax) { k.flag[0] = 3; return; }
-  if (rhr == 0.0 || omega == 0.0) { k.flag[0] = 2; k.flag[2] = 5; return; }
-  k.sc[S_BETA] = (rhr / k.sc[S_RHO]) * (k.sc[S_ALPHA] / omega);
-  k.sc[S_RHO] = rhr;
+  int stop = 0, code = 0;
+  if (!(rr == rr)) { stop = 2; code = 4; }
+  else if (rr <= (k.inner ? k.sc[S_ITOL] : k.tol2) * k.sc[S_REF]) stop = 1;
+  else if (write && k.flag[1] + 1 >= k.itmax) stop = 3;
+  else if (rhr == 0.0 || omega == 0.0) { stop = 2; code = 5; }
+  if (write) {
+    k.flag[1] = k.flag[1] + 1;
+    k.sc[S_RR] = rr;
+    if (stop) k.flag[0] = stop;
+    if (code) k.flag[2] = code;
+  }
+  if (stop) return false;
+  beta = (rhr / k.sc[S_RHOP]) * (k.sc[S_ALPHA] / omega);
+  if (write) { k.sc[S_BETA] = beta; k.sc[S_RHO] = rhr; }
+  return true;
 }
 
 }  // namespace nhw

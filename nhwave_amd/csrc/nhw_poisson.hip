@@ -135,7 +135,7 @@ struct KVT {
   const double *b;
   V *x, *r, *rh, *p, *v, *s, *t, *ph, *sh;
   double *lu_c, *lu_d;
-  double *part, *sc;
+  double *part, *part2, *sc;  // partials of the dots, of the update's
   int *flag;
   int itmax;
   double tol2, itol2;
@@ -188,37 +188,133 @@ __global__ void k_line_factor(KV k) {
   }
 }
 
-// z = M^-1 y on one column (y already stored in z)
-__device__ __forceinline__ void line_solve(const KV &k, long col, double *z) {
-  const double *c13 = k.coef + 12 * k.n;
-  double gp = 0.0;
-  for (int kk = 0; kk < k.K; ++kk) {
-    const long r = col + kk * k.MN;
-    const double gv = (kk == 0 ? z[r] : z[r] - c13[r] * gp) * k.lu_d[r];
-    z[r] = gv;
-    gp = gv;
+// The line preconditioner, z = M^-1 y with y = rhs(a, b, c) row by row.  What a
+// launch over a few columns takes is its waits for memory, one after the
+// other.  So a workgroup takes few columns (over as many CUs as there are)
+// and asks for everything they need at once, all of its threads together;
+// one lane a column then walks the levels in the LDS.  880 columns x 20
+// levels: 13.6 us with a thread a column in memory, now 6.3 to 7, the
+// reduction before it (3.2 us by itself) included; 9 to 10 with the levels of a
+// column in one lane's registers, whose code alone is 24 KB read once.
+// Columns too long for the LDS walk in memory.
+constexpr int kLineBS = 256;
+constexpr int kLineCols = 16;           // columns a workgroup, fewer of long ones
+constexpr long kLineLds = 64 * 1024;    // bytes
+inline int line_cols(int K) {
+  int nc = kLineCols;
+  while (nc > 1 && 4L * sizeof(double) * nc * K > kLineLds) nc /= 2;
+  return nc;
+}
+inline size_t line_lds(int K) {
+  const long bytes = 4L * sizeof(double) * line_cols(K) * K;
+  return bytes > kLineLds ? 0 : bytes;
+}
+
+// rows that a thread has in flight at once
+constexpr int kLineRows = 2;
+struct LineRows {
+  double a[kLineRows], b[kLineRows], c[kLineRows], lo[kLineRows], id[kLineRows], up[kLineRows];
+  long r[kLineRows];
+  // rows e0, e0 + kLineBS, .. of the workgroup's nc columns (level by level)
+  __device__ __forceinline__ void load(const KV &k, int e0, int nc, const double *pa, const double *pb,
+                                       const double *pc) {
+    const double *c13 = k.coef + 12 * k.n;
+#pragma unroll
+    for (int q = 0; q < kLineRows; ++q) {
+      const int e = min(e0 + q * kLineBS, nc * k.K - 1), kk = e / nc;
+      r[q] = min((long)blockIdx.x * nc + (e - kk * nc), k.MN - 1) + kk * k.MN;
+      a[q] = pa[r[q]];
+      b[q] = pb[r[q]];
+      c[q] = pc[r[q]];
+      lo[q] = c13[r[q]];
+      id[q] = k.lu_d[r[q]];
+      up[q] = k.lu_c[r[q]];
+    }
   }
-  double zn = gp;
-  for (int kk = k.K - 2; kk >= 0; --kk) {
-    const long r = col + kk * k.MN;
-    zn = z[r] - k.lu_c[r] * zn;
-    z[r] = zn;
+};
+
+// y = rhs(a, b, c), z = M^-1 y of the workgroup's nc columns, whose first
+// rows are loaded; columns past the last repeat it
+template <class Rhs>
+__device__ __forceinline__ void line_lds_solve(const KV &k, int nc, LineRows &L, const double *pa, const double *pb,
+                                               const double *pc, double *y, double *z, Rhs rhs) {
+  extern __shared__ double line_sm[];
+  const int K = k.K, n = nc * K;
+  double *g = line_sm, *lo = g + n, *id = lo + n, *up = id + n;
+  for (int e0 = threadIdx.x; e0 < n; e0 += kLineRows * kLineBS) {
+    if (e0 != (int)threadIdx.x) L.load(k, e0, nc, pa, pb, pc);
+#pragma unroll
+    for (int q = 0; q < kLineRows; ++q) {
+      const int e = e0 + q * kLineBS;
+      if (e >= n) break;
+      const double yv = rhs(L.a[q], L.b[q], L.c[q]);
+      y[L.r[q]] = yv;
+      g[e] = yv; lo[e] = L.lo[q]; id[e] = L.id[q]; up[e] = L.up[q];
+    }
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < nc) {
+    int e = threadIdx.x;
+    double v = g[e] * id[e];
+    g[e] = v;
+#pragma unroll 4
+    for (int kk = 1; kk < K; ++kk) {
+      e += nc;
+      v = (g[e] - lo[e] * v) * id[e];
+      g[e] = v;
+    }
+#pragma unroll 4
+    for (int kk = K - 2; kk >= 0; --kk) {
+      e -= nc;
+      v = g[e] - up[e] * v;
+      g[e] = v;
+    }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < n; e += kLineBS) {
+    const int kk = e / nc;
+    z[min((long)blockIdx.x * nc + (e - kk * nc), k.MN - 1) + kk * k.MN] = g[e];
   }
 }
 
-// p = r + beta*(p - omega*v); ph = M^-1 p
-__global__ void k_prec_p(KV k) {
-  if (k.flag[0]) return;
-  long col = (long)blockIdx.x * blockDim.x + threadIdx.x;
+// the same on one column a lane, in memory
+template <class Rhs>
+__device__ __forceinline__ void line_mem_solve(const KV &k, const double *pa, const double *pb, const double *pc,
+                                               double *y, double *z, Rhs rhs) {
+  const long col = (long)blockIdx.x * kLineBS + threadIdx.x;
   if (col >= k.MN) return;
-  const double beta = k.sc[S_BETA], omega = k.sc[S_OMEGA];
+  const double *c13 = k.coef + 12 * k.n;
+  double v = 0.0;
   for (int kk = 0; kk < k.K; ++kk) {
     const long r = col + kk * k.MN;
-    const double pv = k.r[r] + beta * (k.p[r] - omega * k.v[r]);
-    k.p[r] = pv;
-    k.ph[r] = pv;
+    const double yv = rhs(pa[r], pb[r], pc[r]);
+    y[r] = yv;
+    v = (kk == 0 ? yv : yv - c13[r] * v) * k.lu_d[r];
+    z[r] = v;
   }
-  line_solve(k, col, k.ph);
+  for (int kk = k.K - 2; kk >= 0; --kk) {
+    const long r = col + kk * k.MN;
+    v = z[r] - k.lu_c[r] * v;
+    z[r] = v;
+  }
+}
+
+// nc: columns a workgroup (0: one a lane, in memory); fin > 0: the scalar
+// step before this launch is its own, from `fin` partials
+
+// p = r + beta*(p - omega*v); ph = M^-1 p
+__global__ __launch_bounds__(kLineBS) void k_prec_p(KV k, int nc, int fin) {
+  const int stop = k.flag[0];
+  double beta = k.sc[S_BETA];
+  const double omega = k.sc[S_OMEGA];
+  const WaveSum rhr(k.part2, 0, fin), rr(k.part2, 1, fin);
+  LineRows L;
+  if (nc) L.load(k, threadIdx.x, nc, k.r, k.p, k.v);
+  if (stop) return;
+  if (fin && !fin3_logic(k.scal(), rhr.sum(), rr.sum(), beta, blockIdx.x == 0 && threadIdx.x == 0)) return;
+  auto rhs = [&](double r, double p, double v) { return r + beta * (p - omega * v); };
+  if (nc) line_lds_solve(k, nc, L, k.r, k.p, k.v, k.p, k.ph, rhs);
+  else line_mem_solve(k, k.r, k.p, k.v, k.p, k.ph, rhs);
 }
 
 // v = A ph; partial (rh, v)
@@ -237,22 +333,22 @@ template <class V>
 __global__ void k_fin1(KVT<V> k, int nblk) {
   if (k.flag[0]) return;
   const double rhv = final_sum(k.part, 0, 0, nblk);
-  if (threadIdx.x == 0) fin1_logic(k.scal(), rhv);
+  double alpha;
+  if (threadIdx.x == 0) fin1_logic(k.scal(), rhv, alpha);
 }
 
 // s = r - alpha*v; sh = M^-1 s
-__global__ void k_prec_s(KV k) {
-  if (k.flag[0]) return;
-  long col = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (col >= k.MN) return;
-  const double alpha = k.sc[S_ALPHA];
-  for (int kk = 0; kk < k.K; ++kk) {
-    const long r = col + kk * k.MN;
-    const double sv = k.r[r] - alpha * k.v[r];
-    k.s[r] = sv;
-    k.sh[r] = sv;
-  }
-  line_solve(k, col, k.sh);
+__global__ __launch_bounds__(kLineBS) void k_prec_s(KV k, int nc, int fin) {
+  const int stop = k.flag[0];
+  double alpha = k.sc[S_ALPHA];
+  const WaveSum rhv(k.part, 0, fin);
+  LineRows L;
+  if (nc) L.load(k, threadIdx.x, nc, k.r, k.r, k.v);
+  if (stop) return;
+  if (fin && !fin1_logic(k.scal(), rhv.sum(), alpha, blockIdx.x == 0 && threadIdx.x == 0)) return;
+  auto rhs = [&](double r, double, double v) { return r - alpha * v; };
+  if (nc) line_lds_solve(k, nc, L, k.r, k.r, k.v, k.s, k.sh, rhs);
+  else line_mem_solve(k, k.r, k.r, k.v, k.s, k.sh, rhs);
 }
 
 // t = A sh; partials (t,s), (t,t)
@@ -273,14 +369,24 @@ __global__ void k_fin2(KVT<V> k, int nblk) {
   if (k.flag[0]) return;
   const double ts = final_sum(k.part, 0, 0, nblk);
   const double tt = final_sum(k.part, 1, 0, nblk);
-  if (threadIdx.x == 0) fin2_logic(k.scal(), ts, tt);
+  double omega;
+  if (threadIdx.x == 0) fin2_logic(k.scal(), ts, tt, omega);
 }
 
-// x += alpha*ph + omega*sh; r = s - omega*t; partials (rh,r), (r,r)
+// x += alpha*ph + omega*sh; r = s - omega*t; partials (rh,r), (r,r), apart
+// from those of the dots before it, which the launch may still be reading
+// (fin > 0: omega from `fin` of them)
 template <class V>
-__global__ __launch_bounds__(kBS) void k_update(KVT<V> k) {
+__global__ __launch_bounds__(kBS) void k_update(KVT<V> k, int fin) {
   if (k.flag[0]) return;
-  const V alpha = (V)k.sc[S_ALPHA], omega = (V)k.sc[S_OMEGA];
+  double w = 0.0;
+  if (!fin) {
+    w = k.sc[S_OMEGA];
+  } else {
+    const WaveSum ts(k.part, 0, fin), tt(k.part, 1, fin);
+    if (!fin2_logic(k.scal(), ts.sum(), tt.sum(), w, blockIdx.x == 0 && threadIdx.x == 0)) return;
+  }
+  const V alpha = (V)k.sc[S_ALPHA], omega = (V)w;
   double acc[2] = {0.0, 0.0};
   for (long r = (long)blockIdx.x * kBS + threadIdx.x; r < k.n; r += (long)gridDim.x * kBS) {
     k.x[r] = k.x[r] + alpha * k.ph[r] + omega * k.sh[r];
@@ -289,15 +395,16 @@ __global__ __launch_bounds__(kBS) void k_update(KVT<V> k) {
     acc[0] += (double)k.rh[r] * (double)rv;
     acc[1] += (double)rv * (double)rv;
   }
-  block_reduce<2>(acc, k.part);
+  block_reduce<2>(acc, k.part2);
 }
 
 template <class V>
 __global__ void k_fin3(KVT<V> k, int nblk) {
   if (k.flag[0]) return;
-  const double rhr = final_sum(k.part, 0, 0, nblk);
-  const double rr = final_sum(k.part, 1, 0, nblk);
-  if (threadIdx.x == 0) fin3_logic(k.scal(), rhr, rr);
+  const double rhr = final_sum(k.part2, 0, 0, nblk);
+  const double rr = final_sum(k.part2, 1, 0, nblk);
+  double beta;
+  if (threadIdx.x == 0) fin3_logic(k.scal(), rhr, rr, beta);
 }
 
 // p = r + beta*(p - omega*v)  (multigrid path: the preconditioner is a
@@ -372,7 +479,7 @@ int poisson_alloc(nhw_ctx *c) {
   };
   k.nblk = (int)std::min<long>(kRedBlocks, (k.n + kBS - 1) / kBS);
   const bool line = c->cfg.solver == NHW_SOLVER_LINE;
-  bool ok = al(&k.rhs, k.n) && al(&k.x, nv) && al(&k.part, 3 * kRedBlocks) && al(&k.sc, 16);
+  bool ok = al(&k.rhs, k.n) && al(&k.x, nv) && al(&k.part, 2 * 3 * kRedBlocks) && al(&k.sc, 16);
   if (line)  // the assembled matrix and line factors exist only for NHW_SOLVER_LINE
     ok = ok && al(&k.coef, 15 * k.n) && al(&k.lu_c, k.n) && al(&k.lu_d, k.n);
   if (c->mixed)  // FP32 inner Krylov vectors; the FP64 ones are not needed
@@ -420,7 +527,7 @@ static KV make_kv(nhw_ctx *c) {
   k.coef = kr.coef; k.b = kr.rhs;
   k.x = kr.x + kr.pad; k.r = kr.r; k.rh = kr.rh; k.p = kr.p; k.v = kr.v; k.s = kr.s; k.t = kr.t;
   k.ph = kr.ph ? kr.ph + kr.pad : nullptr; k.sh = kr.sh ? kr.sh + kr.pad : nullptr;
-  k.lu_c = kr.lu_c; k.lu_d = kr.lu_d; k.part = kr.part; k.sc = kr.sc; k.flag = kr.flag;
+  k.lu_c = kr.lu_c; k.lu_d = kr.lu_d; k.part = kr.part; k.part2 = kr.part + 3 * kRedBlocks; k.sc = kr.sc; k.flag = kr.flag;
   k.itmax = c->cfg.itmax;
   k.tol2 = c->cfg.tol * c->cfg.tol;
   k.itol2 = k.tol2;
@@ -437,7 +544,7 @@ static KVT<float> make_kvf(nhw_ctx *c) {
   k.coef = nullptr; k.b = nullptr;
   k.x = kr.fe; k.r = kr.fr; k.rh = kr.frh; k.p = kr.fp; k.v = kr.fv; k.s = kr.fs; k.t = kr.ft;
   k.ph = kr.fph; k.sh = kr.fsh;
-  k.lu_c = nullptr; k.lu_d = nullptr; k.part = kr.part; k.sc = kr.sc; k.flag = kr.flag;
+  k.lu_c = nullptr; k.lu_d = nullptr; k.part = kr.part; k.part2 = kr.part + 3 * kRedBlocks; k.sc = kr.sc; k.flag = kr.flag;
   k.itmax = c->cfg.itmax;
   k.tol2 = c->cfg.tol * c->cfg.tol;
   k.itol2 = kInnerTol * kInnerTol;
@@ -532,7 +639,7 @@ static int bicgstab_mg(nhw_ctx *c, const KVT<V> &k, const std::vector<MGLevel> &
       mg_apply<V>(c, lvs, k.s, k.sh, stop);
       mf_apply<V>(c, lvs, k.sh, k.t, k.s, 2, k.part, stop, ncb, KID_MF_T);
       { Timed _t(c, KID_KREDUCE); hipLaunchKernelGGL(k_fin2<V>, dim3(1), dim3(kBS), 0, st, k, ncb); }
-      { Timed _t(c, KID_KUPDATE, sizeof(V) * 8 * n); hipLaunchKernelGGL(k_update<V>, dim3(nblk), dim3(kBS), 0, st, k); }
+      { Timed _t(c, KID_KUPDATE, sizeof(V) * 8 * n); hipLaunchKernelGGL(k_update<V>, dim3(nblk), dim3(kBS), 0, st, k, 0); }
       { Timed _t(c, KID_KREDUCE); hipLaunchKernelGGL(k_fin3<V>, dim3(1), dim3(kBS), 0, st, k, nblk); }
     }
     const int rc = poll_flags(c, done, iters);
@@ -705,24 +812,30 @@ int poisson_solve(nhw_ctx *c) {
   { Timed _t(c, KID_ASSEMBLE); hipLaunchKernelGGL((k_assemble<true, double>), dim3(nb), dim3(kBS), 0, st, g, c->d, kr.coef, kr.rhs); }
   const KV k = make_kv(c);
   const Off15 o = stencil(g);
-  const unsigned ncol = (unsigned)((k.MN + kBS - 1) / kBS);
-  const int nblk = kr.nblk;
+  const size_t lds = line_lds(k.K);
+  const int nc = lds ? line_cols(k.K) : 0, per = nc ? nc : kLineBS;  // columns a workgroup
+  const unsigned ncol = (unsigned)((k.MN + per - 1) / per);
+  const int nblk = kr.nblk, fin = nblk <= kFuseParts ? nblk : 0;
   { Timed _t(c, KID_KMISC); hipLaunchKernelGGL(k_x_from_p, dim3(nb), dim3(kBS), 0, st, g, c->d, k.x, zlayout(c)); }
-  { Timed _t(c, KID_LINE_FACTOR); hipLaunchKernelGGL(k_line_factor, dim3(ncol), dim3(kBS), 0, st, k); }
+  { Timed _t(c, KID_LINE_FACTOR); hipLaunchKernelGGL(k_line_factor, dim3((unsigned)((k.MN + kBS - 1) / kBS)), dim3(kBS), 0, st, k); }
   { Timed _t(c, KID_RESID); hipLaunchKernelGGL(k_resid0, dim3(nblk), dim3(kBS), 0, st, k, o); }
   { Timed _t(c, KID_KREDUCE); hipLaunchKernelGGL(k_fin0<double>, dim3(1), dim3(kBS), 0, st, k, nblk); }
   { Timed _t(c, KID_KMISC); hipLaunchKernelGGL(k_zero_if, dim3(nblk), dim3(kBS), 0, st, k.x, n, (const int *)k.flag, 4); }
   int done = 0, iters = 0, chunk = 4;
   while (true) {
     for (int q = 0; q < chunk; ++q) {
-      { Timed _t(c, KID_PREC_P); hipLaunchKernelGGL(k_prec_p, dim3(ncol), dim3(kBS), 0, st, k); }
+      { Timed _t(c, KID_PREC_P); hipLaunchKernelGGL(k_prec_p, dim3(ncol), dim3(kLineBS), lds, st, k, nc, q > 0 ? fin : 0); }
       { Timed _t(c, KID_SPMV_V); hipLaunchKernelGGL(k_spmv_v, dim3(nblk), dim3(kBS), 0, st, k, o); }
-      { Timed _t(c, KID_KREDUCE); hipLaunchKernelGGL(k_fin1<double>, dim3(1), dim3(kBS), 0, st, k, nblk); }
-      { Timed _t(c, KID_PREC_S); hipLaunchKernelGGL(k_prec_s, dim3(ncol), dim3(kBS), 0, st, k); }
+      if (!fin) { Timed _t(c, KID_KREDUCE); hipLaunchKernelGGL(k_fin1<double>, dim3(1), dim3(kBS), 0, st, k, nblk); }
+      { Timed _t(c, KID_PREC_S); hipLaunchKernelGGL(k_prec_s, dim3(ncol), dim3(kLineBS), lds, st, k, nc, fin); }
       { Timed _t(c, KID_SPMV_T); hipLaunchKernelGGL(k_spmv_t, dim3(nblk), dim3(kBS), 0, st, k, o); }
-      { Timed _t(c, KID_KREDUCE); hipLaunchKernelGGL(k_fin2<double>, dim3(1), dim3(kBS), 0, st, k, nblk); }
-      { Timed _t(c, KID_KUPDATE); hipLaunchKernelGGL(k_update<double>, dim3(nblk), dim3(kBS), 0, st, k); }
-      { Timed _t(c, KID_KREDUCE); hipLaunchKernelGGL(k_fin3<double>, dim3(1), dim3(kBS), 0, st, k, nblk); }
+      if (!fin) { Timed _t(c, KID_KREDUCE); hipLaunchKernelGGL(k_fin2<double>, dim3(1), dim3(kBS), 0, st, k, nblk); }
+      { Timed _t(c, KID_KUPDATE); hipLaunchKernelGGL(k_update<double>, dim3(nblk), dim3(kBS), 0, st, k, fin); }
+      // the next iteration's k_prec_p does the last step's, but for the poll
+      if (!fin || q == chunk - 1) {
+        Timed _t(c, KID_KREDUCE);
+        hipLaunchKernelGGL(k_fin3<double>, dim3(1), dim3(kBS), 0, st, k, nblk);
+      }
     }
     const int rc = poll_flags(c, &done, &iters);
     if (rc) return rc;
@@ -905,11 +1018,12 @@ __global__ void kb_fin(BTab<R> T, const int *off_red, const double *part, int wh
   const double s0 = final_sum(part, 0, b0, b1);
   const double s1 = final_sum(part, 1, b0, b1);
   if (threadIdx.x) return;
+  double c;
   switch (which) {
     case 0: fin0_logic(k, s0, s1); break;
-    case 1: fin1_logic(k, s0); break;
-    case 2: fin2_logic(k, s0, s1); break;
-    case 3: fin3_logic(k, s0, s1); break;
+    case 1: fin1_logic(k, s0, c); break;
+    case 2: fin2_logic(k, s0, s1, c); break;
+    case 3: fin3_logic(k, s0, s1, c); break;
     default: S.sc[S_TRUE] = s0; break;
   }
 }
