@@ -269,7 +269,7 @@ struct Krylov {
   long n = 0, pad = 0;
   double *coef = nullptr;   // 15*n, diag-major (Coef(neqns,15), src/pressure.F:536-555)
   double *rhs = nullptr;
-  double *x = nullptr, *r = nullptr, *rh = nullptr, *p = nullptr, *v = nullptr;
+  double *x = nullptr, *r = nullptr, *rh = nullptr, *p = nullptr, *p2 = nullptr, *v = nullptr;
   double *s = nullptr, *t = nullptr, *ph = nullptr, *sh = nullptr;
   double *lu_c = nullptr, *lu_d = nullptr;   // line-preconditioner factors
   double *part = nullptr;   // block partial sums (nblk * 4)
@@ -277,7 +277,7 @@ struct Krylov {
   int *flag = nullptr;      // [0] converged/stop, [1] iterations, [2] breakdown
   int nblk = 0;
   // FP32 vectors of the mixed form's inner solve (e: the correction)
-  float *fe = nullptr, *fr = nullptr, *frh = nullptr, *fp = nullptr, *fv = nullptr;
+  float *fe = nullptr, *fr = nullptr, *frh = nullptr, *fp = nullptr, *fp2 = nullptr, *fv = nullptr;
   float *fs = nullptr, *ft = nullptr, *fph = nullptr, *fsh = nullptr;
 };
 
@@ -457,13 +457,15 @@ int mg_alloc(nhw_ctx *c, std::vector<MGLevel> &lvs, int esize, int maxlev);
 void mg_free(std::vector<MGLevel> &lvs);
 int mg_upload_consts(nhw_ctx *c);  // per-level sigma constants, after nhw_set_grid
 template <class V> int mg_setup(nhw_ctx *c, std::vector<MGLevel> &lvs);
-template <class V> void mg_apply(nhw_ctx *c, const std::vector<MGLevel> &lvs, const V *b, V *x, const int *stop);
+template <class V> struct MgRhs;  // the cycle's right side (nhw_mg_dev.h)
+template <class V>
+void mg_apply(nhw_ctx *c, const std::vector<MGLevel> &lvs, int kind, const MgRhs<V> &b, V *x, const int *stop);
 template <class V>
 void mf_apply(nhw_ctx *c, const std::vector<MGLevel> &lvs, const V *x, V *y, const V *d1, int ndot, double *part,
               const int *stop, int nblk, int kid);
 template <class R>
-void mf_init(nhw_ctx *c, const std::vector<MGLevel> &lvs, const double *x, const double *b, R *r, R *rh, R *p, R *v,
-             R *e, double *part, int nblk);
+void mf_init(nhw_ctx *c, const std::vector<MGLevel> &lvs, const double *x, const double *b, R *rh, double *part,
+             int nblk);
 void mf_true_resid(nhw_ctx *c, const std::vector<MGLevel> &lvs, const double *x, const double *b, double *part,
                    int nblk);
 }  // namespace nhw

@@ -190,11 +190,13 @@ static void coarse(nhw_ctx *c, const LvlC<V> &L, const G2<V> &G, const V *b, V *
 
 // algorithmic bytes of the two halves of a level's cycle: b, the five column
 // fields and the coarse right side; b, the fields, the coarse solution and x
-template <class V, int KM, int TX, int TY>
-static void down_t(nhw_ctx *c, const LvlC<V> &L, const MGLevel &lv, const MGLevel &q, const V *b, const int *stop) {
+template <class V, int KM, int TX, int TY, int KIND>
+static void down_t(nhw_ctx *c, const LvlC<V> &L, const MGLevel &lv, const MGLevel &q, const MgRhs<V> &b,
+                   const int *stop) {
   using T = MgTile<TX, TY>;
-  Timed t(c, KID_MG_DOWN, sizeof(V) * ((double)L.MN * L.K + (double)q.M * q.N * L.K + 5.0 * L.MN));
-  hipLaunchKernelGGL((k_mg_down<V, KM, TX, TY>), dim3(mg_tiles<TX, TY>(lv)), dim3(T::NT), T::lds(L.K, sizeof(V)), c->stream, L, g2<V>(lv),
+  constexpr double rows = KIND == MG_B ? 1.0 : KIND == MG_S ? 3.0 : 4.0;
+  Timed t(c, KID_MG_DOWN, sizeof(V) * (rows * L.MN * L.K + (double)q.M * q.N * L.K + 5.0 * L.MN));
+  hipLaunchKernelGGL((k_mg_down<V, KM, TX, TY, KIND>), dim3(mg_tiles<TX, TY>(lv)), dim3(T::NT), T::lds(L.K, sizeof(V)), c->stream, L, g2<V>(lv),
                      b, q.M, q.N, lv.fx, lv.fy, (V *)q.b, stop);
 }
 template <class V, int KM, int TX, int TY>
@@ -207,10 +209,11 @@ static void up_t(nhw_ctx *c, const LvlC<V> &L, const MGLevel &lv, const MGLevel 
 }
 // x = V(b): one V(1,1) cycle from a zero guess on level l; the coarsest
 // level (at most kMgCoarseCols columns) gets coarse_sweeps zebra sweeps
-template <class V>
-static void vcycle(nhw_ctx *c, const std::vector<MGLevel> &lvs, size_t l, const V *b, V *x, const int *stop) {
+template <class V, int KIND>
+static void vcycle(nhw_ctx *c, const std::vector<MGLevel> &lvs, size_t l, const MgRhs<V> &in, V *x, const int *stop) {
   const MGLevel &lv = lvs[l];
   const LvlC<V> L = make_lvl<V>(c, lv);
+  const V *b = KIND == MG_B ? in.b : in.out;
   if (l + 1 == lvs.size()) {
     coarse(c, L, g2<V>(lv), b, x, stop);
     return;
@@ -219,10 +222,10 @@ static void vcycle(nhw_ctx *c, const std::vector<MGLevel> &lvs, size_t l, const 
   const bool big = mg_big_tiles((long)lv.M * lv.N);
   by_rows<kMgKMax>(L.K, [&](auto km) {
     constexpr int KM = decltype(km)::value;
-    if (big) down_t<V, KM, kTileX, kTileY>(c, L, lv, q, b, stop);
-    else down_t<V, KM, kTileSX, kTileSY>(c, L, lv, q, b, stop);
+    if (big) down_t<V, KM, kTileX, kTileY, KIND>(c, L, lv, q, in, stop);
+    else down_t<V, KM, kTileSX, kTileSY, KIND>(c, L, lv, q, in, stop);
   });
-  vcycle<V>(c, lvs, l + 1, (const V *)q.b, (V *)q.x, stop);
+  vcycle<V, MG_B>(c, lvs, l + 1, MgRhs<V>{(const V *)q.b}, (V *)q.x, stop);
   by_rows<kMgKMax>(L.K, [&](auto km) {
     constexpr int KM = decltype(km)::value;
     if (big) up_t<V, KM, kTileX, kTileY>(c, L, lv, q, b, x, stop);
@@ -231,11 +234,15 @@ static void vcycle(nhw_ctx *c, const std::vector<MGLevel> &lvs, size_t l, const 
 }
 
 template <class V>
-void mg_apply(nhw_ctx *c, const std::vector<MGLevel> &lvs, const V *b, V *x, const int *stop) {
-  vcycle<V>(c, lvs, 0, b, x, stop);
+void mg_apply(nhw_ctx *c, const std::vector<MGLevel> &lvs, int kind, const MgRhs<V> &b, V *x, const int *stop) {
+  if (kind == MG_B) vcycle<V, MG_B>(c, lvs, 0, b, x, stop);
+  else if (kind == MG_S) vcycle<V, MG_S>(c, lvs, 0, b, x, stop);
+  else vcycle<V, MG_P>(c, lvs, 0, b, x, stop);
 }
-template void mg_apply<double>(nhw_ctx *, const std::vector<MGLevel> &, const double *, double *, const int *);
-template void mg_apply<float>(nhw_ctx *, const std::vector<MGLevel> &, const float *, float *, const int *);
+template void mg_apply<double>(nhw_ctx *, const std::vector<MGLevel> &, int, const MgRhs<double> &, double *,
+                               const int *);
+template void mg_apply<float>(nhw_ctx *, const std::vector<MGLevel> &, int, const MgRhs<float> &, float *,
+                              const int *);
 
 // y = A x on the fine level, with ndot dot partials (y,d1) [and (y,y)]
 template <class V>
@@ -262,19 +269,18 @@ template void mf_apply<float>(nhw_ctx *, const std::vector<MGLevel> &, const flo
 // FP64 residual of x against b into the Krylov vectors of type R (see
 // k_mf_init); geometry from the FP64 level 0 of `lvs`
 template <class R>
-void mf_init(nhw_ctx *c, const std::vector<MGLevel> &lvs, const double *x, const double *b, R *r, R *rh, R *p, R *v,
-             R *e, double *part, int nblk) {
+void mf_init(nhw_ctx *c, const std::vector<MGLevel> &lvs, const double *x, const double *b, R *rh, double *part,
+             int nblk) {
   const MGLevel &l0 = lvs[0];
   const LvlC<double> L = make_lvl<double>(c, l0);
   const double n = (double)L.MN * L.K;
-  Timed t(c, KID_MF_RESID, 16.0 * n + sizeof(R) * (e ? 5.0 : 4.0) * n + 40.0 * L.MN);
-  hipLaunchKernelGGL(k_mf_init<R>, dim3(nblk), dim3(kBSm), 0, c->stream, L, g2<double>(l0), x, b, r, rh, p, v, e,
-                     part);
+  Timed t(c, KID_MF_RESID, (16.0 + sizeof(R)) * n + 40.0 * L.MN);
+  hipLaunchKernelGGL(k_mf_init<R>, dim3(nblk), dim3(kBSm), 0, c->stream, L, g2<double>(l0), x, b, rh, part);
 }
 template void mf_init<double>(nhw_ctx *, const std::vector<MGLevel> &, const double *, const double *, double *,
-                              double *, double *, double *, double *, double *, int);
+                              double *, int);
 template void mf_init<float>(nhw_ctx *, const std::vector<MGLevel> &, const double *, const double *, float *,
-                             float *, float *, float *, float *, double *, int);
+                             double *, int);
 
 void mf_true_resid(nhw_ctx *c, const std::vector<MGLevel> &lvs, const double *x, const double *b, double *part,
                    int nblk) {

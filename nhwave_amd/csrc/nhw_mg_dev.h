@@ -4,6 +4,7 @@
 #pragma once
 #include <type_traits>
 
+#include "nhw_krylov_dev.h"
 #include "nhw_impl.h"
 
 namespace nhw {
@@ -370,13 +371,11 @@ __global__ __launch_bounds__(kBSm) void k_mf_apply(LvlC<V> L, G2<V> G, const V *
 }
 
 // start of a (sub)solve, in the FP64 operator: res = b - A x with x and b
-// FP64; r = rh = res in the Krylov type R, p = v = 0, and e = 0 when given
-// (the inner correction of the mixed form); partials (res,res), (b,b)
+// FP64, into rh in the Krylov type R; partials (res,res), (b,b)
 template <class R>
 __global__ __launch_bounds__(kBSm) void k_mf_init(LvlC<double> L, G2<double> G, const double *__restrict__ x,
-                                                  const double *__restrict__ b, R *__restrict__ r,
-                                                  R *__restrict__ rh, R *__restrict__ p, R *__restrict__ v,
-                                                  R *__restrict__ e, double *part) {
+                                                  const double *__restrict__ b, R *__restrict__ rh,
+                                                  double *part) {
   double acc[2] = {0.0, 0.0};
   for (long col = (long)xcd_block() * kBSm + threadIdx.x; col < L.MN; col += (long)gridDim.x * kBSm) {
     const int i = (int)(col % L.M), j = (int)(col / L.M);
@@ -391,8 +390,7 @@ __global__ __launch_bounds__(kBSm) void k_mf_init(LvlC<double> L, G2<double> G, 
       const long q = (long)k * L.MN + o.c;
       const double bv = b[q];
       const double rv = bv - arow3(c, pv, cu, nx);
-      r[q] = (R)rv; rh[q] = (R)rv; p[q] = R(0); v[q] = R(0);
-      if (e) e[q] = R(0);
+      rh[q] = (R)rv;
       acc[0] += rv * rv;
       acc[1] += bv * bv;
       pv = cu;
@@ -683,12 +681,91 @@ __device__ __forceinline__ Nb tile_nbrs(int r, int p, int colour) {
   return o;
 }
 
+// The right side of a level's cycle.  On the fine level the iteration's
+// vectors are formed where the cycle reads them: MG_S, s = r - alpha v; MG_P,
+// p = r + beta (p - omega v).  MG_B: a vector.
+enum { MG_B = 0, MG_S, MG_P };
+template <class V, int KIND>
+struct TileRhs {
+  const V *__restrict__ b, *__restrict__ p, *__restrict__ v;
+  V *out;
+  V f, w;
+  // a column's rows of the vectors, and what they make
+  template <int KM>
+  struct Raw {
+    V b[KM], v[KIND == MG_B ? 1 : KM], p[KIND == MG_P ? KM : 1];
+  };
+  template <int KM>
+  __device__ __forceinline__ void ask(unsigned zc, const LvlC<V> &L, Raw<KM> &q) const {
+    load_rows<V, KM>(b, zc, L, q.b);
+    if constexpr (KIND != MG_B) load_rows<V, KM>(v, zc, L, q.v);
+    if constexpr (KIND == MG_P) load_rows<V, KM>(p, zc, L, q.p);
+  }
+  template <int KM>
+  __device__ __forceinline__ void form(const Raw<KM> &q, V (&r)[KM]) const {
+#pragma unroll
+    for (int k = 0; k < KM; ++k) {
+      r[k] = q.b[k];
+      if constexpr (KIND == MG_S) r[k] = q.b[k] - f * q.v[k];
+      if constexpr (KIND == MG_P) r[k] = q.b[k] + f * (q.p[k] - w * q.v[k]);
+    }
+  }
+  template <int KM>
+  __device__ __forceinline__ void load(unsigned zc, const LvlC<V> &L, V (&r)[KM]) const {
+    Raw<KM> q;
+    ask(zc, L, q);
+    form(q, r);
+  }
+  // the vector formed, where the column is the tile's own
+  template <int KM>
+  __device__ __forceinline__ void keep(bool own, unsigned zc, const LvlC<V> &L, const V (&r)[KM]) const {
+    if (KIND != MG_B && own) store_rows<V, KM>(L, r, out, zc);
+  }
+};
+// host side of it: fin > 0, the scalar step before the launch is its own,
+// from `fin` partials (kFuseParts)
+template <class V>
+struct MgRhs {
+  const V *b, *p, *v;
+  V *out;
+  KScal sc;
+  const double *part;
+  int fin;
+};
+template <class V, int KIND>
+__device__ __forceinline__ TileRhs<V, KIND> tile_vecs(const MgRhs<V> &in) {
+  return TileRhs<V, KIND>{in.b, in.p, in.v, in.out, V(0), V(0)};
+}
+// the scalars; asked() asks for what else the launch waits for, between the
+// partials and their sum.  false: the iteration has stopped.
+template <class V, int KIND, class F>
+__device__ __forceinline__ bool tile_scalars(const MgRhs<V> &in, TileRhs<V, KIND> &R, F asked) {
+  const bool write = blockIdx.x == 0 && threadIdx.x == 0;
+  if constexpr (KIND == MG_S) {
+    double alpha = in.sc.sc[S_ALPHA];
+    const WaveSum rhv(in.part, 0, in.fin);
+    asked();
+    if (in.fin && !fin1_logic(in.sc, rhv.sum(), alpha, write)) return false;
+    R.f = (V)alpha;
+  } else if constexpr (KIND == MG_P) {
+    double beta = in.sc.sc[S_BETA];
+    R.w = (V)in.sc.sc[S_OMEGA];
+    const WaveSum rhr(in.part, 0, in.fin), rr(in.part, 1, in.fin);
+    asked();
+    if (in.fin && !fin3_logic(in.sc, rhr.sum(), rr.sum(), beta, write)) return false;
+    R.f = (V)beta;
+  } else {
+    asked();
+  }
+  return true;
+}
+
 // right-side rows of a tile column, zeros outside the level
-template <class V, int KM>
-__device__ __forceinline__ void tile_rows(const V *__restrict__ b, const LvlC<V> &L, const TCol &c, V (&r)[KM]) {
+template <class V, int KM, int KIND>
+__device__ __forceinline__ void tile_rows(const TileRhs<V, KIND> &b, const LvlC<V> &L, const TCol &c, V (&r)[KM]) {
 #pragma unroll
   for (int k = 0; k < KM; ++k) r[k] = V(0);
-  if (c.in) load_rows<V, KM>(b, (unsigned)zcol(c.i, c.j, L.M), L, r);
+  if (c.in) b.load((unsigned)zcol(c.i, c.j, L.M), L, r);
 }
 template <class V, int KM, int SL>
 __device__ __forceinline__ void tile_put(const LvlC<V> &L, const V (&r)[KM], V *xs, int slot) {
@@ -697,11 +774,9 @@ __device__ __forceinline__ void tile_put(const LvlC<V> &L, const V (&r)[KM], V *
     if (k < L.K) xs[k * SL + slot] = r[k];
 }
 
-// zero-guess solve of the thread's even column (tile slot threadIdx.x), in r
+// zero-guess solve of an even column of the tile from its right side in r
 template <class V, int KM>
-__device__ __forceinline__ void tile_even_zero(const LvlC<V> &L, const G2<V> &G, const V *__restrict__ b,
-                                               const TCol &c, V (&r)[KM]) {
-  tile_rows<V, KM>(b, L, c, r);
+__device__ __forceinline__ void tile_even_zero(const LvlC<V> &L, const G2<V> &G, const TCol &c, V (&r)[KM]) {
   if (c.in) zero_rows<V, KM>(L, col_consts_centre(G, L, c.i, c.j), r);
 }
 
@@ -722,14 +797,14 @@ __device__ __forceinline__ void tile_odd(const LvlC<V> &L, const LvlC<V> &Ls, co
 
 // residual b - A x of a tile column from its own values xc and its
 // neighbours' xn, added to s
-template <class V, int KM, int HW>
+template <class V, int KM, int HW, int KIND>
 __device__ __forceinline__ void tile_resid(const LvlC<V> &L, const LvlC<V> &Ls, const G2<V> &G,
-                                           const V *__restrict__ b, int i, int j, int x0, int y0, int colour,
+                                           const TileRhs<V, KIND> &b, int i, int j, int x0, int y0, int colour,
                                            const V *xc, const V *xn, V (&s)[KM]) {
   const int r = j - y0 + 2, p = (i - x0 + 2 - ((r + colour) & 1)) >> 1;
   const Nb o = tile_nbrs<HW>(r, p, colour);
   V bv[KM];
-  load_rows<V, KM>(b, (unsigned)zcol(i, j, L.M), L, bv);
+  b.load((unsigned)zcol(i, j, L.M), L, bv);
   const int K1 = L.K - 1, SL = (int)Ls.MN;
   V below = xc[o.c], at = below, above = xc[min(1, K1) * SL + o.c];
   walk_col<V, KM>(Ls, col_consts(G, L, i, j), o, xn,
@@ -741,9 +816,10 @@ __device__ __forceinline__ void tile_resid(const LvlC<V> &L, const LvlC<V> &Ls, 
   });
 }
 
-template <class V, int KM, int TX, int TY>
-__device__ __forceinline__ void mg_down_body(const LvlC<V> &L, const G2<V> &G, const V *__restrict__ b, int Mc,
-                                             int Nc, int fx, int fy, V *__restrict__ bc, long tile, V *xs) {
+// scalars(b, asked) completes b (tile_scalars); false ends the launch
+template <class V, int KM, int TX, int TY, int KIND, class F>
+__device__ __forceinline__ void mg_down_body(const LvlC<V> &L, const G2<V> &G, TileRhs<V, KIND> b, int Mc, int Nc,
+                                             int fx, int fy, V *__restrict__ bc, long tile, V *xs, F scalars) {
   using T = MgTile<TX, TY>;
   const int ntx = (L.M + TX - 1) / TX;
   const int ty = (int)(tile / ntx), x0 = (int)(tile - (long)ty * ntx) * TX, y0 = ty * TY;
@@ -759,8 +835,22 @@ __device__ __forceinline__ void mg_down_body(const LvlC<V> &L, const G2<V> &G, c
   {
     V re[KM];
     const TCol ec = tile_col(L, x0, y0, t / T::HW, t % T::HW, 0);
-    tile_even_zero<V, KM>(L, G, b, ec, re);
+    auto own = [&](const TCol &q) {
+      return q.in && q.i >= x0 && q.i < x0 + TX && q.j >= y0 && q.j < y0 + TY;
+    };
+    const unsigned ez = (unsigned)zcol(ec.i, ec.j, L.M);
+    typename TileRhs<V, KIND>::template Raw<KM> raw;
+    if (!scalars(b, [&] {
+          if (ec.in) b.ask(ez, L, raw);
+        }))
+      return;
+#pragma unroll
+    for (int k = 0; k < KM; ++k) re[k] = V(0);
+    if (ec.in) b.form(raw, re);
+    b.keep(t < T::SL && own(ec), ez, L, re);
+    tile_even_zero<V, KM>(L, G, ec, re);
     tile_rows<V, KM>(b, L, oc, ro);
+    b.keep(olive && own(oc), (unsigned)zcol(oc.i, oc.j, L.M), L, ro);
     if (t < T::SL) tile_put<V, KM, T::SL>(L, re, xe, t);
   }
   tile_odd<V, KM, TX, TY>(L, Ls, G, oc, olive, ro, xe, xo, [] {});
@@ -812,7 +902,9 @@ __device__ __forceinline__ void mg_up_body(const LvlC<V> &L, const G2<V> &G, con
   {
     V re[KM];
     const TCol ec = tile_col(L, x0, y0, t / T::HW, t % T::HW, 0);
-    tile_even_zero<V, KM>(L, G, b, ec, re);
+    const TileRhs<V, MG_B> rhs{b};
+    tile_rows<V, KM>(rhs, L, ec, re);
+    tile_even_zero<V, KM>(L, G, ec, re);
     if (ec.in) {
       const Pro<V> w = pro_at<V>(Mc, Nc, fx, fy, ec.i, ec.j);
       const long MNc = (long)Mc * Nc;
@@ -824,7 +916,7 @@ __device__ __forceinline__ void mg_up_body(const LvlC<V> &L, const G2<V> &G, con
                  w.wy1 * (w.wx0 * ldo(xk, w.c01) + w.wx1 * ldo(xk, w.c11));
       }
     }
-    tile_rows<V, KM>(b, L, oc, ro);
+    tile_rows<V, KM>(rhs, L, oc, ro);
     if (t < T::SL) tile_put<V, KM, T::SL>(L, re, xe, t);
   }
   // the tile's own columns of either colour are stored; the halo's are
@@ -850,13 +942,14 @@ __device__ __forceinline__ V *tile_lds() {
   return (V *)mg_tile_lds;
 }
 
-template <class V, int KM, int TX, int TY>
-__global__ __launch_bounds__((MgTile<TX, TY>::NT)) void k_mg_down(LvlC<V> L, G2<V> G, const V *__restrict__ b, int Mc,
-                                                                int Nc, int fx, int fy, V *__restrict__ bc,
+template <class V, int KM, int TX, int TY, int KIND>
+__global__ __launch_bounds__((MgTile<TX, TY>::NT)) void k_mg_down(LvlC<V> L, G2<V> G, MgRhs<V> in, int Mc, int Nc,
+                                                                int fx, int fy, V *__restrict__ bc,
                                                                 const int *stop) {
   if (stop[0]) return;
   V *xs = tile_lds<V>();
-  mg_down_body<V, KM, TX, TY>(L, G, b, Mc, Nc, fx, fy, bc, (long)xcd_block(), xs);
+  mg_down_body<V, KM, TX, TY>(L, G, tile_vecs<V, KIND>(in), Mc, Nc, fx, fy, bc, (long)xcd_block(), xs,
+                              [&](TileRhs<V, KIND> &b, auto asked) { return tile_scalars<V, KIND>(in, b, asked); });
 }
 
 template <class V, int KM, int TX, int TY>

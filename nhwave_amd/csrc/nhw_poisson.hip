@@ -133,7 +133,7 @@ struct KVT {
   int K;
   const double *coef;
   const double *b;
-  V *x, *r, *rh, *p, *v, *s, *t, *ph, *sh;
+  V *x, *r, *rh, *p, *p2, *v, *s, *t, *ph, *sh;
   double *lu_c, *lu_d;
   double *part, *part2, *sc;  // partials of the dots, of the update's
   int *flag;
@@ -167,9 +167,9 @@ __global__ __launch_bounds__(kBS) void k_resid0(KV k, Off15 o) {
 
 template <class V>
 __global__ void k_fin0(KVT<V> k, int nblk) {
-  const double rr = final_sum(k.part, 0, 0, nblk);
-  const double bb = final_sum(k.part, 1, 0, nblk);
-  if (threadIdx.x == 0) fin0_logic(k.scal(), rr, bb);
+  double s[2];
+  final_sums(k.part, 0, nblk, s);
+  if (threadIdx.x == 0) fin0_logic(k.scal(), s[0], s[1]);
 }
 
 // Thomas factors of the vertical tridiagonal (c13, c1, c6) per column
@@ -332,9 +332,9 @@ __global__ __launch_bounds__(kBS) void k_spmv_v(KV k, Off15 o) {
 template <class V>
 __global__ void k_fin1(KVT<V> k, int nblk) {
   if (k.flag[0]) return;
-  const double rhv = final_sum(k.part, 0, 0, nblk);
-  double alpha;
-  if (threadIdx.x == 0) fin1_logic(k.scal(), rhv, alpha);
+  double rhv[1], alpha;
+  final_sums(k.part, 0, nblk, rhv);
+  if (threadIdx.x == 0) fin1_logic(k.scal(), rhv[0], alpha);
 }
 
 // s = r - alpha*v; sh = M^-1 s
@@ -367,33 +367,40 @@ __global__ __launch_bounds__(kBS) void k_spmv_t(KV k, Off15 o) {
 template <class V>
 __global__ void k_fin2(KVT<V> k, int nblk) {
   if (k.flag[0]) return;
-  const double ts = final_sum(k.part, 0, 0, nblk);
-  const double tt = final_sum(k.part, 1, 0, nblk);
-  double omega;
-  if (threadIdx.x == 0) fin2_logic(k.scal(), ts, tt, omega);
+  double s[2], omega;
+  final_sums(k.part, 0, nblk, s);
+  if (threadIdx.x == 0) fin2_logic(k.scal(), s[0], s[1], omega);
 }
 
 // x += alpha*ph + omega*sh; r = s - omega*t; partials (rh,r), (r,r), apart
 // from those of the dots before it, which the launch may still be reading
-// (fin > 0: omega from `fin` of them)
+// (fin > 0: omega from `fin` of them); zero: x has not been written yet
 template <class V>
-__global__ __launch_bounds__(kBS) void k_update(KVT<V> k, int fin) {
+__global__ __launch_bounds__(kBS) void k_update(KVT<V> k, int fin, int zero) {
   if (k.flag[0]) return;
-  double w = 0.0;
-  if (!fin) {
-    w = k.sc[S_OMEGA];
-  } else {
+  double w = k.sc[S_OMEGA], acc[2] = {0.0, 0.0};
+  const V alpha = (V)k.sc[S_ALPHA];
+  long r = (long)blockIdx.x * kBS + threadIdx.x;
+  V x, ph, sh, s, t, rh;
+  auto ask = [&](long q) {
+    x = zero ? V(0) : k.x[q]; ph = k.ph[q]; sh = k.sh[q]; s = k.s[q]; t = k.t[q]; rh = k.rh[q];
+  };
+  if (fin) {
     const WaveSum ts(k.part, 0, fin), tt(k.part, 1, fin);
+    ask(min(r, k.n - 1));
     if (!fin2_logic(k.scal(), ts.sum(), tt.sum(), w, blockIdx.x == 0 && threadIdx.x == 0)) return;
+  } else {
+    ask(min(r, k.n - 1));
   }
-  const V alpha = (V)k.sc[S_ALPHA], omega = (V)w;
-  double acc[2] = {0.0, 0.0};
-  for (long r = (long)blockIdx.x * kBS + threadIdx.x; r < k.n; r += (long)gridDim.x * kBS) {
-    k.x[r] = k.x[r] + alpha * k.ph[r] + omega * k.sh[r];
-    const V rv = k.s[r] - omega * k.t[r];
+  const V omega = (V)w;
+  while (r < k.n) {
+    k.x[r] = x + alpha * ph + omega * sh;
+    const V rv = s - omega * t;
     k.r[r] = rv;
-    acc[0] += (double)k.rh[r] * (double)rv;
+    acc[0] += (double)rh * (double)rv;
     acc[1] += (double)rv * (double)rv;
+    r += (long)gridDim.x * kBS;
+    if (r < k.n) ask(r);
   }
   block_reduce<2>(acc, k.part2);
 }
@@ -401,28 +408,27 @@ __global__ __launch_bounds__(kBS) void k_update(KVT<V> k, int fin) {
 template <class V>
 __global__ void k_fin3(KVT<V> k, int nblk) {
   if (k.flag[0]) return;
-  const double rhr = final_sum(k.part2, 0, 0, nblk);
-  const double rr = final_sum(k.part2, 1, 0, nblk);
-  double beta;
-  if (threadIdx.x == 0) fin3_logic(k.scal(), rhr, rr, beta);
+  double s[2], beta;
+  final_sums(k.part2, 0, nblk, s);
+  if (threadIdx.x == 0) fin3_logic(k.scal(), s[0], s[1], beta);
 }
 
-// p = r + beta*(p - omega*v)  (multigrid path: the preconditioner is a
+// p = r + beta*(pin - omega*v)  (multigrid path: the preconditioner is a
 // separate V-cycle)
 template <class V>
-__global__ __launch_bounds__(kBS) void k_pvec(KVT<V> k) {
+__global__ __launch_bounds__(kBS) void k_pvec(KVT<V> k, const V *pin) {
   if (k.flag[0]) return;
   const V beta = (V)k.sc[S_BETA], omega = (V)k.sc[S_OMEGA];
   for (long r = (long)blockIdx.x * kBS + threadIdx.x; r < k.n; r += (long)gridDim.x * kBS)
-    k.p[r] = k.r[r] + beta * (k.p[r] - omega * k.v[r]);
+    k.p[r] = k.r[r] + beta * (pin[r] - omega * k.v[r]);
 }
-// s = r - alpha*v
+// s = rin - alpha*v
 template <class V>
-__global__ __launch_bounds__(kBS) void k_svec(KVT<V> k) {
+__global__ __launch_bounds__(kBS) void k_svec(KVT<V> k, const V *rin) {
   if (k.flag[0]) return;
   const V alpha = (V)k.sc[S_ALPHA];
   for (long r = (long)blockIdx.x * kBS + threadIdx.x; r < k.n; r += (long)gridDim.x * kBS)
-    k.s[r] = k.r[r] - alpha * k.v[r];
+    k.s[r] = rin[r] - alpha * k.v[r];
 }
 
 // true residual |b - A x|^2 for the solve report
@@ -435,8 +441,9 @@ __global__ __launch_bounds__(kBS) void k_true_res(KV k, Off15 o) {
   block_reduce<1>(acc, k.part);
 }
 __global__ void k_fin_true(KV k, int nblk) {
-  const double rr = final_sum(k.part, 0, 0, nblk);
-  if (threadIdx.x == 0) k.sc[S_TRUE] = rr;
+  double rr[1];
+  final_sums(k.part, 0, nblk, rr);
+  if (threadIdx.x == 0) k.sc[S_TRUE] = rr[0];
 }
 
 // initial guess x = P (interior), src/pressure.F:105-113; zero when the
@@ -483,10 +490,10 @@ int poisson_alloc(nhw_ctx *c) {
   if (line)  // the assembled matrix and line factors exist only for NHW_SOLVER_LINE
     ok = ok && al(&k.coef, 15 * k.n) && al(&k.lu_c, k.n) && al(&k.lu_d, k.n);
   if (c->mixed)  // FP32 inner Krylov vectors; the FP64 ones are not needed
-    ok = ok && alf(&k.fe, k.n) && alf(&k.fr, k.n) && alf(&k.frh, k.n) && alf(&k.fp, k.n) && alf(&k.fv, k.n) &&
+    ok = ok && alf(&k.fe, k.n) && alf(&k.fr, k.n) && alf(&k.frh, k.n) && alf(&k.fp, k.n) && alf(&k.fp2, k.n) && alf(&k.fv, k.n) &&
          alf(&k.fs, k.n) && alf(&k.ft, k.n) && alf(&k.fph, k.n) && alf(&k.fsh, k.n);
   else
-    ok = ok && al(&k.r, k.n) && al(&k.rh, k.n) && al(&k.p, k.n) && al(&k.v, k.n) && al(&k.s, k.n) &&
+    ok = ok && al(&k.r, k.n) && al(&k.rh, k.n) && al(&k.p, k.n) && (line || al(&k.p2, k.n)) && al(&k.v, k.n) && al(&k.s, k.n) &&
          al(&k.t, k.n) && al(&k.ph, nv) && al(&k.sh, nv);
   ok = ok && hipMalloc(&k.flag, sizeof(int) * 4) == hipSuccess && hipMemset(k.flag, 0, sizeof(int) * 4) == hipSuccess;
   if (!ok) {
@@ -505,10 +512,10 @@ int poisson_alloc(nhw_ctx *c) {
 
 void poisson_free(nhw_ctx *c) {
   Krylov &k = c->kr;
-  double *ps[] = {k.coef, k.rhs, k.x, k.r, k.rh, k.p, k.v, k.s, k.t, k.ph, k.sh, k.lu_c, k.lu_d, k.part, k.sc};
+  double *ps[] = {k.coef, k.rhs, k.x, k.r, k.rh, k.p, k.p2, k.v, k.s, k.t, k.ph, k.sh, k.lu_c, k.lu_d, k.part, k.sc};
   for (double *p : ps)
     if (p) (void)hipFree(p);
-  float *pf[] = {k.fe, k.fr, k.frh, k.fp, k.fv, k.fs, k.ft, k.fph, k.fsh};
+  float *pf[] = {k.fe, k.fr, k.frh, k.fp, k.fp2, k.fv, k.fs, k.ft, k.fph, k.fsh};
   for (float *p : pf)
     if (p) (void)hipFree(p);
   if (k.flag) (void)hipFree(k.flag);
@@ -525,7 +532,7 @@ static KV make_kv(nhw_ctx *c) {
   KV k;
   k.n = kr.n; k.M = g.M; k.MN = (long)g.M * g.N; k.K = g.K;
   k.coef = kr.coef; k.b = kr.rhs;
-  k.x = kr.x + kr.pad; k.r = kr.r; k.rh = kr.rh; k.p = kr.p; k.v = kr.v; k.s = kr.s; k.t = kr.t;
+  k.x = kr.x + kr.pad; k.r = kr.r; k.rh = kr.rh; k.p = kr.p; k.p2 = kr.p2; k.v = kr.v; k.s = kr.s; k.t = kr.t;
   k.ph = kr.ph ? kr.ph + kr.pad : nullptr; k.sh = kr.sh ? kr.sh + kr.pad : nullptr;
   k.lu_c = kr.lu_c; k.lu_d = kr.lu_d; k.part = kr.part; k.part2 = kr.part + 3 * kRedBlocks; k.sc = kr.sc; k.flag = kr.flag;
   k.itmax = c->cfg.itmax;
@@ -542,7 +549,7 @@ static KVT<float> make_kvf(nhw_ctx *c) {
   KVT<float> k;
   k.n = kr.n; k.M = g.M; k.MN = (long)g.M * g.N; k.K = g.K;
   k.coef = nullptr; k.b = nullptr;
-  k.x = kr.fe; k.r = kr.fr; k.rh = kr.frh; k.p = kr.fp; k.v = kr.fv; k.s = kr.fs; k.t = kr.ft;
+  k.x = kr.fe; k.r = kr.fr; k.rh = kr.frh; k.p = kr.fp; k.p2 = kr.fp2; k.v = kr.fv; k.s = kr.fs; k.t = kr.ft;
   k.ph = kr.fph; k.sh = kr.fsh;
   k.lu_c = nullptr; k.lu_d = nullptr; k.part = kr.part; k.part2 = kr.part + 3 * kRedBlocks; k.sc = kr.sc; k.flag = kr.flag;
   k.itmax = c->cfg.itmax;
@@ -622,25 +629,63 @@ static int col_blocks(const nhw_ctx *c) {
 // BiCGStab iterations with the multigrid preconditioner on hierarchy `lvs`,
 // queued in chunks sized by the previous solve's count; every kernel of an
 // iteration returns at once after the device-side flag is set.
+//
+// The solve starts with its residual in rh alone: the first p is rh, the first
+// s is formed from rh, and r and p come to be with the first update and the
+// second direction, so neither they nor v are set beforehand (1024 x 1024 x
+// 10: 151 us in k_mf_init and 61 for a first p, now NEWINIT and none).  A correction
+// (k.inner) starts from zero the same way.
+//
+// A small solve (tiles: at most kFuseParts workgroups of rows) is a chain of
+// launches that each take little more than a launch does: there the cycle's
+// first launch forms s and p as it reads them, and the scalars are formed by
+// the launches that need them, seven launches fewer an iteration (512 x 8 x 3:
+// 4.5 to 8.4 us in the three of them for 25.5 in the eight).  Larger ones lose by
+// it: the halo of the tiles makes the first launch 66 and 116 us longer at 1024
+// x 1024 x 10, where k_svec and k_pvec take 40 and 65.
 template <class V>
 static int bicgstab_mg(nhw_ctx *c, const KVT<V> &k, const std::vector<MGLevel> &lvs, int *done, int *iters) {
   hipStream_t st = c->stream;
   const int nblk = c->kr.nblk, ncb = col_blocks(c);
   const int *stop = k.flag;
   const double n = (double)k.n;
+  const bool tiles = lvs.size() > 1 && nblk <= kFuseParts;
+  // scalar steps formed in the launches that need them (kFuseParts)
+  const int fin12 = tiles ? ncb : 0, fin3 = tiles ? nblk : 0;
   int chunk = std::max(1, std::min(c->mg.last_iters, 64));
+  const V *p = nullptr;  // the direction's latest copy
   while (true) {
     for (int q = 0; q < chunk; ++q) {
-      { Timed _t(c, KID_KVEC, sizeof(V) * 4 * n); hipLaunchKernelGGL(k_pvec<V>, dim3(nblk), dim3(kBS), 0, st, k); }
-      mg_apply<V>(c, lvs, k.p, k.ph, stop);
+      const bool first = p == nullptr;
+      const V *r = first ? k.rh : k.r;
+      if (first) {
+        p = k.rh;
+        mg_apply<V>(c, lvs, MG_B, MgRhs<V>{p}, k.ph, stop);
+      } else if (tiles) {
+        V *out = p == k.p ? k.p2 : k.p;
+        mg_apply<V>(c, lvs, MG_P, MgRhs<V>{r, p, k.v, out, k.scal(), k.part2, q > 0 ? fin3 : 0}, k.ph, stop);
+        p = out;
+      } else {
+        { Timed _t(c, KID_KVEC, sizeof(V) * 4 * n); hipLaunchKernelGGL(k_pvec<V>, dim3(nblk), dim3(kBS), 0, st, k, p); }
+        p = k.p;
+        mg_apply<V>(c, lvs, MG_B, MgRhs<V>{p}, k.ph, stop);
+      }
       mf_apply<V>(c, lvs, k.ph, k.v, k.rh, 1, k.part, stop, ncb, KID_MF_V);
-      { Timed _t(c, KID_KREDUCE); hipLaunchKernelGGL(k_fin1<V>, dim3(1), dim3(kBS), 0, st, k, ncb); }
-      { Timed _t(c, KID_KVEC, sizeof(V) * 3 * n); hipLaunchKernelGGL(k_svec<V>, dim3(nblk), dim3(kBS), 0, st, k); }
-      mg_apply<V>(c, lvs, k.s, k.sh, stop);
+      if (!fin12) { Timed _t(c, KID_KREDUCE); hipLaunchKernelGGL(k_fin1<V>, dim3(1), dim3(kBS), 0, st, k, ncb); }
+      if (tiles) {
+        mg_apply<V>(c, lvs, MG_S, MgRhs<V>{r, nullptr, k.v, k.s, k.scal(), k.part, fin12}, k.sh, stop);
+      } else {
+        { Timed _t(c, KID_KVEC, sizeof(V) * 3 * n); hipLaunchKernelGGL(k_svec<V>, dim3(nblk), dim3(kBS), 0, st, k, r); }
+        mg_apply<V>(c, lvs, MG_B, MgRhs<V>{k.s}, k.sh, stop);
+      }
       mf_apply<V>(c, lvs, k.sh, k.t, k.s, 2, k.part, stop, ncb, KID_MF_T);
-      { Timed _t(c, KID_KREDUCE); hipLaunchKernelGGL(k_fin2<V>, dim3(1), dim3(kBS), 0, st, k, ncb); }
-      { Timed _t(c, KID_KUPDATE, sizeof(V) * 8 * n); hipLaunchKernelGGL(k_update<V>, dim3(nblk), dim3(kBS), 0, st, k, 0); }
-      { Timed _t(c, KID_KREDUCE); hipLaunchKernelGGL(k_fin3<V>, dim3(1), dim3(kBS), 0, st, k, nblk); }
+      if (!fin12) { Timed _t(c, KID_KREDUCE); hipLaunchKernelGGL(k_fin2<V>, dim3(1), dim3(kBS), 0, st, k, ncb); }
+      { Timed _t(c, KID_KUPDATE, sizeof(V) * 8 * n); hipLaunchKernelGGL(k_update<V>, dim3(nblk), dim3(kBS), 0, st, k, fin12, first && k.inner); }
+      // the next direction does the last step's, but for the poll
+      if (!fin3 || q == chunk - 1) {
+        Timed _t(c, KID_KREDUCE);
+        hipLaunchKernelGGL(k_fin3<V>, dim3(1), dim3(kBS), 0, st, k, nblk);
+      }
     }
     const int rc = poll_flags(c, done, iters);
     if (rc) return rc;
@@ -664,7 +709,7 @@ static int poisson_solve_mg(nhw_ctx *c) {
   const KV k = make_kv(c);
   const int nblk = kr.nblk, ncb = col_blocks(c);
   { Timed _t(c, KID_KMISC); hipLaunchKernelGGL(k_x_from_p, dim3(nb), dim3(kBS), 0, st, g, c->d, k.x, zlayout(c)); }
-  mf_init<double>(c, c->mg.lv, k.x, k.b, k.r, k.rh, k.p, k.v, (double *)nullptr, k.part, ncb);
+  mf_init<double>(c, c->mg.lv, k.x, k.b, k.rh, k.part, ncb);
   { Timed _t(c, KID_KREDUCE); hipLaunchKernelGGL(k_fin0<double>, dim3(1), dim3(kBS), 0, st, k, ncb); }
   { Timed _t(c, KID_KMISC); hipLaunchKernelGGL(k_zero_if, dim3(nblk), dim3(kBS), 0, st, k.x, n, (const int *)k.flag, 4); }
   int done = 0, iters = 0;
@@ -696,8 +741,8 @@ static int poisson_solve_mixed(nhw_ctx *c) {
   { Timed _t(c, KID_KMISC); hipLaunchKernelGGL(k_x_from_p, dim3(nb), dim3(kBS), 0, st, g, c->d, k.x, zlayout(c)); }
   int done = 0, inner_total = 0, rounds = 0;
   while (true) {
-    // outer residual into the inner vectors (e = 0); S_TRUE = |b - A x|^2
-    mf_init<float>(c, c->mg.lv, k.x, k.b, kf.r, kf.rh, kf.p, kf.v, kf.x, k.part, ncb);
+    // outer residual for the inner solve; S_TRUE = |b - A x|^2
+    mf_init<float>(c, c->mg.lv, k.x, k.b, kf.rh, k.part, ncb);
     { Timed _t(c, KID_KREDUCE); hipLaunchKernelGGL(k_fin0<float>, dim3(1), dim3(kBS), 0, st, kf, ncb); }
     int it = 0;
     rc = poll_flags(c, &done, &it);
@@ -830,7 +875,7 @@ int poisson_solve(nhw_ctx *c) {
       { Timed _t(c, KID_PREC_S); hipLaunchKernelGGL(k_prec_s, dim3(ncol), dim3(kLineBS), lds, st, k, nc, fin); }
       { Timed _t(c, KID_SPMV_T); hipLaunchKernelGGL(k_spmv_t, dim3(nblk), dim3(kBS), 0, st, k, o); }
       if (!fin) { Timed _t(c, KID_KREDUCE); hipLaunchKernelGGL(k_fin2<double>, dim3(1), dim3(kBS), 0, st, k, nblk); }
-      { Timed _t(c, KID_KUPDATE); hipLaunchKernelGGL(k_update<double>, dim3(nblk), dim3(kBS), 0, st, k, fin); }
+      { Timed _t(c, KID_KUPDATE); hipLaunchKernelGGL(k_update<double>, dim3(nblk), dim3(kBS), 0, st, k, fin, 0); }
       // the next iteration's k_prec_p does the last step's, but for the poll
       if (!fin || q == chunk - 1) {
         Timed _t(c, KID_KREDUCE);
@@ -966,8 +1011,7 @@ __global__ __launch_bounds__(256) void kb_mf_init(BTab<R> T, double *part) {
       const long q = (long)k * L.MN + o.c;
       const double bv = S.rhs[q];
       const double rv = bv - arow3(c, pv, cu, nx);
-      S.r[q] = (R)rv; S.rh[q] = (R)rv; S.pp[q] = R(0); S.v[q] = R(0);
-      if (S.inner) S.e[q] = R(0);
+      S.rh[q] = (R)rv;
       acc[0] += rv * rv;
       acc[1] += bv * bv;
       pv = cu;
@@ -1015,10 +1059,10 @@ __global__ void kb_fin(BTab<R> T, const int *off_red, const double *part, int wh
   const KScal k = bscal(S);
   if (which >= 1 && which <= 3 && S.flag[0]) return;
   const long b0 = off_red[b.u], b1 = off_red[b.u + 1];
-  const double s0 = final_sum(part, 0, b0, b1);
-  const double s1 = final_sum(part, 1, b0, b1);
+  double s[2], c;
+  final_sums(part, b0, b1, s);
   if (threadIdx.x) return;
-  double c;
+  const double s0 = s[0], s1 = s[1];
   switch (which) {
     case 0: fin0_logic(k, s0, s1); break;
     case 1: fin1_logic(k, s0, c); break;
@@ -1029,28 +1073,28 @@ __global__ void kb_fin(BTab<R> T, const int *off_red, const double *part, int wh
 }
 
 template <class R>
-__global__ __launch_bounds__(256) void kb_pvec(BTab<R> T) {
+__global__ __launch_bounds__(256) void kb_pvec(BTab<R> T, int vin) {
   const BPos b = bfind(T);
   const BScn<R> &S = T.scn[b.s];
   if (S.flag[0]) return;
   const long q = b.b * blockDim.x + threadIdx.x;
   if (q >= S.g.neq()) return;
   const R beta = (R)S.sc[S_BETA], omega = (R)S.sc[S_OMEGA];
-  S.pp[q] = S.r[q] + beta * (S.pp[q] - omega * S.v[q]);
+  S.pp[q] = S.r[q] + beta * (bvec(S, vin)[q] - omega * S.v[q]);
 }
 
 template <class R>
-__global__ __launch_bounds__(256) void kb_svec(BTab<R> T) {
+__global__ __launch_bounds__(256) void kb_svec(BTab<R> T, int vin) {
   const BPos b = bfind(T);
   const BScn<R> &S = T.scn[b.s];
   if (S.flag[0]) return;
   const long q = b.b * blockDim.x + threadIdx.x;
   if (q >= S.g.neq()) return;
-  S.s[q] = S.r[q] - (R)S.sc[S_ALPHA] * S.v[q];
+  S.s[q] = bvec(S, vin)[q] - (R)S.sc[S_ALPHA] * S.v[q];
 }
 
 template <class R>
-__global__ __launch_bounds__(256) void kb_update(BTab<R> T, double *part) {
+__global__ __launch_bounds__(256) void kb_update(BTab<R> T, double *part, int first) {
   const BPos b = bfind(T);
   const BScn<R> &S = T.scn[b.s];
   if (S.flag[0]) return;
@@ -1058,7 +1102,7 @@ __global__ __launch_bounds__(256) void kb_update(BTab<R> T, double *part) {
   double acc[2] = {0.0, 0.0};
   if (q < S.g.neq()) {
     const R alpha = (R)S.sc[S_ALPHA], omega = (R)S.sc[S_OMEGA];
-    S.kx[q] = S.kx[q] + alpha * S.ph[q] + omega * S.sh[q];
+    S.kx[q] = (first && S.inner ? R(0) : S.kx[q]) + alpha * S.ph[q] + omega * S.sh[q];
     const R rv = S.s[q] - omega * S.t[q];
     S.r[q] = rv;
     acc[0] = (double)S.rh[q] * (double)rv;
@@ -1121,8 +1165,10 @@ __global__ __launch_bounds__((MgTile<TX, TY>::NT)) void kb_mg_down(BTab<R> T, in
   if (S.flag[0]) return;
   R *xs = tile_lds<R>();
   by_rows<KM>(S.L[l].K, [&](auto km) {
-    mg_down_body<R, decltype(km)::value, TX, TY>(S.L[l], S.G[l], lvl_b(S, l, vin), S.L[l + 1].M, S.L[l + 1].N,
-                                                 S.lfx[l], S.lfy[l], S.lb[l + 1], bp.b, xs);
+    const TileRhs<R, MG_B> rhs{lvl_b(S, l, vin)};
+    mg_down_body<R, decltype(km)::value, TX, TY>(S.L[l], S.G[l], rhs, S.L[l + 1].M, S.L[l + 1].N,
+                                                 S.lfx[l], S.lfy[l], S.lb[l + 1], bp.b, xs,
+        [](TileRhs<R, MG_B> &, auto asked) { asked(); return true; });
   });
 }
 
@@ -1143,7 +1189,8 @@ __global__ __launch_bounds__(256) void kb_add_correction(BTab<R> T) {
   const BPos b = bfind(T);
   const BScn<R> &S = T.scn[b.s];
   const long q = b.b * blockDim.x + threadIdx.x;
-  if (q < S.g.neq()) S.x[q] += (double)S.e[q];
+  // a solve that broke down before its first update has no correction
+  if (S.flag[1] > 0 && q < S.g.neq()) S.x[q] += (double)S.e[q];
 }
 
 template <class R>
@@ -1259,18 +1306,22 @@ static int bbicgstab(Batch *B, const std::vector<int> &round, int *iters_out) {
   double *part = B->part;
   int chunk = std::max(1, std::min(B->last_iters, 64)), iters = 0;
   std::vector<int> act = round;
+  int total = 0;  // iterations queued
   while (true) {
-    for (int q = 0; q < chunk; ++q) {
+    for (int q = 0; q < chunk; ++q, ++total) {
       const BShape &rows = bshape(B, "k:c3/256"), &cols = bshape(B, "k:c2/256"), &one = bshape(B, "k:one");
-      PBL(KID_KVEC, 0.0, kb_pvec<R>, rows);
-      bvcycle<R, KM>(B, BV_P, BV_PH);
+      // as in bicgstab_mg, the residual is in rh alone at first
+      const bool first = total == 0;
+      const int vr = first ? BV_RH : BV_R;
+      if (!first) PBL(KID_KVEC, 0.0, kb_pvec<R>, rows, total == 1 ? BV_RH : BV_P);
+      bvcycle<R, KM>(B, first ? BV_RH : BV_P, BV_PH);
       PBL(KID_MF_V, 0.0, (kb_mf_apply<R, 1>), cols, BV_PH, BV_V, BV_RH, part);
       PBL(KID_KREDUCE, 0.0, kb_fin<R>, one, cols.off, (const double *)part, 1);
-      PBL(KID_KVEC, 0.0, kb_svec<R>, rows);
+      PBL(KID_KVEC, 0.0, kb_svec<R>, rows, vr);
       bvcycle<R, KM>(B, BV_S, BV_SH);
       PBL(KID_MF_T, 0.0, (kb_mf_apply<R, 2>), cols, BV_SH, BV_T, BV_S, part);
       PBL(KID_KREDUCE, 0.0, kb_fin<R>, one, cols.off, (const double *)part, 2);
-      PBL(KID_KUPDATE, 0.0, kb_update<R>, rows, part);
+      PBL(KID_KUPDATE, 0.0, kb_update<R>, rows, part, (int)first);
       PBL(KID_KREDUCE, 0.0, kb_fin<R>, one, rows.off, (const double *)part, 3);
     }
     const int running = bpoll(B, &iters);
