@@ -1446,6 +1446,24 @@ __global__ void k_p_from_x(Geo g, const double *__restrict__ x, Dev d, int zl) {
 NHW_KERNELS(flux_x, 0)
 NHW_KERNELS(flux_y, 0)
 NHW_KERNELS(flux_z, 0)
+// The face kernels of a small grid in one launch, a range of workgroups each:
+// where the chip is half empty they run beside one another, and the last
+// waves of one no longer wait alone (x, y and sigma faces at 257 x 33 x 5: 20 us,
+// now 10.9, of Omega 9.8, now 5.3; at 301 x 420 x 9: 103, now 89, and 39, now 28).
+template <class R>
+__global__ __launch_bounds__(256) void k_flux_xyz(Geo g, Par p, DevT<R> d, int px, int fy, int pz, unsigned bx,
+                                                  unsigned by) {
+  const long b = blockIdx.x;
+  if (b < bx) flux_x_body<R>(g, p, d, b * 256 + threadIdx.x, px);
+  else if (b < bx + by) flux_y_body<R>(g, p, d, (b - bx) * 256 + threadIdx.x, fy);
+  else flux_z_body<R>(g, p, d, (b - bx - by) * 256 + threadIdx.x, pz);
+}
+template <class R>
+__global__ __launch_bounds__(256) void k_omega_xy(Geo g, Par p, DevT<R> d, int px, int fy, unsigned bx) {
+  const long b = blockIdx.x;
+  if (b < bx) omega_x_body<R>(g, p, d, b * 256 + threadIdx.x, px);
+  else omega_y_body<R>(g, p, d, (b - bx) * 256 + threadIdx.x, fy);
+}
 NHW_KERNELS(source_terms, 0)
 NHW_KERNELS(eval_explicit, 1)
 NHW_KERNELS(eta_slopes, 0)
@@ -1654,9 +1672,21 @@ int launch_begin_step(nhw_ctx *c) {
   return rc;
 }
 
+// One launch for the faces of all directions, but when each kernel is timed.
+// On a full chip the kernels are better apart, each with the registers it
+// needs (a hydrostatic step of 400 x 400 x 8: 494 us in one launch, 518 apart;
+// of 450 x 450 x 10: 775 and 754; of 724 x 724 x 8: 1660 and 1479).
+static bool one_face_launch(const nhw_ctx *c) { return c->g.neq() <= 12 * kFillThreads && !c->kt.on; }
+
 int launch_fluxes(nhw_ctx *c) {
   const Geo &g = c->g;
   const int px = level_parts(g, flux_x_threads(g)), fy = row_faces(g), pz = level_parts(g, (long)g.M * g.N);
+  if (one_face_launch(c)) {
+    const unsigned bx = nblocks(flux_x_threads(g, px), 256), by = nblocks(flux_y_threads(g, fy), 256);
+    LAUNCH_R(KID_FLUX_X, k_flux_xyz, (bx + by + (long)nblocks((long)g.M * g.N * pz, 256)) * 256, g, c->p, dv, px, fy,
+             pz, bx, by);
+    return post("fluxes");
+  }
   LAUNCH_R(KID_FLUX_X, k_flux_x, flux_x_threads(g, px), g, c->p, dv, px);
   LAUNCH_R(KID_FLUX_Y, k_flux_y, flux_y_threads(g, fy), g, c->p, dv, fy);
   LAUNCH_R(KID_FLUX_Z, k_flux_z, (long)g.M * g.N * pz, g, c->p, dv, pz);
@@ -1704,8 +1734,13 @@ int launch_p_from_x(nhw_ctx *c, const double *x) {
 int launch_get_omega(nhw_ctx *c) {
   const Geo &g = c->g;
   const int px = level_parts(g, flux_x_threads(g)), fy = row_faces(g);
-  LAUNCH_R(KID_OMEGA_X, k_omega_x, flux_x_threads(g, px), g, c->p, dv, px);
-  LAUNCH_R(KID_OMEGA_Y, k_omega_y, flux_y_threads(g, fy), g, c->p, dv, fy);
+  if (one_face_launch(c)) {
+    const unsigned bx = nblocks(flux_x_threads(g, px), 256);
+    LAUNCH_R(KID_OMEGA_X, k_omega_xy, (bx + (long)nblocks(flux_y_threads(g, fy), 256)) * 256, g, c->p, dv, px, fy, bx);
+  } else {
+    LAUNCH_R(KID_OMEGA_X, k_omega_x, flux_x_threads(g, px), g, c->p, dv, px);
+    LAUNCH_R(KID_OMEGA_Y, k_omega_y, flux_y_threads(g, fy), g, c->p, dv, fy);
+  }
   LAUNCH_R(KID_OMEGA_COL, k_omega_col, (long)g.M * g.N, g, c->p, dv, 0);
   return post("get_Omega");
 }

@@ -633,7 +633,7 @@ static int col_blocks(const nhw_ctx *c) {
 // The solve starts with its residual in rh alone: the first p is rh, the first
 // s is formed from rh, and r and p come to be with the first update and the
 // second direction, so neither they nor v are set beforehand (1024 x 1024 x
-// 10: 151 us in k_mf_init and 61 for a first p, now NEWINIT and none).  A correction
+// 10: 151 us in k_mf_init and 61 for a first p, now 93 and none).  A correction
 // (k.inner) starts from zero the same way.
 //
 // A small solve (tiles: at most kFuseParts workgroups of rows) is a chain of
