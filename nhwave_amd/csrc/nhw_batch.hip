@@ -257,7 +257,7 @@ static int batch_build(Batch *B) {
   if (maxblk > B->part_blocks) {
     if (B->part) (void)hipFree(B->part);
     B->part = nullptr;
-    if (hip_check(hipMalloc(&B->part, sizeof(double) * 3 * maxblk), "batch partials")) return NHW_ENOMEM;
+    if (hip_check(hipMalloc(&B->part, 2 * sizeof(double) * 3 * maxblk), "batch partials")) return NHW_ENOMEM;
     B->part_blocks = maxblk;
   }
   // member table

@@ -1072,43 +1072,66 @@ __global__ void kb_fin(BTab<R> T, const int *off_red, const double *part, int wh
   }
 }
 
+// off: where given, the scalar step before the launch is its own (k_prec_p),
+// from the partials of blocks off[u] .. off[u+1]-1 of each member u: at most
+// kFuseParts of them
+struct BSums {
+  WaveSum a, b;
+  __device__ __forceinline__ BSums(const double *part, const int *off, int u)
+      : a(part + (off ? 3L * off[u] : 0), 0, off ? off[u + 1] - off[u] : 0),
+        b(part + (off ? 3L * off[u] : 0), 1, off ? off[u + 1] - off[u] : 0) {}
+};
+
 template <class R>
-__global__ __launch_bounds__(256) void kb_pvec(BTab<R> T, int vin) {
+__global__ __launch_bounds__(256) void kb_pvec(BTab<R> T, int vin, const int *off, const double *part) {
   const BPos b = bfind(T);
   const BScn<R> &S = T.scn[b.s];
   if (S.flag[0]) return;
-  const long q = b.b * blockDim.x + threadIdx.x;
+  const long q = b.b * blockDim.x + threadIdx.x, qc = min(q, S.g.neq() - 1);
+  const BSums s(part, off, b.u);
+  const R r = S.r[qc], p = bvec(S, vin)[qc], v = S.v[qc];
+  double bt = S.sc[S_BETA];
+  if (off && !fin3_logic(bscal(S), s.a.sum(), s.b.sum(), bt, b.b == 0 && threadIdx.x == 0)) return;
   if (q >= S.g.neq()) return;
-  const R beta = (R)S.sc[S_BETA], omega = (R)S.sc[S_OMEGA];
-  S.pp[q] = S.r[q] + beta * (bvec(S, vin)[q] - omega * S.v[q]);
+  const R beta = (R)bt, omega = (R)S.sc[S_OMEGA];
+  S.pp[q] = r + beta * (p - omega * v);
 }
 
 template <class R>
-__global__ __launch_bounds__(256) void kb_svec(BTab<R> T, int vin) {
+__global__ __launch_bounds__(256) void kb_svec(BTab<R> T, int vin, const int *off, const double *part) {
   const BPos b = bfind(T);
   const BScn<R> &S = T.scn[b.s];
   if (S.flag[0]) return;
-  const long q = b.b * blockDim.x + threadIdx.x;
+  const long q = b.b * blockDim.x + threadIdx.x, qc = min(q, S.g.neq() - 1);
+  const BSums s(part, off, b.u);
+  const R r = bvec(S, vin)[qc], v = S.v[qc];
+  double alpha = S.sc[S_ALPHA];
+  if (off && !fin1_logic(bscal(S), s.a.sum(), alpha, b.b == 0 && threadIdx.x == 0)) return;
   if (q >= S.g.neq()) return;
-  S.s[q] = bvec(S, vin)[q] - (R)S.sc[S_ALPHA] * S.v[q];
+  S.s[q] = r - (R)alpha * v;
 }
 
 template <class R>
-__global__ __launch_bounds__(256) void kb_update(BTab<R> T, double *part, int first) {
+__global__ __launch_bounds__(256) void kb_update(BTab<R> T, const int *off, const double *part, double *part2,
+                                                 int first) {
   const BPos b = bfind(T);
   const BScn<R> &S = T.scn[b.s];
   if (S.flag[0]) return;
-  const long q = b.b * blockDim.x + threadIdx.x;
-  double acc[2] = {0.0, 0.0};
+  const long q = b.b * blockDim.x + threadIdx.x, qc = min(q, S.g.neq() - 1);
+  const BSums sums(part, off, b.u);
+  const R x = first && S.inner ? R(0) : S.kx[qc], ph = S.ph[qc], sh = S.sh[qc], s = S.s[qc], t = S.t[qc],
+          rh = S.rh[qc];
+  double w = S.sc[S_OMEGA], acc[2] = {0.0, 0.0};
+  if (off && !fin2_logic(bscal(S), sums.a.sum(), sums.b.sum(), w, b.b == 0 && threadIdx.x == 0)) return;
   if (q < S.g.neq()) {
-    const R alpha = (R)S.sc[S_ALPHA], omega = (R)S.sc[S_OMEGA];
-    S.kx[q] = (first && S.inner ? R(0) : S.kx[q]) + alpha * S.ph[q] + omega * S.sh[q];
-    const R rv = S.s[q] - omega * S.t[q];
+    const R alpha = (R)S.sc[S_ALPHA], omega = (R)w;
+    S.kx[q] = x + alpha * ph + omega * sh;
+    const R rv = s - omega * t;
     S.r[q] = rv;
-    acc[0] = (double)S.rh[q] * (double)rv;
+    acc[0] = (double)rh * (double)rv;
     acc[1] = (double)rv * (double)rv;
   }
-  block_reduce<2>(acc, part);
+  block_reduce<2>(acc, part2);
 }
 
 // y = A x on the fine level in R, with dot partials (y, d1) [and (y, y)]
@@ -1303,26 +1326,33 @@ static std::vector<int> running_of(Batch *B, const std::vector<int> &set) {
 // every poll the launch tables shrink to the members not yet converged
 template <class R, int KM>
 static int bbicgstab(Batch *B, const std::vector<int> &round, int *iters_out) {
-  double *part = B->part;
+  // the dots' partials, the update's (which reads the former)
+  double *part = B->part, *part2 = B->part + 3 * B->part_blocks;
+  // small members: the scalars are formed by the launches that need them
+  // (24 members of 32 to 96 cells a side: kb_fin took 12 of 164 us an iteration)
+  bool small = true;
+  for (int u : round) small = small && (B->m[u]->g.neq() + kBS - 1) / kBS <= kFuseParts;
   int chunk = std::max(1, std::min(B->last_iters, 64)), iters = 0;
   std::vector<int> act = round;
   int total = 0;  // iterations queued
   while (true) {
     for (int q = 0; q < chunk; ++q, ++total) {
       const BShape &rows = bshape(B, "k:c3/256"), &cols = bshape(B, "k:c2/256"), &one = bshape(B, "k:one");
+      const int *fin = small ? cols.off : nullptr, *fin3 = small && q > 0 ? rows.off : nullptr;
       // as in bicgstab_mg, the residual is in rh alone at first
       const bool first = total == 0;
       const int vr = first ? BV_RH : BV_R;
-      if (!first) PBL(KID_KVEC, 0.0, kb_pvec<R>, rows, total == 1 ? BV_RH : BV_P);
+      if (!first) PBL(KID_KVEC, 0.0, kb_pvec<R>, rows, total == 1 ? BV_RH : BV_P, fin3, (const double *)part2);
       bvcycle<R, KM>(B, first ? BV_RH : BV_P, BV_PH);
       PBL(KID_MF_V, 0.0, (kb_mf_apply<R, 1>), cols, BV_PH, BV_V, BV_RH, part);
-      PBL(KID_KREDUCE, 0.0, kb_fin<R>, one, cols.off, (const double *)part, 1);
-      PBL(KID_KVEC, 0.0, kb_svec<R>, rows, vr);
+      if (!small) PBL(KID_KREDUCE, 0.0, kb_fin<R>, one, cols.off, (const double *)part, 1);
+      PBL(KID_KVEC, 0.0, kb_svec<R>, rows, vr, fin, (const double *)part);
       bvcycle<R, KM>(B, BV_S, BV_SH);
       PBL(KID_MF_T, 0.0, (kb_mf_apply<R, 2>), cols, BV_SH, BV_T, BV_S, part);
-      PBL(KID_KREDUCE, 0.0, kb_fin<R>, one, cols.off, (const double *)part, 2);
-      PBL(KID_KUPDATE, 0.0, kb_update<R>, rows, part, (int)first);
-      PBL(KID_KREDUCE, 0.0, kb_fin<R>, one, rows.off, (const double *)part, 3);
+      if (!small) PBL(KID_KREDUCE, 0.0, kb_fin<R>, one, cols.off, (const double *)part, 2);
+      PBL(KID_KUPDATE, 0.0, kb_update<R>, rows, fin, (const double *)part, part2, (int)first);
+      // the next direction does the last step's, but for the poll
+      if (!small || q == chunk - 1) PBL(KID_KREDUCE, 0.0, kb_fin<R>, one, rows.off, (const double *)part2, 3);
     }
     const int running = bpoll(B, &iters);
     if (running < 0) return NHW_EHIP;
