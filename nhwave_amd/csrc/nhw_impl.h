@@ -307,6 +307,19 @@ template <int TX, int TY>
 inline unsigned mg_tiles(const MGLevel &lv) {
   return (unsigned)(((lv.M + TX - 1) / TX) * ((lv.N + TY - 1) / TY));
 }
+// The cycle from a level down that one workgroup does in one launch
+// (k_mg_tail): launches of a few tiles take little more than a launch does.
+// One CU's rate of instructions bounds it: at most one column of a colour on
+// each lane of four wavefronts, and at least two levels to descend, so that the
+// launches saved are worth the walk in one place.  Levels of so few columns
+// that still descend twice have one long side and halve along it alone (three
+// columns or fewer across).  An iteration of a one-row flume, FP64, in tiles
+// and so: 130 x 3 110 us, 104; 300 x 3 133, 121; 300 x 8 185, 169; 500 x 16 319,
+// 273; with a single level to descend, 128 x 4 x 5: 97 and 104.
+constexpr int kTailLevels = 8, kTailCols = 512;
+inline bool mg_tail(long columns, size_t levels) {
+  return columns <= kTailCols && levels > 2 && levels <= (size_t)kTailLevels;
+}
 struct MG {
   std::vector<MGLevel> lv;    // FP64 hierarchy (plain form), or FP64 level 0 only (mixed form)
   std::vector<MGLevel> lvf;   // FP32 hierarchy of the mixed form's inner solve

@@ -207,6 +207,25 @@ static void up_t(nhw_ctx *c, const LvlC<V> &L, const MGLevel &lv, const MGLevel 
   hipLaunchKernelGGL((k_mg_up<V, KM, TX, TY>), dim3(mg_tiles<TX, TY>(lv)), dim3(T::NT), T::lds(L.K, sizeof(V)), c->stream, L, g2<V>(lv), b,
                      q.M, q.N, lv.fx, lv.fy, (const V *)q.x, x, stop);
 }
+// level l and all below it
+template <class V, int KIND>
+static void tail(nhw_ctx *c, const std::vector<MGLevel> &lvs, size_t l, const MgRhs<V> &in, const V *b, V *x,
+                 const int *stop) {
+  Tail<V> A{};
+  A.n = (int)(lvs.size() - l);
+  double bytes = 0.0;
+  for (int a = 0; a < A.n; ++a) {
+    const MGLevel &lv = lvs[l + a];
+    A.l[a] = TailLevel<V>{make_lvl<V>(c, lv), g2<V>(lv), a ? (V *)lv.b : (V *)b, a ? (V *)lv.x : x, lv.fx, lv.fy};
+    bytes += sizeof(V) * (3.0 * A.l[a].L.MN * A.l[a].L.K + 10.0 * A.l[a].L.MN);
+  }
+  Timed t(c, KID_MG_COARSE, bytes);
+  by_rows<kMgKMax>(A.l[0].L.K, [&](auto km) {
+    hipLaunchKernelGGL((k_mg_tail<V, decltype(km)::value, KIND>), dim3(1), dim3(kCoarseBS), 0, c->stream, A, in,
+                       c->mg.coarse_sweeps, stop);
+  });
+}
+
 // x = V(b): one V(1,1) cycle from a zero guess on level l; the coarsest
 // level (at most kMgCoarseCols columns) gets coarse_sweeps zebra sweeps
 template <class V, int KIND>
@@ -216,6 +235,10 @@ static void vcycle(nhw_ctx *c, const std::vector<MGLevel> &lvs, size_t l, const 
   const V *b = KIND == MG_B ? in.b : in.out;
   if (l + 1 == lvs.size()) {
     coarse(c, L, g2<V>(lv), b, x, stop);
+    return;
+  }
+  if (mg_tail((long)lv.M * lv.N, lvs.size() - l)) {
+    tail<V, KIND>(c, lvs, l, in, b, x, stop);
     return;
   }
   const MGLevel &q = lvs[l + 1];

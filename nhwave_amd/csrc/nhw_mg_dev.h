@@ -961,4 +961,136 @@ __global__ __launch_bounds__((MgTile<TX, TY>::NT)) void k_mg_up(LvlC<V> L, G2<V>
   mg_up_body<V, KM, TX, TY>(L, G, b, Mc, Nc, fx, fy, xc, x, (long)xcd_block(), xs);
 }
 
+// ---------------------------------------------------------------------------
+// the rest of a cycle in one workgroup
+// ---------------------------------------------------------------------------
+template <class V>
+struct TailLevel {
+  LvlC<V> L;
+  G2<V> G;
+  V *b, *x;    // of the first level: the caller's
+  int fx, fy;  // to the next level
+};
+template <class V>
+struct Tail {
+  int n;  // levels, the last of them the hierarchy's coarsest
+  TailLevel<V> l[kTailLevels];
+};
+
+// thread t's column of a colour (the t-th, as in coarse_solve)
+template <class V>
+__device__ __forceinline__ bool colour_col(const LvlC<V> &L, int t, int colour, int &i, int &j) {
+  const int P = t / L.M, rem = t - P * L.M;
+  const int h0 = (L.M + 1) >> 1, h = colour == 0 ? h0 : L.M - h0;
+  j = rem < h ? 2 * P : 2 * P + 1;
+  i = 2 * (rem < h ? rem : rem - h) + ((j + colour) & 1);
+  return t < (int)(L.MN + 1) / 2 && j < L.N && i < L.M;
+}
+
+// The V(1,1) cycle of k_mg_down and k_mg_up, every half sweep over the whole
+// level with a barrier after it: the same operations on the same values, so
+// the same result.  x in LDS; b and the coarse solutions go through memory
+// (one CU's: the barrier is enough).
+template <class V, int KM, int KIND>
+__global__ __launch_bounds__(kCoarseBS) void k_mg_tail(Tail<V> A, MgRhs<V> in, int sweeps, const int *stop) {
+  if (stop[0]) return;
+  __shared__ V xs[KM * kTailCols];
+  const int t = threadIdx.x, K = A.l[0].L.K;
+  if constexpr (KIND != MG_B) {  // the first level's right side
+    TileRhs<V, KIND> R = tile_vecs<V, KIND>(in);
+    if (!tile_scalars<V, KIND>(in, R, [] {})) return;
+    const int n = (int)A.l[0].L.MN * K;
+    for (int q = t; q < n; q += kCoarseBS) {
+      V r = R.b[q];
+      if constexpr (KIND == MG_S) r = r - R.f * R.v[q];
+      if constexpr (KIND == MG_P) r = r + R.f * (R.p[q] - R.w * R.v[q]);
+      R.out[q] = r;
+    }
+  }
+  // a neighbour past the edge is the column itself with a zero coefficient:
+  // what it reads has to be finite
+  for (int q = t; q < KM * kTailCols; q += kCoarseBS) xs[q] = V(0);
+  __syncthreads();
+  // even columns from a zero guess, corrected by the coarse solution on the
+  // way up; odd columns against them
+  auto even_odd = [&](const TailLevel<V> &l, const TailLevel<V> *q) {
+    int i, j;
+    V r[KM];
+    if (colour_col(l.L, t, 0, i, j)) {
+      const unsigned zc = (unsigned)zcol(i, j, l.L.M);
+      load_rows<V, KM>((const V *)l.b, zc, l.L, r);
+      zero_rows<V, KM>(l.L, col_consts_centre(l.G, l.L, i, j), r);
+      if (q) {
+        const Pro<V> w = pro_at<V>(q->L.M, q->L.N, l.fx, l.fy, i, j);
+#pragma unroll
+        for (int k = 0; k < KM; ++k) {
+          const V *xk = q->x + q->L.MN * min(k, K - 1);
+          r[k] += w.wy0 * (w.wx0 * ldo(xk, w.c00) + w.wx1 * ldo(xk, w.c10)) +
+                  w.wy1 * (w.wx0 * ldo(xk, w.c01) + w.wx1 * ldo(xk, w.c11));
+        }
+      }
+      store_rows<V, KM>(l.L, r, xs, zc);
+    }
+    __syncthreads();
+    if (colour_col(l.L, t, 1, i, j)) {
+      const Nb o = nbrs(l.L, i, j);
+      load_rows<V, KM>((const V *)l.b, o.c, l.L, r);
+      line_rows<V, KM>(l.L, col_consts(l.G, l.L, i, j), o, r, xs);
+      store_rows<V, KM>(l.L, r, xs, o.c);
+      if (q) store_rows<V, KM>(l.L, r, l.x, o.c);
+    }
+    __syncthreads();
+  };
+  const int last = A.n - 1;
+  for (int a = 0; a < last; ++a) {
+    const TailLevel<V> &l = A.l[a], &q = A.l[a + 1];
+    even_odd(l, nullptr);
+    // the residual onto the coarse right side, as in mg_down_body.  Levels so
+    // narrow halve along one axis: both columns of a cell on one lane.
+    const int I = t % q.L.M, J = t / q.L.M, i0 = I * l.fx, j0 = J * l.fy;
+    if (J < q.L.N) {
+      V s[KM];
+#pragma unroll
+      for (int k = 0; k < KM; ++k) s[k] = V(0);
+      for (int h = 0; h < 2; ++h) {
+        const int i = l.fx == 2 ? i0 + h : i0, j = l.fx == 2 ? j0 : j0 + h;
+        if (i >= l.L.M || j >= l.L.N) continue;
+        const Nb o = nbrs(l.L, i, j);
+        V bv[KM];
+        load_rows<V, KM>((const V *)l.b, o.c, l.L, bv);
+        const int MN = (int)l.L.MN;
+        V below = xs[o.c], at = below, above = xs[min(1, K - 1) * MN + o.c];
+        walk_col<V, KM>(l.L, col_consts(l.G, l.L, i, j), o, (const V *)xs,
+                        [&](int k, const ZRow<V> &z, const Pl<V> &, const Pl<V> &, const Pl<V> &) {
+          s[k] += bv[k] - fma(z.c0, at, fma(z.c5, above, fma(z.c12, below, z.s)));
+          below = at;
+          at = above;
+          above = xs[min(k + 2, K - 1) * MN + o.c];
+        });
+      }
+      const int cnt = (min(i0 + l.fx, l.L.M) - i0) * (min(j0 + l.fy, l.L.N) - j0);
+      const V w = V(1) / (V)cnt;
+#pragma unroll
+      for (int k = 0; k < KM; ++k) s[k] = s[k] * w;
+      store_rows<V, KM>(q.L, s, q.b, (unsigned)zcol(I, J, q.L.M));
+    }
+    __syncthreads();
+  }
+  coarse_solve<V, KM>(A.l[last].L, A.l[last].G, (const V *)A.l[last].b, A.l[last].x, sweeps, xs);
+  __syncthreads();
+  for (int a = last - 1; a >= 0; --a) {
+    const TailLevel<V> &l = A.l[a];
+    even_odd(l, &A.l[a + 1]);
+    int i, j;
+    if (colour_col(l.L, t, 0, i, j)) {
+      const Nb o = nbrs(l.L, i, j);
+      V r[KM];
+      load_rows<V, KM>((const V *)l.b, o.c, l.L, r);
+      line_rows<V, KM>(l.L, col_consts(l.G, l.L, i, j), o, r, (const V *)xs);
+      store_rows<V, KM>(l.L, r, l.x, o.c);
+    }
+    __syncthreads();
+  }
+}
+
 }  // namespace nhw

@@ -3,7 +3,8 @@ columns, 12 x 12 below) at sizes around their edges: two steps with the
 multigrid solver against the line solver, which shares none of the cycle,
 alone (small tiles) and in a batch whose other member brings the launch over
 the threshold (large tiles).  Up to 131072 rows the cycle forms the iteration's
-vectors itself; 128 x 64 x 16 is the last such size.
+vectors itself; 128 x 64 x 16 is the last such size.  From a level of at most
+512 columns that descends twice one workgroup does the rest: narrow grids only.
 
 Both solvers leave |b - A x| <= 1e-12 |b|; the pressure's error is that times
 the condition of the system, below 1e4 on these grids (dx of the order of the
@@ -31,7 +32,9 @@ def interior(f):
 
 
 @pytest.mark.parametrize("m,n,k", [(12, 12, 3), (13, 11, 2), (28, 12, 10), (29, 13, 9), (27, 25, 16), (57, 24, 12),
-                                   (100, 3, 5), (70, 1, 4), (3, 400, 7), (83, 41, 6), (128, 64, 16), (129, 64, 16)])
+                                   (100, 3, 5), (70, 1, 4), (3, 400, 7), (83, 41, 6), (128, 64, 16), (129, 64, 16),
+                                   (129, 1, 3), (511, 1, 16), (512, 1, 2), (255, 2, 6), (2, 251, 10), (170, 3, 9),
+                                   (515, 1, 12)])
 def test_tiles_against_the_line_solver(gpu, m, n, k):
     s = case(m, n, k)
     with Model(s, solver=capi.NHW_SOLVER_LINE) as a:
