@@ -50,12 +50,17 @@ __device__ __forceinline__ T z_slope(T qm, T q0, T qp, T hp, T hm) {
 }
 
 // HLL, src/nhwave.F:2741-2776
-__device__ __forceinline__ double hll(double sl, double sr, double fl, double fr, double ul, double ur) {
+// ds: sr - sl, as it is or as the shared divisor of a face's fluxes (which the
+// y faces have no registers for: 168 allow a third wavefront a SIMD)
+__device__ __forceinline__ double value(double v) { return v; }
+__device__ __forceinline__ double value(const Quot &q) { return q.b; }
+template <class D>
+__device__ __forceinline__ double hll(double sl, double sr, const D &ds, double fl, double fr, double ul, double ur) {
   if (sl >= 0.0) return fl;
   if (sr <= 0.0) return fr;
   double f = sr * fl - sl * fr + sl * sr * (ur - ul);
-  if (fabs(sr - sl) < kSmall) return f / kSmall;
-  return f / (sr - sl);
+  if (fabs(value(ds)) < kSmall) return f / kSmall;
+  return f / ds;
 }
 
 // hydrostatic pressure term 0.5*Grav*(eta*eta+2*eta*h) (src/nhwave.F:1793-1794)
@@ -201,12 +206,13 @@ __device__ __forceinline__ void flux_x_body(const Geo &g, const Par &p, const De
   const double PL = pres(etaL, h0), PR = pres(etaR, h0);
   const double pl = sqrt(kGrav * fabs(DL)), pr = sqrt(kGrav * fabs(DR));
 
-  const R dxR = (R)dx, hdxR = (R)hdx;
+  const QuotT<R> dxq((R)dx);
+  const R hdxR = (R)hdx;
   for (int k = ka; k < kb; ++k) {
     const long c0 = g.c3(ic, j, k);
     auto recon = [&](const R *F, R &qL, R &qR) {
       const R c = F[c0];
-      const R t1 = (F[c0 + 1] - c) / dxR;
+      const R t1 = (F[c0 + 1] - c) / dxq;
       const R s = slope_of<R>(t1, from_below(t1), mr);
       qR = c - hdxR * s;
       qL = from_below(c + hdxR * s);
@@ -223,10 +229,11 @@ __device__ __forceinline__ void flux_x_body(const Geo &g, const Par &p, const De
 
     double E = 0.0, F = 0.0, G = 0.0, H = 0.0, sL, sR;
     if (wave_speeds_r(ml, mr, pl, pr, uL, uR, sL, sR)) {
-      E = hll(sL, sR, duL, duR, DL, DR);
-      F = hll(sL, sR, duL * uL + PL, duR * uR + PR, duL, duR);
-      G = hll(sL, sR, DL * uL * vL, DR * uR * vR, dvL, dvR);
-      H = hll(sL, sR, DL * uL * wL, DR * uR * wR, dwL, dwR);
+      const Quot ds(sR - sL);
+      E = hll(sL, sR, ds, duL, duR, DL, DR);
+      F = hll(sL, sR, ds, duL * uL + PL, duR * uR + PR, duL, duR);
+      G = hll(sL, sR, ds, DL * uL * vL, DR * uR * vR, dvL, dvR);
+      H = hll(sL, sR, ds, DL * uL * wL, DR * uR * wR, dwL, dwR);
     }
     // flux_bc, src/nhwave.F:2354-2552 (inflow at the west, :2381-2386)
     if (i == g.Ibeg && is_wall(p.bc_x0)) { E = 0.0; F = PR; G = 0.0; H = 0.0; }
@@ -387,10 +394,11 @@ __device__ __forceinline__ void flux_y_body(const Geo &g, const Par &p, const De
     const double PL = pres(etaL, h0), PR = pres(etaR, h0);
     double E = 0.0, F = 0.0, G = 0.0, H = 0.0, sL, sR;
     if (wave_speeds(ml, mr, DL, DR, vL, vR, sL, sR)) {
-      E = hll(sL, sR, dvL, dvR, DL, DR);
-      F = hll(sL, sR, DL * uL * vL, DR * uR * vR, duL, duR);
-      G = hll(sL, sR, dvL * vL + PL, dvR * vR + PR, dvL, dvR);
-      H = hll(sL, sR, DL * vL * wL, DR * vR * wR, dwL, dwR);
+      const double ds = sR - sL;
+      E = hll(sL, sR, ds, dvL, dvR, DL, DR);
+      F = hll(sL, sR, ds, DL * uL * vL, DR * uR * vR, duL, duR);
+      G = hll(sL, sR, ds, dvL * vL + PL, dvR * vR + PR, dvL, dvR);
+      H = hll(sL, sR, ds, DL * vL * wL, DR * vR * wR, dwL, dwR);
     }
     if (j == g.Jbeg && is_wall(p.bc_y0)) { E = 0.0; F = 0.0; G = PR; H = 0.0; }
     if (j == g.Jend1 && is_wall(p.bc_yn)) { E = 0.0; F = 0.0; G = PL; H = 0.0; }
@@ -629,21 +637,27 @@ __device__ __forceinline__ double wall_phi(const Par &p, const DevT<R> &d, doubl
 // DU/D, and the surface slopes DelxEta/DelyEta.
 enum { UVW_DIVIDE = 1, UVW_BLEND = 2, UVW_PROJECT = 4, UVW_SLOPES = 8 };
 
+// divisors that the cells of a column share
+struct ProjQ {
+  Quot dx2, dy2, D;
+  __device__ __forceinline__ ProjQ(const Geo &g, double d) : dx2(2. * g.dx), dy2(2. * g.dy), D(d) {}
+};
 // projection_corrector, src/nhwave.F:487-536, of one wet cell (DelxSc/DelySc
 // of sigma_transform, :6505-6541, formed in place).  lo, hi: the pressures on
 // the sigma faces below and above it: of the column, then its west, east,
 // south and north neighbours.
 template <class R>
 __device__ __forceinline__ void project_cell(const Geo &g, const DevT<R> &d, long c, int k, const double (&lo)[5],
-                                             const double (&hi)[5], R &du, R &dv, R &dw) {
-  const double dx = g.dx, dy = g.dy, dt = d.scal[0];
+                                             const double (&hi)[5], const ProjQ &pq, R &du, R &dv, R &dw) {
+  const double dt = d.scal[0];
   const double *dsig = d.dsig - 1, *sigc = d.sigc - 1;
-  const double dxp = 0.5 * ((lo[2] - lo[1]) / (2. * dx) + (hi[2] - hi[1]) / (2. * dx));
-  const double dyp = 0.5 * ((lo[4] - lo[3]) / (2. * dy) + (hi[4] - hi[3]) / (2. * dy));
+  const double dxp = 0.5 * ((lo[2] - lo[1]) / pq.dx2 + (hi[2] - hi[1]) / pq.dx2);
+  const double dyp = 0.5 * ((lo[4] - lo[3]) / pq.dy2 + (hi[4] - hi[3]) / pq.dy2);
   const double dzp = (hi[0] - lo[0]) / dsig[k];
-  const double Dd = d.D[c];
-  const double dxsc = (1.0 - sigc[k]) / Dd * d.DelxH[c] - sigc[k] / Dd * d.DelxEta[c];
-  const double dysc = (1.0 - sigc[k]) / Dd * d.DelyH[c] - sigc[k] / Dd * d.DelyEta[c];
+  const double Dd = pq.D.b;
+  const double sD = (1.0 - sigc[k]) / pq.D, hD = sigc[k] / pq.D;
+  const double dxsc = sD * d.DelxH[c] - hD * d.DelxEta[c];
+  const double dysc = sD * d.DelyH[c] - hD * d.DelyEta[c];
   du = du - Dd * dt / kRho0 * (dxp + dzp * dxsc);
   dv = dv - Dd * dt / kRho0 * (dyp + dzp * dysc);
   dw = dw - dt / kRho0 * dzp;
@@ -684,7 +698,7 @@ __device__ __forceinline__ void blend_cell(const Par &p, int stage, int m, doubl
 // face states there, from values still in registers.  Projection, blend,
 // division and ghosts were a launch each, every one streaming the momenta
 // again, the last of them a thread per column (1024 x 1024 x 10: 182 + 137 +
-// 195 us, now 324; 333 x 217 x 7: 38 + 8, now 15).  Every load is issued before the first value is used: a
+// 195 us, now 306; 333 x 217 x 7: 38 + 8, now 14).  Every load is issued before the first value is used: a
 // wait for memory, not the rate of the loads, is what a thread spends its
 // time on.  Rows go one by one with the groups of a row next to one another,
 // so that the pressures of neighbouring rows and levels are in the L2.
@@ -725,6 +739,7 @@ __device__ __forceinline__ void uvw_a_body(const Geo &g, const Par &p, const Dev
   {
     const int m = blend || project ? d.Mask[c] : 1;
     const double fu = blend ? sqrt(kGrav * Dd) * p.froude_cap * Dd : 0.0;
+    const ProjQ pq(g, Dd);
     R u0[NL], v0[NL], w0[NL];
     double P[NL + 1][5];
     if (project) face_pressures(g, d.P, qa, P[0]);
@@ -740,11 +755,11 @@ __device__ __forceinline__ void uvw_a_body(const Geo &g, const Par &p, const Dev
     for (int n = 0; n < NL; ++n) {
       if (n >= nk) break;
       const long q = qa + n * sk;
-      if (project && m != 0) project_cell(g, d, c, ka + n, P[n], P[n + 1], du[n], dv[n], dw[n]);
+      if (project && m != 0) project_cell(g, d, c, ka + n, P[n], P[n + 1], pq, du[n], dv[n], dw[n]);
       if (blend) blend_cell(p, stage, m, fu, u0[n], v0[n], w0[n], du[n], dv[n], dw[n]);
       if (project || blend) { d.DU[q] = du[n]; d.DV[q] = dv[n]; d.DW[q] = dw[n]; }
       if (divide) {
-        u[n] = (R)(du[n] / Dd); v[n] = (R)(dv[n] / Dd); w[n] = (R)(dw[n] / Dd);
+        u[n] = (R)((double)du[n] / pq.D); v[n] = (R)((double)dv[n] / pq.D); w[n] = (R)((double)dw[n] / pq.D);
         d.U[q] = u[n]; d.V[q] = v[n]; d.W[q] = w[n];
       }
     }
@@ -1003,7 +1018,7 @@ __device__ __forceinline__ void momenta_body(const Geo &g, const Par &p, const D
     double lo[5], hi[5];
     face_pressures(g, d.P, q, lo);
     face_pressures(g, d.P, q + (long)g.Mloc * g.Nloc, hi);
-    project_cell(g, d, c, k, lo, hi, du, dv, dw);
+    project_cell(g, d, c, k, lo, hi, ProjQ(g, Dd), du, dv, dw);
   }
   blend_cell(p, arg >> 8, m, sqrt(kGrav * Dd) * p.froude_cap * Dd, d.DU0[q], d.DV0[q], d.DW0[q], du, dv, dw);
   d.DU[q] = du; d.DV[q] = dv; d.DW[q] = dw;
@@ -1036,6 +1051,7 @@ __device__ __forceinline__ void omega_x_body(const Geo &g, const Par &p, const D
   const int ic = min(i, g.Iend + 1), im = max(ic - 1, 1);
   const bool face = lane >= 2 && i <= g.Iend1;
   const double dx = g.dx, hdx = 0.5 * dx, MinDep = p.min_dep;
+  const Quot dxq(dx);
   const long c20 = g.c2(ic, j), c2m1 = g.c2(im, j);
   const int ml = d.Mask[c2m1], mr = d.Mask[c20], mrr = d.Mask[c20 + 1];
   const double em1 = d.Eta[c2m1], e0 = d.Eta[c20];
@@ -1061,7 +1077,7 @@ __device__ __forceinline__ void omega_x_body(const Geo &g, const Par &p, const D
     const long c0 = g.c3(ic, j, k);
     auto recon = [&](const R *F, double &qL, double &qR) {
       const double c = F[c0];
-      const double t1 = ((double)F[c0 + 1] - c) / dx;
+      const double t1 = ((double)F[c0 + 1] - c) / dxq;
       const double s = slope_of(t1, from_below(t1), mr);
       qR = c - hdx * s;
       qL = from_below(c + hdx * s);
@@ -1072,7 +1088,7 @@ __device__ __forceinline__ void omega_x_body(const Geo &g, const Par &p, const D
     if (leftOv) duL = 0.0;
     if (rightOv) duR = 0.0;
     double E = 0.0, sL, sR;
-    if (wave_speeds_r(ml, mr, pl, pr, uL, uR, sL, sR)) E = hll(sL, sR, duL, duR, DL, DR);
+    if (wave_speeds_r(ml, mr, pl, pr, uL, uR, sL, sR)) E = hll(sL, sR, sR - sL, duL, duR, DL, DR);
     if (i == g.Ibeg && is_wall(p.bc_x0)) E = 0.0;
     if (i == g.Ibeg && p.bc_x0 == 3) E = d.Din0[j - 1] * d.Uin0[inflow_idx(g, j, k)];  // :1564-1565
     if (i == g.Iend1 && is_wall(p.bc_xn)) E = 0.0;
@@ -1159,7 +1175,7 @@ __device__ __forceinline__ void omega_y_body(const Geo &g, const Par &p, const D
     if (leftOv) { etaL = em1; DL = d.D[c2 - sj]; dvL = 0.0; }
     if (rightOv) { etaR = e0; DR = d.D[c2]; dvR = 0.0; }
     double E = 0.0, sL, sR;
-    if (wave_speeds(ml, mr, DL, DR, vL, vR, sL, sR)) E = hll(sL, sR, dvL, dvR, DL, DR);
+    if (wave_speeds(ml, mr, DL, DR, vL, vR, sL, sR)) E = hll(sL, sR, sR - sL, dvL, dvR, DL, DR);
     if (j == g.Jbeg && is_wall(p.bc_y0)) E = 0.0;
     if (j == g.Jend1 && is_wall(p.bc_yn)) E = 0.0;
     d.Ey[g.y3(i, j, k)] = E;
@@ -1428,9 +1444,10 @@ __global__ void k_p_from_x(Geo g, const double *__restrict__ x, Dev d, int zl) {
 // the neighbouring rows and planes its stencil reads are mostly worked by the
 // same XCD and found in its L2.  Measured per kernel at 1024x1024x10: it pays
 // for the projection (momenta; 176 -> 109 us) and the Omega column sweep (65 ->
-// 55 us) and costs the sigma-face fluxes (190 -> 225 us), the y sweeps (99 ->
-// 104 and 240 -> 246 us) and the velocity pass (318 -> 330 us); the others are
-// unchanged.
+// 55 us) and costs the sigma-face fluxes (190 -> 225 us) and the y sweeps (99 ->
+// 104 and 240 -> 246 us); the others are unchanged.  The velocity pass takes
+// it for the largest grids (2048x2048x8 in float: 822 -> 735 us; 1024x1024x10: 318
+// -> 330).
 #define NHW_KERNELS(NAME, XCD)                                                                  \
   template <class R>                                                                            \
   __global__ __launch_bounds__(256) void k_##NAME(Geo g, Par p, DevT<R> d, int arg) {          \
@@ -1469,7 +1486,7 @@ NHW_KERNELS(eval_explicit, 1)
 NHW_KERNELS(eta_slopes, 0)
 template <class R, int MODE>
 __global__ __launch_bounds__(256) void k_uvw_a(Geo g, Par p, DevT<R> d, int arg) {
-  uvw_a_body<R, MODE>(g, p, d, (long)blockIdx.x * blockDim.x + threadIdx.x, arg);
+  uvw_a_body<R, MODE>(g, p, d, (long)xcd_block() * blockDim.x + threadIdx.x, arg);
 }
 template <class R, int MODE>
 __global__ __launch_bounds__(256) void kb_uvw_a(BTab<R> T, int arg) {
