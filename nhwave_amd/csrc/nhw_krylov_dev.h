@@ -45,7 +45,7 @@ __device__ __forceinline__ void block_reduce(double (&v)[NV], double *part) {
 // sums of the first NV partials of blocks b0 .. b1-1 (fixed order:
 // deterministic).  One workgroup: eight partials a thread are under way at
 // once, and the sums share the barriers (8192 blocks, two sums: 17.6 us one
-// after the other, now NEWFIN).
+// after the other, now 7.6).
 template <int NV>
 __device__ __forceinline__ void final_sums(const double *part, long b0, long b1, double (&out)[NV]) {
   constexpr int U = 8;
