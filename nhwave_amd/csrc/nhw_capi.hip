@@ -259,7 +259,8 @@ int nhw_create(const nhw_config *cfg, nhw_ctx **out) {
 }
 
 // Device bytes nhw_create allocates for a configuration (same arithmetic as
-// the allocations in nhw_create, poisson_alloc and mg_alloc), without
+// the allocations in nhw_create, forcing_setup, viscous_setup, poisson_alloc
+// and mg_alloc; a cnoidal wave's table of a few numbers is left out), without
 // allocating: the admission test of a serving loop.
 int nhw_footprint(const nhw_config *cfg, int64_t *bytes) {
   if (!cfg || !bytes) {
@@ -276,7 +277,8 @@ int nhw_footprint(const nhw_config *cfg, int64_t *bytes) {
   const double r3 = mixed ? 4.0 : 8.0;
   double b = 8.0 * (3 * Kl + 1) + 8.0 * 20 * n2 + 4.0 * 4 * n2 + 8.0 * 4 * (nx2 + ny2);
   b += r3 * (9 * n3 + 4 * nx3 + 4 * ny3 + 4 * nz3) + 8.0 * nz3 + 8.0 * (8 + 4096) + 4.0 * 8;
-  if (west_wavemaker(cfg->wavemaker) || cfg->wavemaker == NHW_WAVE_FLUX_LR) b += 8.0 * (3.0 * Nl + 3.0 * Nl * Kl);
+  if (west_wavemaker(cfg->wavemaker) || cfg->wavemaker == NHW_WAVE_FLUX_LR) b += 8.0 * (2.0 * Nl + 3.0 * Nl * Kl);
+  if (cfg->wavemaker == NHW_WAVE_LEF_LIN) b += 8.0 * Nl;  // phase lag of each row
   if (cfg->wavemaker == NHW_WAVE_FLUX_LR) b += 8.0 * (2.0 * Nl + 5.0 * Nl * Kl + n2 + 6.0 * n3);
   if (cfg->wavemaker == NHW_WAVE_INT_IRR) b += 8.0 * n2;  // SourceC (the spectrum table is extra)
   if (cfg->sponge_on) b += 8.0 * n2;
@@ -285,10 +287,11 @@ int nhw_footprint(const nhw_config *cfg, int64_t *bytes) {
   if (cfg->non_hydro) {
     const double n = (double)M * N * K;
     const double pad = (double)(((long)M * N + M + 1 + 63) / 64 * 64);
-    b += 8.0 * (n + (n + 2 * pad) + 3 * 8192 + 16) + 16;
-    if (cfg->solver == NHW_SOLVER_LINE) b += 8.0 * 17 * n;
-    if (mixed) b += 4.0 * 9 * n;
-    else b += 8.0 * (6 * n + 2 * (n + 2 * pad));
+    const bool line = cfg->solver == NHW_SOLVER_LINE;
+    b += 8.0 * (n + (n + 2 * pad) + kPartials + 16) + 16;
+    if (line) b += 8.0 * 17 * n;
+    if (mixed) b += 4.0 * 10 * n;
+    else b += 8.0 * ((line ? 6 : 7) * n + 2 * (n + 2 * pad));
     if (cfg->solver == NHW_SOLVER_MG) {
       // hierarchy levels: 5 column fields each, and x, b below level 0
       auto levels = [&](double es, int maxlev) {

@@ -291,6 +291,10 @@ inline DevT<R> view(const Dev &d) {
 }
 
 // Krylov workspace (interior vectors padded by `pad` zeros on both sides).
+// Block partials: three numbers of each of at most kRedBlocks workgroups, of
+// the dots and of the update (which reads the former) apart.
+constexpr int kRedBlocks = 8192;
+constexpr long kPartials = 2 * 3 * kRedBlocks;
 struct Krylov {
   long n = 0, pad = 0;
   double *coef = nullptr;   // 15*n, diag-major (Coef(neqns,15), src/pressure.F:536-555)
@@ -298,7 +302,7 @@ struct Krylov {
   double *x = nullptr, *r = nullptr, *rh = nullptr, *p = nullptr, *p2 = nullptr, *v = nullptr;
   double *s = nullptr, *t = nullptr, *ph = nullptr, *sh = nullptr;
   double *lu_c = nullptr, *lu_d = nullptr;   // line-preconditioner factors
-  double *part = nullptr;   // block partial sums (nblk * 4)
+  double *part = nullptr;   // block partial sums (kPartials)
   double *sc = nullptr;     // device scalars
   int *flag = nullptr;      // [0] converged/stop, [1] iterations, [2] breakdown
   int nblk = 0;

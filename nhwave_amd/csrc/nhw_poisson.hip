@@ -14,8 +14,6 @@
 
 namespace nhw {
 
-constexpr int kRedBlocks = 8192;
-
 struct Off15 {
   long o[15];
 };
@@ -486,7 +484,7 @@ int poisson_alloc(nhw_ctx *c) {
   };
   k.nblk = (int)std::min<long>(kRedBlocks, (k.n + kBS - 1) / kBS);
   const bool line = c->cfg.solver == NHW_SOLVER_LINE;
-  bool ok = al(&k.rhs, k.n) && al(&k.x, nv) && al(&k.part, 2 * 3 * kRedBlocks) && al(&k.sc, 16);
+  bool ok = al(&k.rhs, k.n) && al(&k.x, nv) && al(&k.part, kPartials) && al(&k.sc, 16);
   if (line)  // the assembled matrix and line factors exist only for NHW_SOLVER_LINE
     ok = ok && al(&k.coef, 15 * k.n) && al(&k.lu_c, k.n) && al(&k.lu_d, k.n);
   if (c->mixed)  // FP32 inner Krylov vectors; the FP64 ones are not needed
@@ -534,7 +532,7 @@ static KV make_kv(nhw_ctx *c) {
   k.coef = kr.coef; k.b = kr.rhs;
   k.x = kr.x + kr.pad; k.r = kr.r; k.rh = kr.rh; k.p = kr.p; k.p2 = kr.p2; k.v = kr.v; k.s = kr.s; k.t = kr.t;
   k.ph = kr.ph ? kr.ph + kr.pad : nullptr; k.sh = kr.sh ? kr.sh + kr.pad : nullptr;
-  k.lu_c = kr.lu_c; k.lu_d = kr.lu_d; k.part = kr.part; k.part2 = kr.part + 3 * kRedBlocks; k.sc = kr.sc; k.flag = kr.flag;
+  k.lu_c = kr.lu_c; k.lu_d = kr.lu_d; k.part = kr.part; k.part2 = kr.part + kPartials / 2; k.sc = kr.sc; k.flag = kr.flag;
   k.itmax = c->cfg.itmax;
   k.tol2 = c->cfg.tol * c->cfg.tol;
   k.itol2 = k.tol2;
@@ -551,7 +549,7 @@ static KVT<float> make_kvf(nhw_ctx *c) {
   k.coef = nullptr; k.b = nullptr;
   k.x = kr.fe; k.r = kr.fr; k.rh = kr.frh; k.p = kr.fp; k.p2 = kr.fp2; k.v = kr.fv; k.s = kr.fs; k.t = kr.ft;
   k.ph = kr.fph; k.sh = kr.fsh;
-  k.lu_c = nullptr; k.lu_d = nullptr; k.part = kr.part; k.part2 = kr.part + 3 * kRedBlocks; k.sc = kr.sc; k.flag = kr.flag;
+  k.lu_c = nullptr; k.lu_d = nullptr; k.part = kr.part; k.part2 = kr.part + kPartials / 2; k.sc = kr.sc; k.flag = kr.flag;
   k.itmax = c->cfg.itmax;
   k.tol2 = c->cfg.tol * c->cfg.tol;
   k.itol2 = kInnerTol * kInnerTol;
