@@ -290,8 +290,9 @@ int nhw_footprint(const nhw_config *cfg, int64_t *bytes) {
     const bool line = cfg->solver == NHW_SOLVER_LINE;
     b += 8.0 * (n + (n + 2 * pad) + kPartials + 16) + 16;
     if (line) b += 8.0 * 17 * n;
-    if (mixed) b += 4.0 * 10 * n;
-    else b += 8.0 * ((line ? 6 : 7) * n + 2 * (n + 2 * pad));
+    const bool p2 = !line && mg_forms_vectors(M, N, K);
+    if (mixed) b += 4.0 * (p2 ? 10 : 9) * n;
+    else b += 8.0 * ((p2 ? 7 : 6) * n + 2 * (n + 2 * pad));
     if (cfg->solver == NHW_SOLVER_MG) {
       // hierarchy levels: 5 column fields each, and x, b below level 0
       auto levels = [&](double es, int maxlev) {
@@ -300,9 +301,8 @@ int nhw_footprint(const nhw_config *cfg, int64_t *bytes) {
         for (int l = 0;; ++l) {
           t += es * 5 * (double)(m + 2) * (nn + 2) + es * 5 * kMgKMax;
           if (maxlev > 1 && l > 0) t += es * 2 * (double)m * nn * K;
+          if (l + 1 >= maxlev || !mg_coarsens(m, nn)) break;
           const int fx = m >= 4 ? 2 : 1, fy = nn >= 4 ? 2 : 1;
-          if (l + 1 >= maxlev || (fx == 1 && fy == 1) || (m * nn <= kMgCoarseCols && std::max(m, nn) <= kMgCoarseSide))
-            break;
           m = (m + fx - 1) / fx;
           nn = (nn + fy - 1) / fy;
         }

@@ -293,13 +293,16 @@ inline DevT<R> view(const Dev &d) {
 // Krylov workspace (interior vectors padded by `pad` zeros on both sides).
 // Block partials: three numbers of each of at most kRedBlocks workgroups, of
 // the dots and of the update (which reads the former) apart.
+constexpr int kBS = 256;         // threads per block of the Krylov kernels
+constexpr int kFuseParts = 512;  // partials at most that a launch sums by itself (WaveSum)
 constexpr int kRedBlocks = 8192;
 constexpr long kPartials = 2 * 3 * kRedBlocks;
 struct Krylov {
   long n = 0, pad = 0;
   double *coef = nullptr;   // 15*n, diag-major (Coef(neqns,15), src/pressure.F:536-555)
   double *rhs = nullptr;
-  double *x = nullptr, *r = nullptr, *rh = nullptr, *p = nullptr, *p2 = nullptr, *v = nullptr;
+  double *x = nullptr, *r = nullptr, *rh = nullptr, *p = nullptr, *v = nullptr;
+  double *p2 = nullptr;     // where the cycle forms p (mg_forms_vectors); as fp2
   double *s = nullptr, *t = nullptr, *ph = nullptr, *sh = nullptr;
   double *lu_c = nullptr, *lu_d = nullptr;   // line-preconditioner factors
   double *part = nullptr;   // block partial sums (kPartials)
@@ -318,6 +321,16 @@ constexpr int kMgKMax = 16;      // largest Kglob the multigrid kernels take
 constexpr long kMgCoarseCols = 1024;  // coarsest level: at most this many columns ...
 constexpr int kMgCoarseSide = 64;     // ... and at most this many along either axis (a long,
                                       // narrow grid such as a one-row flume keeps coarsening)
+// a level of M x N columns has a coarser one
+inline bool mg_coarsens(long M, long N) {
+  return (M >= 4 || N >= 4) && (M * N > kMgCoarseCols || M > kMgCoarseSide || N > kMgCoarseSide);
+}
+// the solves of an M x N x K grid whose cycle forms s and p as it reads them,
+// p from one copy into another (bicgstab_mg): several levels, and few enough
+// rows that a launch can sum their partials
+inline bool mg_forms_vectors(long M, long N, long K) {
+  return mg_coarsens(M, N) && M * N * K <= (long)kFuseParts * kBS;
+}
 struct MGLevel {
   int M = 0, N = 0, fx = 0, fy = 0;  // fx, fy: coarsening factors to the next level
   double dx = 0.0, dy = 0.0;

@@ -6,7 +6,6 @@
 
 namespace nhw {
 
-constexpr int kBS = 256;  // threads per block of the Krylov kernels
 constexpr double kInnerTol = 1e-4;  // relative residual reduction of one FP32 inner solve
 constexpr int kMaxRefine = 20;      // refinement rounds of the mixed form
 
@@ -82,7 +81,6 @@ __device__ __forceinline__ void final_sums(const double *part, long b0, long b1,
 // lanes.  A kernel that needs a scalar of the iteration forms it like this in
 // each of its wavefronts, where a launch of one workgroup had done it.  The
 // constructor only asks for the partials; other loads may follow before sum().
-constexpr int kFuseParts = 512;
 struct WaveSum {
   double v[2][4];
   __device__ __forceinline__ WaveSum(const double *part, int m, int nblk) {

@@ -125,10 +125,8 @@ int mg_alloc(nhw_ctx *c, std::vector<MGLevel> &lvs, int esize, int maxlev) {
       set_error("mg_alloc: hipMalloc failed");
       return NHW_ENOMEM;
     }
+    if ((int)lvs.size() >= maxlev || !mg_coarsens(M, N)) break;
     const int fx = M >= 4 ? 2 : 1, fy = N >= 4 ? 2 : 1;
-    if ((int)lvs.size() >= maxlev || (fx == 1 && fy == 1) ||
-        ((long)M * N <= kMgCoarseCols && std::max(M, N) <= kMgCoarseSide))
-      break;
     lvs.back().fx = fx;
     lvs.back().fy = fy;
     M = (M + fx - 1) / fx;

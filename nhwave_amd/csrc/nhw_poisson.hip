@@ -487,12 +487,13 @@ int poisson_alloc(nhw_ctx *c) {
   bool ok = al(&k.rhs, k.n) && al(&k.x, nv) && al(&k.part, kPartials) && al(&k.sc, 16);
   if (line)  // the assembled matrix and line factors exist only for NHW_SOLVER_LINE
     ok = ok && al(&k.coef, 15 * k.n) && al(&k.lu_c, k.n) && al(&k.lu_d, k.n);
+  const bool p2 = !line && mg_forms_vectors(g.M, g.N, g.K);
   if (c->mixed)  // FP32 inner Krylov vectors; the FP64 ones are not needed
-    ok = ok && alf(&k.fe, k.n) && alf(&k.fr, k.n) && alf(&k.frh, k.n) && alf(&k.fp, k.n) && alf(&k.fp2, k.n) && alf(&k.fv, k.n) &&
-         alf(&k.fs, k.n) && alf(&k.ft, k.n) && alf(&k.fph, k.n) && alf(&k.fsh, k.n);
+    ok = ok && alf(&k.fe, k.n) && alf(&k.fr, k.n) && alf(&k.frh, k.n) && alf(&k.fp, k.n) && alf(&k.fv, k.n) &&
+         alf(&k.fs, k.n) && alf(&k.ft, k.n) && alf(&k.fph, k.n) && alf(&k.fsh, k.n) && (!p2 || alf(&k.fp2, k.n));
   else
-    ok = ok && al(&k.r, k.n) && al(&k.rh, k.n) && al(&k.p, k.n) && (line || al(&k.p2, k.n)) && al(&k.v, k.n) && al(&k.s, k.n) &&
-         al(&k.t, k.n) && al(&k.ph, nv) && al(&k.sh, nv);
+    ok = ok && al(&k.r, k.n) && al(&k.rh, k.n) && al(&k.p, k.n) && al(&k.v, k.n) && al(&k.s, k.n) &&
+         al(&k.t, k.n) && al(&k.ph, nv) && al(&k.sh, nv) && (!p2 || al(&k.p2, k.n));
   ok = ok && hipMalloc(&k.flag, sizeof(int) * 4) == hipSuccess && hipMemset(k.flag, 0, sizeof(int) * 4) == hipSuccess;
   if (!ok) {
     set_error("poisson_alloc: hipMalloc failed");
@@ -634,20 +635,20 @@ static int col_blocks(const nhw_ctx *c) {
 // 10: 151 us in k_mf_init and 61 for a first p, now 93 and none).  A correction
 // (k.inner) starts from zero the same way.
 //
-// A small solve (tiles: at most kFuseParts workgroups of rows) is a chain of
-// launches that each take little more than a launch does: there the cycle's
-// first launch forms s and p as it reads them, and the scalars are formed by
-// the launches that need them, seven launches fewer an iteration (512 x 8 x 3:
-// 4.5 to 8.4 us in the three of them for 25.5 in the eight).  Larger ones lose by
-// it: the halo of the tiles makes the first launch 66 and 116 us longer at 1024
-// x 1024 x 10, where k_svec and k_pvec take 40 and 65.
+// A small solve (tiles: mg_forms_vectors) is a chain of launches that each
+// take little more than a launch does: there the cycle's first launch forms s
+// and p as it reads them, and the scalars are formed by the launches that need
+// them, seven launches fewer an iteration (512 x 8 x 3: 4.5 to 8.4 us in the
+// three of them for 25.5 in the eight).  Larger ones lose by it: the halo of the
+// tiles makes the first launch 66 and 116 us longer at 1024 x 1024 x 10, where
+// k_svec and k_pvec take 40 and 65.
 template <class V>
 static int bicgstab_mg(nhw_ctx *c, const KVT<V> &k, const std::vector<MGLevel> &lvs, int *done, int *iters) {
   hipStream_t st = c->stream;
   const int nblk = c->kr.nblk, ncb = col_blocks(c);
   const int *stop = k.flag;
   const double n = (double)k.n;
-  const bool tiles = lvs.size() > 1 && nblk <= kFuseParts;
+  const bool tiles = mg_forms_vectors(c->g.M, c->g.N, c->g.K);
   // scalar steps formed in the launches that need them (kFuseParts)
   const int fin12 = tiles ? ncb : 0, fin3 = tiles ? nblk : 0;
   int chunk = std::max(1, std::min(c->mg.last_iters, 64));

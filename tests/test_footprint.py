@@ -73,3 +73,16 @@ def test_footprint_is_what_is_allocated(created):
         configs.append(dict(size=z, fields=dict(non_hydro=False), precision=1))
     wrong = [(c, want, got) for c, (want, got, _) in zip(configs, created(configs)) if want != got]
     assert wrong == []
+
+
+def test_second_direction_only_where_it_is_used(created):
+    """The multigrid solver keeps two copies of its direction where the cycle
+    forms it as it reads it: solves of several levels and at most 131072 rows.
+    Vectors of one number a row: rhs, r, rh, p, v, s, t (mixed: e, r, rh, p, v,
+    s, t, ph, sh) and the second p."""
+    two = {(12, 12, 3): 0, (32, 32, 16): 0, (70, 1, 4): 1, (83, 41, 6): 1, (128, 64, 16): 1, (129, 64, 16): 0,
+           (256, 128, 4): 1, (2, 20000, 8): 0, (1024, 1024, 10): 0}
+    assert sorted(two) == sorted(SIZES)
+    configs = [dict(size=z, precision=p) for z in SIZES for p in (0, 1)]
+    for c, (_, _, vectors) in zip(configs, created(configs)):
+        assert vectors == (9 if c["precision"] else 7) + two[tuple(c["size"])], c
