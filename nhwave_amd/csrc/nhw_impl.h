@@ -176,9 +176,12 @@ struct Par {
 // double as x / b, in six instructions where a division takes about twelve
 // and a reciprocal estimate.  r = 1 / b is correctly rounded, x r is within 1.5
 // units of the quotient, the first residual step brings that within one, and
-// the second then rounds correctly (Markstein, IBM J. Res. Dev. 34, 1990);
-// div_fixup does zeros, infinities and NaN.  x below 2^-900, where the residuals
-// underflow, may come out a unit off.  Floats are divided as they are.
+// the second then rounds correctly (Markstein, IBM J. Res. Dev. 34, 1990).
+// div_fixup does zeros, infinities and NaN, and turns the NaN that the residual
+// steps make of a quotient that overflows into infinity, as a division gives.
+// Not the same double: x below 2^-900, where the residuals underflow, may come
+// out a unit off (a difference of 3e-287 / b at most), and a subnormal divisor
+// has no finite r.  Floats are divided as they are.
 template <class R>
 struct QuotT {
   R b;
