@@ -671,7 +671,9 @@ __device__ __forceinline__ void face_pressures(const Geo &g, const double *P, lo
 
 // SSP-RK blend + dry zeroing + Froude cap, src/nhwave.F:1227-1261, of one cell
 // with the step's momenta DU0, DV0, DW0; fu: the capped momentum.  The square
-// root waits for a sum of squares that can reach fu (rounding included).
+// root waits for a sum of squares that can reach fu (rounding included), where
+// fu has a square to compare with: not so a negative one, which every momentum
+// reaches, and those whose square over- or underflows.
 template <class R>
 __device__ __forceinline__ void blend_cell(const Par &p, int stage, int m, double fu, R DU0, R DV0, R DW0, R &DU,
                                            R &DV, R &DW) {
@@ -682,7 +684,8 @@ __device__ __forceinline__ void blend_cell(const Par &p, int stage, int m, doubl
   if (m == 0) { du = 0.0; dv = 0.0; dw = 0.0; }
   if (p.froude_on && m > 0) {
     const double s = du * du + dv * dv + dw * dw;
-    if (s > fu * fu * (1.0 - 1e-14) && sqrt(s) > fu) {
+    const double reach = fu > 1e-150 && fu < 1e150 ? fu * fu * (1.0 - 1e-14) : -1.0;
+    if (s > reach && sqrt(s) > fu) {
       const double ang = atan2(dv, du);
       du = fu * cos(ang);
       dv = fu * sin(ang);
