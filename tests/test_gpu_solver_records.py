@@ -1,0 +1,60 @@
+"""What the preconditioners do, by what the solves leave at a loose tolerance:
+the iterations of one step's two solves and the last one's true relative
+residual, which every value of a preconditioner enters, where a converged
+field shows only the system.
+
+tests/golden/solver_records.json was recorded with other kernels: the
+multigrid cycle one half sweep, restriction or prolongation a launch, the line
+preconditioner a column a thread in memory, the iteration's scalars in launches
+of one workgroup.  The kernels of today do the same operations on the same
+values: the same iterations, and the residual to rounding (1e-6 in FP64;
+0.05 in the mixed form, whose residual of 1e-4 to 1e-3 is that of an FP32
+solve).
+
+Multigrid: TOL 1e-6 (mixed 1e-3), alone and as the first of a batch whose
+second member keeps its launches below the 32768 columns of the large column
+tiles or takes them above.  The sizes are one level only; 12 x 12 tiles with the
+iteration's vectors formed in them, up to 131072 rows, and given; the same in 28 x 12
+tiles, where four rows or fewer leave 32768 columns room; levels halved along
+one axis; and narrow grids, whose cycle one workgroup ends.  Line: TOL 1e-6,
+columns 16 and fewer a workgroup in LDS (128 and 129 levels are either side of
+16 and 8), in memory (2049), and more rows than scalars are formed in line for."""
+import json
+
+import pytest
+
+from nhw_testutil import GOLD
+from nhwave_amd import capi
+from nhwave_amd import scenario as S
+from nhwave_amd.batch import Batch
+from nhwave_amd.model import Model
+
+pytestmark = pytest.mark.gpu
+RECORDS = json.loads((GOLD / "solver_records.json").read_text())
+SECOND = {"batch-small": dict(n=50, m=40, beach_width=100.0), "batch-big": dict(n=192, m=180, beach_width=400.0)}
+
+
+def steps(form, prec, m, n, k):
+    """The stats of the scenario `form prec m n k` after one step."""
+    mixed = prec == "mixed"
+    s = S.random_scenario(9 if form == "line" else 7, mglob=m, nglob=n, kglob=k, steps=1, dry=False,
+                          tol=1e-3 if mixed else 1e-6)
+    p = capi.NHW_MIXED if mixed else capi.NHW_FP64
+    if form in SECOND:
+        with Batch([s, S.bumps_beach(kglob=3, dx=10.0, nbumps=4, tol=s.tol, **SECOND[form])], precision=p,
+                   autotune=False) as b:
+            b.step(1)
+            return b.members[0].stats()
+    with Model(s, precision=p, solver=capi.NHW_SOLVER_LINE if form == "line" else capi.NHW_SOLVER_MG) as a:
+        a.step(1)
+        return a.stats()
+
+
+@pytest.mark.parametrize("name", sorted(RECORDS))
+def test_solver_record(gpu, name):
+    form, prec, *size = name.split()
+    st = steps(form, prec, *map(int, size))
+    iters, relres = RECORDS[name]
+    assert st.not_converged == 0
+    assert st.total_iters == iters
+    assert st.last_relres == pytest.approx(relres, rel=0.05 if prec == "mixed" else 1e-6)
