@@ -243,8 +243,11 @@ static void vcycle(nhw_ctx *c, const std::vector<MGLevel> &lvs, size_t l, const 
   const bool big = mg_big_tiles((long)lv.M * lv.N);
   by_rows<kMgKMax>(L.K, [&](auto km) {
     constexpr int KM = decltype(km)::value;
-    if (big) down_t<V, KM, kTileX, kTileY, KIND>(c, L, lv, q, in, stop);
-    else down_t<V, KM, kTileSX, kTileSY, KIND>(c, L, lv, q, in, stop);
+    // where the cycle forms the vectors, only columns of few rows make up a
+    // large level (mg_forms_vectors)
+    if constexpr (KIND == MG_B || KM * kMgBigCols <= (long)kFuseParts * kBS)
+      if (big) return down_t<V, KM, kTileX, kTileY, KIND>(c, L, lv, q, in, stop);
+    down_t<V, KM, kTileSX, kTileSY, KIND>(c, L, lv, q, in, stop);
   });
   vcycle<V, MG_B>(c, lvs, l + 1, MgRhs<V>{(const V *)q.b}, (V *)q.x, stop);
   by_rows<kMgKMax>(L.K, [&](auto km) {
