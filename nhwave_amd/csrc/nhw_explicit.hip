@@ -1523,11 +1523,13 @@ NHW_KERNELS(begin, 0)
 // ----------------------------------------------------------------------------
 // launchers
 // ----------------------------------------------------------------------------
-#define LAUNCH(kid, kern, n, ...)                                                         \
+#define LAUNCH(kid, kern, n, ...) LAUNCH_B(kid, -1.0, kern, n, __VA_ARGS__)
+// ... that moves `bytes`
+#define LAUNCH_B(kid, bytes, kern, n, ...)                                                \
   do {                                                                                    \
     long _n = (n);                                                                        \
     if (_n > 0) {                                                                         \
-      Timed _t(c, kid);                                                                   \
+      Timed _t(c, kid, bytes);                                                            \
       hipLaunchKernelGGL(kern, dim3(nblocks(_n, 256)), dim3(256), 0, c->stream, __VA_ARGS__); \
     }                                                                                     \
   } while (0)
@@ -1547,14 +1549,24 @@ NHW_KERNELS(begin, 0)
 
 static int post(const char *what) { return hip_check(hipGetLastError(), what); }
 
+// bytes of a velocity pass: U, V, W and, unless it leaves them as they are,
+// DU, DV, DW; the step's momenta read and the momenta written; P; 2-D fields
+static double uvw_bytes(const nhw_ctx *c, int flags) {
+  const double n2 = (double)c->g.M * c->g.N, n = n2 * c->g.K, w3 = c->mixed ? 4.0 : 8.0;
+  const bool blend = flags & UVW_BLEND;
+  return w3 * ((flags & UVW_DIVIDE ? 6 : 3) + (blend ? 6 : 0)) * n + (flags & UVW_PROJECT ? 8.0 * n : 0.0) +
+         8.0 * 12 * n2 + (blend ? 4.0 * n2 : 0.0);
+}
+
 static void launch_uvw_a(nhw_ctx *c, int flags) {
   const Geo &g = c->g;
   const long n = (long)g.M * g.N * level_groups(g);
+  const double bytes = uvw_bytes(c, flags);
   uvw_mode(flags, uvw_plain(g, c->p), [&](auto mode) {
     if (c->mixed)
-      LAUNCH(KID_UVW_A, (k_uvw_a<float, decltype(mode)::value>), n, g, c->p, view<float>(c->d), flags);
+      LAUNCH_B(KID_UVW_A, bytes, (k_uvw_a<float, decltype(mode)::value>), n, g, c->p, view<float>(c->d), flags);
     else
-      LAUNCH(KID_UVW_A, (k_uvw_a<double, decltype(mode)::value>), n, g, c->p, c->d, flags);
+      LAUNCH_B(KID_UVW_A, bytes, (k_uvw_a<double, decltype(mode)::value>), n, g, c->p, c->d, flags);
   });
 }
 
@@ -1566,7 +1578,7 @@ int launch_initial(nhw_ctx *c) {
   launch_uvw_a(c, 0);
   if (int rc = launch_east_ghosts(c)) return rc;
   LAUNCH_R(KID_UVW_B, k_uvw_b, (long)g.M * g.N, g, c->p, dv, 0);
-  LAUNCH_R(KID_RK_BLEND, k_init_du, g.n3(), g, dv);
+  LAUNCH_R(KID_KMISC, k_init_du, g.n3(), g, dv);
   return post("initial");
 }
 
@@ -1686,24 +1698,24 @@ int launch_begin_step(nhw_ctx *c) {
   int rc = launch_flux_lr_history(c);
   if (rc) return rc;
   LAUNCH_R(KID_MASK, k_mask_a, g.n2(), g, c->p, dv, 0);
-  LAUNCH_R(KID_KMISC, k_begin, g.n3(), g, c->p, dv, 0);
+  LAUNCH_R(KID_BEGIN, k_begin, g.n3(), g, c->p, dv, 0);
   rc = post("begin step");
   std::swap(c->d.Mask, c->d.MaskNew);
   return rc;
 }
 
-// One launch for the faces of all directions, but when each kernel is timed.
-// On a full chip the kernels are better apart, each with the registers it
-// needs (a hydrostatic step of 400 x 400 x 8: 494 us in one launch, 518 apart;
-// of 450 x 450 x 10: 775 and 754; of 724 x 724 x 8: 1660 and 1479).
-static bool one_face_launch(const nhw_ctx *c) { return c->g.neq() <= 12 * kFillThreads && !c->kt.on; }
+// One launch for the faces of all directions.  On a full chip the kernels are
+// better apart, each with the registers it needs (a hydrostatic step of 400 x
+// 400 x 8: 494 us in one launch, 518 apart; of 450 x 450 x 10: 775 and 754; of
+// 724 x 724 x 8: 1660 and 1479).
+static bool one_face_launch(const nhw_ctx *c) { return c->g.neq() <= 12 * kFillThreads; }
 
 int launch_fluxes(nhw_ctx *c) {
   const Geo &g = c->g;
   const int px = level_parts(g, flux_x_threads(g)), fy = row_faces(g), pz = level_parts(g, (long)g.M * g.N);
   if (one_face_launch(c)) {
     const unsigned bx = nblocks(flux_x_threads(g, px), 256), by = nblocks(flux_y_threads(g, fy), 256);
-    LAUNCH_R(KID_FLUX_X, k_flux_xyz, (bx + by + (long)nblocks((long)g.M * g.N * pz, 256)) * 256, g, c->p, dv, px, fy,
+    LAUNCH_R(KID_FLUX_XYZ, k_flux_xyz, (bx + by + (long)nblocks((long)g.M * g.N * pz, 256)) * 256, g, c->p, dv, px, fy,
              pz, bx, by);
     return post("fluxes");
   }
@@ -1739,7 +1751,7 @@ int launch_end_stage(nhw_ctx *c, int istep) {
   const int mom = UVW_BLEND | (p.non_hydro ? UVW_PROJECT : 0) | istep << 8;
   const int slopes = !p.non_hydro && !p.viscous ? UVW_SLOPES : 0;
   if (wall_friction(p)) {
-    LAUNCH_R(KID_PROJECTION, k_momenta, g.neq(), g, p, dv, mom);
+    LAUNCH_R(KID_MOMENTA, k_momenta, g.neq(), g, p, dv, mom);
     return uvw_pass(c, UVW_DIVIDE | slopes);
   }
   return uvw_pass(c, UVW_DIVIDE | slopes | mom);
@@ -1747,7 +1759,7 @@ int launch_end_stage(nhw_ctx *c, int istep) {
 
 int launch_p_from_x(nhw_ctx *c, const double *x) {
   const Geo &g = c->g;
-  LAUNCH(KID_PROJECTION, k_p_from_x, g.neq(), g, x, c->d, zlayout(c));
+  LAUNCH(KID_P_FROM_X, k_p_from_x, g.neq(), g, x, c->d, zlayout(c));
   return post("poisson P");
 }
 
@@ -1756,7 +1768,7 @@ int launch_get_omega(nhw_ctx *c) {
   const int px = level_parts(g, flux_x_threads(g)), fy = row_faces(g);
   if (one_face_launch(c)) {
     const unsigned bx = nblocks(flux_x_threads(g, px), 256);
-    LAUNCH_R(KID_OMEGA_X, k_omega_xy, (bx + (long)nblocks(flux_y_threads(g, fy), 256)) * 256, g, c->p, dv, px, fy, bx);
+    LAUNCH_R(KID_OMEGA_XY, k_omega_xy, (bx + (long)nblocks(flux_y_threads(g, fy), 256)) * 256, g, c->p, dv, px, fy, bx);
   } else {
     LAUNCH_R(KID_OMEGA_X, k_omega_x, flux_x_threads(g, px), g, c->p, dv, px);
     LAUNCH_R(KID_OMEGA_Y, k_omega_y, flux_y_threads(g, fy), g, c->p, dv, fy);
@@ -1961,7 +1973,9 @@ int blaunch_eval_explicit(Batch *B, int istep) {
 
 // the plain members in their own form, the others in the general one
 static void blaunch_uvw_a(Batch *B, int flags) {
-  Timed t(B->lead, KID_UVW_A, bbytes(B, KID_UVW_A));
+  double bytes = 0.0;
+  for (nhw_ctx *c : B->m) bytes += uvw_bytes(c, flags);
+  Timed t(B->lead, KID_UVW_A, bytes);
   for (const bool plain : {true, false}) {
     const BShape &S = tuned(B, plain ? "lg" : "lx", BT_UVW_A);
     if (S.nblk == 0) continue;
@@ -1989,7 +2003,7 @@ int blaunch_end_stage(Batch *B, int istep) {
   bool friction = false;
   for (nhw_ctx *c : B->m) friction = friction || wall_friction(c->p);
   if (friction) {
-    BLAUNCH(KID_PROJECTION, kb_momenta, bshape(B, "c3/256"), mom);
+    BLAUNCH(KID_MOMENTA, kb_momenta, bshape(B, "c3/256"), mom);
     return buvw_pass(B, UVW_DIVIDE | slopes);
   }
   return buvw_pass(B, UVW_DIVIDE | slopes | mom);

@@ -394,12 +394,13 @@ struct Snap {
 
 // Kernels timed by the optional per-launch event instrumentation.
 enum KernelId {
-  KID_FLUX_X = 0, KID_FLUX_Y, KID_FLUX_Z, KID_EXPLICIT, KID_UVW_A, KID_UVW_B, KID_PROJECTION,
-  KID_RK_BLEND, KID_OMEGA_X, KID_OMEGA_Y, KID_OMEGA_COL, KID_DT, KID_MASK, KID_SOURCE,
+  KID_FLUX_X = 0, KID_FLUX_Y, KID_FLUX_Z, KID_EXPLICIT, KID_UVW_A, KID_UVW_B, KID_P_FROM_X,
+  KID_MOMENTA, KID_OMEGA_X, KID_OMEGA_Y, KID_OMEGA_COL, KID_DT, KID_MASK, KID_SOURCE,
   KID_ASSEMBLE, KID_SPMV_V, KID_SPMV_T, KID_RESID, KID_PREC_P, KID_PREC_S, KID_LINE_FACTOR,
-  KID_KUPDATE, KID_KREDUCE, KID_KMISC, KID_COPY, KID_RHS, KID_MF_V, KID_MF_T, KID_MF_RESID,
+  KID_KUPDATE, KID_KREDUCE, KID_KMISC, KID_BEGIN, KID_RHS, KID_MF_V, KID_MF_T, KID_MF_RESID,
   KID_MG_SETUP, KID_MG_DOWN, KID_MG_COARSE, KID_MG_UP, KID_KVEC, KID_WAVE_BC,
-  KID_SPONGE, KID_DIFFUSION, KID_VISC_SIGMA, KID_VISC_SOLVE, KID_KEPS, KID_COUNT
+  KID_SPONGE, KID_DIFFUSION, KID_VISC_SIGMA, KID_VISC_SOLVE, KID_KEPS, KID_FLUX_XYZ, KID_OMEGA_XY,
+  KID_MG_TAIL, KID_COUNT
 };
 
 struct KTimer {

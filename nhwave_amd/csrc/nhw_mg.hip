@@ -217,7 +217,7 @@ static void tail(nhw_ctx *c, const std::vector<MGLevel> &lvs, size_t l, const Mg
     A.l[a] = TailLevel<V>{make_lvl<V>(c, lv), g2<V>(lv), a ? (V *)lv.b : (V *)b, a ? (V *)lv.x : x, lv.fx, lv.fy};
     bytes += sizeof(V) * (3.0 * A.l[a].L.MN * A.l[a].L.K + 10.0 * A.l[a].L.MN);
   }
-  Timed t(c, KID_MG_COARSE, bytes);
+  Timed t(c, KID_MG_TAIL, bytes);
   by_rows<kMgKMax>(A.l[0].L.K, [&](auto km) {
     hipLaunchKernelGGL((k_mg_tail<V, decltype(km)::value, KIND>), dim3(1), dim3(kCoarseBS), 0, c->stream, A, in,
                        c->mg.coarse_sweeps, stop);

@@ -1414,7 +1414,7 @@ static int batch_poisson_t(Batch *B) {
   const BShape &rows = bshape(B, "c3/256"), &cols = bshape(B, "c2/256"), &one = bshape(B, "one");
   PBL(KID_MF_RESID, 0.0, kb_mf_true<R>, cols, part);
   PBL(KID_KREDUCE, 0.0, kb_fin<R>, one, cols.off, (const double *)part, 4);
-  PBL(KID_PROJECTION, 0.0, kb_p_from_x<R>, rows);
+  PBL(KID_P_FROM_X, 0.0, kb_p_from_x<R>, rows);
   PBL(KID_KMISC, 0.0, kb_gather_sc<R>, one, B->gsc, ns);
   int dummy = 0;
   if (bpoll(B, &dummy) < 0) return NHW_EHIP;  // also waits for the gather

@@ -52,12 +52,13 @@ void ktimer_flush(nhw_ctx *c) {
 
 const char *kernel_name(int kid) {
   static const char *names[KID_COUNT] = {
-      "k_flux_x", "k_flux_y", "k_flux_z", "k_eval_explicit", "k_uvw_a", "k_uvw_b", "k_projection",
-      "k_rk_blend", "k_omega_x", "k_omega_y", "k_omega_col", "k_dt_partial", "k_mask", "k_source_terms",
+      "k_flux_x", "k_flux_y", "k_flux_z", "k_eval_explicit", "k_uvw_a", "k_uvw_b", "k_p_from_x",
+      "k_momenta", "k_omega_x", "k_omega_y", "k_omega_col", "k_dt_partial", "k_mask", "k_source_terms",
       "k_assemble", "k_spmv_v", "k_spmv_t", "k_resid", "k_prec_p", "k_prec_s", "k_line_factor",
-      "k_update", "k_reduce_final", "k_krylov_misc", "k_copy", "k_rhs", "k_mf_apply_v", "k_mf_apply_t",
+      "k_update", "k_reduce_final", "k_krylov_misc", "k_begin", "k_rhs", "k_mf_apply_v", "k_mf_apply_t",
       "k_mf_resid0", "k_mg_setup", "k_mg_down", "k_coarse", "k_mg_up", "k_krylov_vec",
-      "k_wave_bc", "k_sponge", "k_diffusion", "k_visc_sigma", "k_visc_solve", "k_kepsilon"};
+      "k_wave_bc", "k_sponge", "k_diffusion", "k_visc_sigma", "k_visc_solve", "k_kepsilon",
+      "k_flux_xyz", "k_omega_xy", "k_mg_tail"};
   return (kid >= 0 && kid < KID_COUNT) ? names[kid] : "?";
 }
 
@@ -79,14 +80,22 @@ double kernel_bytes(const nhw_ctx *c, int kid) {
       return w3 * (3 * n + 4 * nfz);
     case KID_EXPLICIT:  // Ex..Hy, Fz..Hz, DU,DV,DW (r/w); D,D0,Hc,SourceX/Y,Mask; D,Eta,R1 written
       return w3 * (4 * nfx + 4 * nfy + 3 * nfz + 6 * n) + w * 9 * n2 + mi * n2;
-    case KID_UVW_A:  // DU,DV,DW -> U,V,W; face states and KBC 2-D
+    case KID_FLUX_XYZ:
+      return kernel_bytes(c, KID_FLUX_X) + kernel_bytes(c, KID_FLUX_Y) + kernel_bytes(c, KID_FLUX_Z);
+    case KID_UVW_A:  // DU,DV,DW -> U,V,W; face states and KBC 2-D (a pass that does more says so: uvw_bytes)
       return w3 * 6 * n + w * 12 * n2;
     case KID_UVW_B:  // 2-D slopes of the face states + 4 ghost layers of 6 fields
       return w * (8 * n2 + 12 * n2) + w3 * 24 * n2 + mi * n2;
-    case KID_PROJECTION:  // P, DU,DV,DW (r/w); D, DelxH/Eta, DelyH/Eta
-      return w * n + w3 * 6 * n + w * 5 * n2 + mi * n2;
-    case KID_RK_BLEND:  // DU0..DW0, DU..DW -> DU..DW
-      return w3 * 9 * n + w * n2 + mi * n2;
+    case KID_P_FROM_X:  // the solver's x -> P
+      return w * 2 * n;
+    case KID_MOMENTA:  // DU0..DW0, DU..DW -> DU..DW; with the projection P, DelxH/Eta, DelyH/Eta
+      return w3 * 9 * n + w * n2 + mi * n2 + (c->p.non_hydro ? w * (n + 4 * n2) : 0.0);
+    case KID_BEGIN: {  // DU,DV,DW, D, Eta -> DU0..Eta0, every cell; masks, Hc, wind
+      const double all2 = (double)g.Mloc * g.Nloc;
+      return w3 * 6 * all2 * g.Kloc + w * (4 * all2 + 3 * n2) + mi * 4 * n2;
+    }
+    case KID_OMEGA_XY:
+      return kernel_bytes(c, KID_OMEGA_X) + kernel_bytes(c, KID_OMEGA_Y);
     case KID_OMEGA_X:  // U, DU + Eta, D, Hfx -> Ex, EtaxL/R
       return w3 * (2 * n + nfx) + w * 5 * n2 + mi * n2;
     case KID_OMEGA_Y:
@@ -118,8 +127,8 @@ double kernel_bytes(const nhw_ctx *c, int kid) {
     case KID_MF_V:  // ph, rh -> v; 5 column fields
     case KID_MF_T:  // sh, s -> t
       return w * 3 * n + w * 5 * n2;
-    case KID_MF_RESID:  // x, b -> r, rh, p, v
-      return w * 6 * n + w * 5 * n2;
+    case KID_MF_RESID:  // x, b -> rh
+      return (w * 2 + w3) * n + w * 5 * n2;
     case KID_MG_SETUP:  // D, DelxH/Eta, DelyH/Eta -> 5 column fields (level 0)
       return w * 10 * n2;
     case KID_WAVE_BC:  // Hfx at the west face -> Ein, Din, Uin/Vin/Win per row
