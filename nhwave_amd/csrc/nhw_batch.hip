@@ -181,8 +181,8 @@ static int batch_build(Batch *B) {
   B->shapes.clear();
   B->ibuf_h.clear();
   B->kbuf_h.clear();
-  std::vector<long> fx, fy, fz, c2, c3, a2, a3, one, ex, lg[2];
-  std::vector<int> lgi[2];  // plain members of the velocity pass, the others
+  std::vector<long> fx, fy, fz, c2, c3, a2, a3, one, ex, lg[UVW_FORMS];
+  std::vector<int> lgi[UVW_FORMS];  // members by the form of their velocity pass
   int at = 0;
   for (nhw_ctx *c : B->m) {
     const Geo &g = c->g;
@@ -192,7 +192,7 @@ static int batch_build(Batch *B) {
     c2.push_back((long)g.M * g.N);
     c3.push_back(g.neq());
     ex.push_back((long)g.M * g.N * (c->p.viscous ? 1 : 1 + g.K));  // mass columns, momentum cells
-    const int form = uvw_plain(g, c->p) ? 0 : 1;
+    const int form = uvw_form(g, c->p);
     lg[form].push_back((long)g.M * g.N * level_groups(g));
     lgi[form].push_back(at++);
     a2.push_back(g.n2());
@@ -206,8 +206,7 @@ static int batch_build(Batch *B) {
     bshape_add(B, "fy" + s, fy, all, bs);
     bshape_add(B, "fz" + s, fz, all, bs);
     bshape_add(B, "c2" + s, c2, all, bs);
-    bshape_add(B, "lg" + s, lg[0], lgi[0], bs);
-    bshape_add(B, "lx" + s, lg[1], lgi[1], bs);
+    for (int f = 0; f < UVW_FORMS; ++f) bshape_add(B, "lg" + std::to_string(f) + s, lg[f], lgi[f], bs);
   }
   bshape_add(B, "c3/256", c3, all, 256);
   bshape_add(B, "ex/256", ex, all, 256);

@@ -701,25 +701,29 @@ __device__ __forceinline__ void blend_cell(const Par &p, int stage, int m, doubl
 // face states there, from values still in registers.  Projection, blend,
 // division and ghosts were a launch each, every one streaming the momenta
 // again, the last of them a thread per column (1024 x 1024 x 10: 182 + 137 +
-// 195 us, now 306; 333 x 217 x 7: 38 + 8, now 14).  Every load is issued before the first value is used: a
-// wait for memory, not the rate of the loads, is what a thread spends its
-// time on.  Rows go one by one with the groups of a row next to one another,
-// so that the pressures of neighbouring rows and levels are in the L2.
+// 195 us, now 306; 333 x 217 x 7: 38 + 8, now 14).  Every load is issued before
+// the first value is used: a wait for memory, not the rate of the loads, is what
+// a thread spends its time on.  Rows go one by one with the groups of a row next
+// to one another, so that the pressures of neighbouring rows and levels are in
+// the L2.
 //
-// MODE is the flags of a pass over walls that mirror (BC 1, 2); the general
-// form, MODE 0, takes them from `arg`, has inflow and friction sides too and
-// groups of three levels, which cost it a third of its wavefronts (registers).
-template <class R, int MODE>
+// MODE: the pass's flags but for the slopes.  ANY: sides of any kind, where the
+// plain form has walls that mirror (BC 1, 2).  NL: levels of a group at most, 3
+// where K is 3.  A form that can do more than a scenario needs holds registers for
+// it: three batched 700 x 600 x 4 with an inflow side 275 us (FP64) and 254 (float)
+// in a form for all flags, sides and groups (208 and 200 VGPRs), now 140 and 105;
+// three 700 x 700 x 3 between walls 231 and 214, now 146 and 112.
+template <class R, int MODE, int NL, bool ANY>
 __device__ __forceinline__ void uvw_a_body(const Geo &g, const Par &p, const DevT<R> &d, long t, int arg) {
-  constexpr int NL = MODE ? 2 : 3;
-  const int what = MODE ? MODE : arg;
-  const bool divide = what & UVW_DIVIDE, blend = what & UVW_BLEND, project = what & UVW_PROJECT;
+  constexpr bool three = NL == 3;
+  constexpr bool divide = MODE & UVW_DIVIDE, blend = MODE & UVW_BLEND, project = MODE & UVW_PROJECT;
+  constexpr bool friction = ANY && !blend && !project;  // with such sides k_momenta does those before
   const int stage = arg >> 8, ng = level_groups(g);
   const int i = g.Ibeg + (int)(t % g.M);
   const long r = t / g.M;
   const int grp = (int)(r % ng), j = g.Jbeg + (int)(r / ng);
   if (j > g.Jend) return;
-  const bool odd = g.K & 1, three = !MODE && g.K == 3;
+  const bool odd = g.K & 1;
   const int ka = g.Kbeg + 2 * grp - (odd && grp > 1), nk = three ? 3 : odd && grp == 1 ? 1 : 2;
   const long c = g.c2(i, j);
   const double Dd = d.D[c];
@@ -768,8 +772,7 @@ __device__ __forceinline__ void uvw_a_body(const Geo &g, const Par &p, const Dev
     }
   }
   // the velocity of interior cell q of column cq as this pass leaves it (a
-  // neighbour's own thread may be writing it: formed again, the same way; a
-  // pass that also projects or blends has no wall friction sides)
+  // neighbour's own thread may be writing it: formed again, the same way)
   auto vel = [&](const R *F, const R *DF, long q, long cq) -> double {
     return divide ? (double)(R)((double)DF[q] / d.D[cq]) : (double)F[q];
   };
@@ -788,19 +791,19 @@ __device__ __forceinline__ void uvw_a_body(const Geo &g, const Par &p, const Dev
   };
   // lateral ghosts, :4440-4761 (inflow at the west, :4468-4476)
   auto xghost = [&](int gi, int bc) {
-    if (!MODE && bc == 3 && gi > g.Iend) return;  // FLUX_LR's open east boundary: k_east_ghosts
+    if (ANY && bc == 3 && gi > g.Iend) return;  // FLUX_LR's open east boundary: k_east_ghosts
     const bool ns = bc == 2;
 #pragma unroll
     for (int n = 0; n < NL; ++n) {
       if (n >= nk) break;
       const int k = ka + n;
       const long gq = g.c3(gi, j, k);
-      if (!MODE && bc == 5) {
+      if (friction && bc == 5) {
         const int ib = gi < g.Ibeg ? g.Ibeg : g.Iend, far = gi < g.Ibeg ? g.Ibeg - gi : gi - g.Iend;
         const long cb = g.c2(ib, j), b = g.c3(ib, j, k);
         const double ph = wall_phi(p, d, g.dx, vel(d.V, d.DV, b, cb), vel(d.W, d.DW, b, cb), b);
         wall5(gq, n, ph, d.D[g.c2(far, j)], true);
-      } else if (!MODE && bc == 3) {
+      } else if (ANY && bc == 3) {
         const long b = inflow_idx(g, j, k);
         const double din = d.Din0[j - 1], uin = d.Uin0[b], vin = d.Vin0[b], win = d.Win0[b];
         d.U[gq] = (R)(2.0 * uin - (double)u[n]);
@@ -826,7 +829,7 @@ __device__ __forceinline__ void uvw_a_body(const Geo &g, const Par &p, const Dev
       if (n >= nk) break;
       const int k = ka + n;
       const long gq = g.c3(i, gj, k);
-      if (!MODE && bc == 5) {
+      if (friction && bc == 5) {
         const int jb = gj < g.Jbeg ? g.Jbeg : g.Jend, far = gj < g.Jbeg ? g.Jbeg - gj : gj - g.Jend;
         const long cb = g.c2(i, jb), b = g.c3(i, jb, k);
         const double ph = wall_phi(p, d, g.dy, vel(d.U, d.DU, b, cb), vel(d.W, d.DW, b, cb), b);
@@ -1448,9 +1451,9 @@ __global__ void k_p_from_x(Geo g, const double *__restrict__ x, Dev d, int zl) {
 // same XCD and found in its L2.  Measured per kernel at 1024x1024x10: it pays
 // for the projection (momenta; 176 -> 109 us) and the Omega column sweep (65 ->
 // 55 us) and costs the sigma-face fluxes (190 -> 225 us) and the y sweeps (99 ->
-// 104 and 240 -> 246 us); the others are unchanged.  The velocity pass takes
-// it for the largest grids (2048x2048x8 in float: 822 -> 735 us; 1024x1024x10: 318
-// -> 330).
+// 104 and 240 -> 246 us); the others are unchanged.  The velocity pass takes it
+// at every size: it gains 87 us on the largest grids (2048x2048x8 in float: 822 ->
+// 735) and loses 12 at 1024x1024x10 (318 -> 330).
 #define NHW_KERNELS(NAME, XCD)                                                                  \
   template <class R>                                                                            \
   __global__ __launch_bounds__(256) void k_##NAME(Geo g, Par p, DevT<R> d, int arg) {          \
@@ -1487,27 +1490,33 @@ __global__ __launch_bounds__(256) void k_omega_xy(Geo g, Par p, DevT<R> d, int p
 NHW_KERNELS(source_terms, 0)
 NHW_KERNELS(eval_explicit, 1)
 NHW_KERNELS(eta_slopes, 0)
-template <class R, int MODE>
+template <class R, int MODE, int NL, bool ANY>
 __global__ __launch_bounds__(256) void k_uvw_a(Geo g, Par p, DevT<R> d, int arg) {
-  uvw_a_body<R, MODE>(g, p, d, (long)xcd_block() * blockDim.x + threadIdx.x, arg);
+  uvw_a_body<R, MODE, NL, ANY>(g, p, d, (long)xcd_block() * blockDim.x + threadIdx.x, arg);
 }
-template <class R, int MODE>
+template <class R, int MODE, int NL, bool ANY>
 __global__ __launch_bounds__(256) void kb_uvw_a(BTab<R> T, int arg) {
   const BPos b = bfind(T);
   const BScn<R> &S = T.scn[b.s];
-  uvw_a_body<R, MODE>(S.g, S.p, S.d, b.b * blockDim.x + threadIdx.x, arg);
+  uvw_a_body<R, MODE, NL, ANY>(S.g, S.p, S.d, b.b * blockDim.x + threadIdx.x, arg);
 }
-// calls `run` with the mode (as an integral constant) of flags `f`; `plain`:
-// the scenario takes a mode of its own
+// calls `run` with the mode of flags `f`, the levels of a group and whether sides
+// may be of any kind (as integral constants) in a form (uvw_form)
 template <class Run>
-static void uvw_mode(int f, bool plain, Run run) {
+static void uvw_mode(int f, int form, Run run) {
   using std::integral_constant;
   constexpr int D = UVW_DIVIDE, DB = D | UVW_BLEND, DBP = DB | UVW_PROJECT;
-  const int what = f & DBP;
-  if (plain && what == D) run(integral_constant<int, D>());
-  else if (plain && what == DB) run(integral_constant<int, DB>());
-  else if (plain && what == DBP) run(integral_constant<int, DBP>());
-  else run(integral_constant<int, 0>());
+  auto mode = [&](auto nl, auto any) {
+    if ((f & DBP) == DBP) run(integral_constant<int, DBP>(), nl, any);
+    else if ((f & DB) == DB) run(integral_constant<int, DB>(), nl, any);
+    else run(integral_constant<int, D>(), nl, any);
+  };
+  auto sides = [&](auto nl) {
+    if (form & UVW_GENERAL) mode(nl, std::true_type());
+    else mode(nl, std::false_type());
+  };
+  if (form & UVW_THREE) sides(integral_constant<int, 3>());
+  else sides(integral_constant<int, 2>());
 }
 NHW_KERNELS(uvw_b, 0)
 NHW_KERNELS(momenta, 1)
@@ -1562,12 +1571,15 @@ static void launch_uvw_a(nhw_ctx *c, int flags) {
   const Geo &g = c->g;
   const long n = (long)g.M * g.N * level_groups(g);
   const double bytes = uvw_bytes(c, flags);
-  uvw_mode(flags, uvw_plain(g, c->p), [&](auto mode) {
-    if (c->mixed)
-      LAUNCH_B(KID_UVW_A, bytes, (k_uvw_a<float, decltype(mode)::value>), n, g, c->p, view<float>(c->d), flags);
-    else
-      LAUNCH_B(KID_UVW_A, bytes, (k_uvw_a<double, decltype(mode)::value>), n, g, c->p, c->d, flags);
-  });
+  auto run = [&](auto mode, auto nl, auto any) {
+    constexpr int MODE = decltype(mode)::value, NL = decltype(nl)::value;
+    constexpr bool ANY = decltype(any)::value;
+    if (c->mixed) LAUNCH_B(KID_UVW_A, bytes, (k_uvw_a<float, MODE, NL, ANY>), n, g, c->p, view<float>(c->d), flags);
+    else LAUNCH_B(KID_UVW_A, bytes, (k_uvw_a<double, MODE, NL, ANY>), n, g, c->p, c->d, flags);
+  };
+  if (flags & UVW_DIVIDE) uvw_mode(flags, uvw_form(g, c->p), run);
+  else if (g.K == 3) run(std::integral_constant<int, 0>(), std::integral_constant<int, 3>(), std::true_type());
+  else run(std::integral_constant<int, 0>(), std::integral_constant<int, 2>(), std::true_type());
 }
 
 int launch_initial(nhw_ctx *c) {
@@ -1971,20 +1983,22 @@ int blaunch_eval_explicit(Batch *B, int istep) {
   return bpost("batch eval_duvw");
 }
 
-// the plain members in their own form, the others in the general one
+// each member in its own form
 static void blaunch_uvw_a(Batch *B, int flags) {
   double bytes = 0.0;
   for (nhw_ctx *c : B->m) bytes += uvw_bytes(c, flags);
   Timed t(B->lead, KID_UVW_A, bytes);
-  for (const bool plain : {true, false}) {
-    const BShape &S = tuned(B, plain ? "lg" : "lx", BT_UVW_A);
+  for (int form = 0; form < UVW_FORMS; ++form) {
+    const BShape &S = tuned(B, ("lg" + std::to_string(form)).c_str(), BT_UVW_A);
     if (S.nblk == 0) continue;
-    uvw_mode(flags, plain, [&](auto mode) {
+    uvw_mode(flags, form, [&](auto mode, auto nl, auto any) {
+      constexpr int MODE = decltype(mode)::value, NL = decltype(nl)::value;
+      constexpr bool ANY = decltype(any)::value;
       if (B->mixed)
-        hipLaunchKernelGGL((kb_uvw_a<float, decltype(mode)::value>), dim3(S.nblk), dim3(S.bs), 0, B->lead->stream,
+        hipLaunchKernelGGL((kb_uvw_a<float, MODE, NL, ANY>), dim3(S.nblk), dim3(S.bs), 0, B->lead->stream,
                            btab<float>(B, S), flags);
       else
-        hipLaunchKernelGGL((kb_uvw_a<double, decltype(mode)::value>), dim3(S.nblk), dim3(S.bs), 0, B->lead->stream,
+        hipLaunchKernelGGL((kb_uvw_a<double, MODE, NL, ANY>), dim3(S.nblk), dim3(S.bs), 0, B->lead->stream,
                            btab<double>(B, S), flags);
     });
   }

@@ -212,9 +212,12 @@ inline bool mirror_walls(const Par &p) {
   return mirrors(p.bc_x0) && mirrors(p.bc_xn) && mirrors(p.bc_y0) && mirrors(p.bc_yn);
 }
 
-// the velocity pass has forms of its own (k_uvw_a) for mirroring walls and
-// groups of at most two levels
-inline bool uvw_plain(const Geo &g, const Par &p) { return mirror_walls(p) && g.K != 3; }
+// the form of the velocity pass (k_uvw_a) that a scenario takes: general or for
+// mirroring walls only, in groups of two levels at most or the one of three
+enum { UVW_GENERAL = 1, UVW_THREE = 2, UVW_FORMS = 4 };
+inline int uvw_form(const Geo &g, const Par &p) {
+  return (mirror_walls(p) ? 0 : UVW_GENERAL) | (g.K == 3 ? UVW_THREE : 0);
+}
 
 // Device pointers of the resident state.  R is the storage type of the 3-D
 // velocity/momentum fields, their stage copies, the face fluxes and Omega:
