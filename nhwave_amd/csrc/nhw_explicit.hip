@@ -155,7 +155,7 @@ __device__ __forceinline__ bool wave_speeds_r(int ml, int mr, double pl, double 
   return false;
 }
 
-template <class R>
+template <class R, class DS>
 __device__ __forceinline__ void flux_x_body(const Geo &g, const Par &p, const DevT<R> &d, long t, int arg) {
   const int wpr = (g.M + 1 + kXFaces - 1) / kXFaces;  // wavefronts per row
   // arg: parts the levels are split into (0: one); a part's wavefronts follow
@@ -229,7 +229,7 @@ __device__ __forceinline__ void flux_x_body(const Geo &g, const Par &p, const De
 
     double E = 0.0, F = 0.0, G = 0.0, H = 0.0, sL, sR;
     if (wave_speeds_r(ml, mr, pl, pr, uL, uR, sL, sR)) {
-      const Quot ds(sR - sL);
+      const DS ds(sR - sL);
       E = hll(sL, sR, ds, duL, duR, DL, DR);
       F = hll(sL, sR, ds, duL * uL + PL, duR * uR + PR, duL, duR);
       G = hll(sL, sR, ds, DL * uL * vL, DR * uR * vR, dvL, dvR);
@@ -1466,7 +1466,20 @@ __global__ void k_p_from_x(Geo g, const double *__restrict__ x, Dev d, int zl) {
     const BScn<R> &S = T.scn[b.s];                                                              \
     NAME##_body<R>(S.g, S.p, S.d, b.b * blockDim.x + threadIdx.x, arg);                         \
   }
-NHW_KERNELS(flux_x, 0)
+// The x faces of a batch, whose pointers come from its table, have no registers
+// left for the shared divisor: with it the float form takes 104, four wavefronts a
+// SIMD, and without it 96, five (three members of 700 x 700 x 3: 134 us, now 114;
+// FP64, 116 either way: 161, now 162).
+template <class R>
+__global__ __launch_bounds__(256) void k_flux_x(Geo g, Par p, DevT<R> d, int arg) {
+  flux_x_body<R, Quot>(g, p, d, (long)blockIdx.x * blockDim.x + threadIdx.x, arg);
+}
+template <class R>
+__global__ __launch_bounds__(256, sizeof(R) == 4 ? 5 : 4) void kb_flux_x(BTab<R> T, int arg) {
+  const BPos b = bfind(T);
+  const BScn<R> &S = T.scn[b.s];
+  flux_x_body<R, double>(S.g, S.p, S.d, b.b * blockDim.x + threadIdx.x, arg);
+}
 NHW_KERNELS(flux_y, 0)
 NHW_KERNELS(flux_z, 0)
 // The face kernels of a small grid in one launch, a range of workgroups each:
@@ -1477,7 +1490,7 @@ template <class R>
 __global__ __launch_bounds__(256) void k_flux_xyz(Geo g, Par p, DevT<R> d, int px, int fy, int pz, unsigned bx,
                                                   unsigned by) {
   const long b = blockIdx.x;
-  if (b < bx) flux_x_body<R>(g, p, d, b * 256 + threadIdx.x, px);
+  if (b < bx) flux_x_body<R, Quot>(g, p, d, b * 256 + threadIdx.x, px);
   else if (b < bx + by) flux_y_body<R>(g, p, d, (b - bx) * 256 + threadIdx.x, fy);
   else flux_z_body<R>(g, p, d, (b - bx - by) * 256 + threadIdx.x, pz);
 }
