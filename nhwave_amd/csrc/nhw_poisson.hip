@@ -194,7 +194,7 @@ __global__ void k_line_factor(KV k) {
 // levels: 13.6 us with a thread a column in memory, now 6.3 to 7, the
 // reduction before it (3.2 us by itself) included; 9 to 10 with the levels of a
 // column in one lane's registers, whose code alone is 24 KB read once.
-// Columns too long for the LDS walk in memory.
+// Columns too long for the LDS, or too many of them, walk in memory.
 constexpr int kLineBS = 256;
 constexpr int kLineCols = 16;           // columns a workgroup, fewer of long ones
 constexpr long kLineLds = 64 * 1024;    // bytes
@@ -203,9 +203,18 @@ inline int line_cols(int K) {
   while (nc > 1 && 4L * sizeof(double) * nc * K > kLineLds) nc /= 2;
   return nc;
 }
-inline size_t line_lds(int K) {
+// LDS of a workgroup of a launch over `columns`, 0: columns walk in memory.  A
+// launch of many columns has wavefronts enough to hide the waits, and there the
+// detour through the LDS costs more, the sooner the shorter the columns are.  An
+// iteration in LDS and in memory: 128^2 x 4 52 us and 51, 256^2 x 4 89 and 81, 1024^2 x 4
+// 799 and 607; 256^2 x 8 115 and 118, 362^2 x 8 191 and 179, 1024^2 x 8 1337 and 1184;
+// 256^2 x 32 378 and 406, 362^2 x 32 723 and 675.
+constexpr int kLineShort = 8;  // levels
+constexpr long kLineManyShort = 16384, kLineMany = 98304;
+inline size_t line_lds(int K, long columns) {
   const long bytes = 4L * sizeof(double) * line_cols(K) * K;
-  return bytes > kLineLds ? 0 : bytes;
+  const bool many = columns > (K < kLineShort ? kLineManyShort : kLineMany);
+  return many || bytes > kLineLds ? 0 : bytes;
 }
 
 // rows that a thread has in flight at once
@@ -856,7 +865,7 @@ int poisson_solve(nhw_ctx *c) {
   { Timed _t(c, KID_ASSEMBLE); hipLaunchKernelGGL((k_assemble<true, double>), dim3(nb), dim3(kBS), 0, st, g, c->d, kr.coef, kr.rhs); }
   const KV k = make_kv(c);
   const Off15 o = stencil(g);
-  const size_t lds = line_lds(k.K);
+  const size_t lds = line_lds(k.K, k.MN);
   const int nc = lds ? line_cols(k.K) : 0, per = nc ? nc : kLineBS;  // columns a workgroup
   const unsigned ncol = (unsigned)((k.MN + per - 1) / per);
   const int nblk = kr.nblk, fin = nblk <= kFuseParts ? nblk : 0;

@@ -18,7 +18,8 @@ iteration's vectors formed in them, up to 131072 rows, and given; the same in 28
 tiles, where four rows or fewer leave 32768 columns room; levels halved along
 one axis; and narrow grids, whose cycle one workgroup ends.  Line: TOL 1e-6,
 columns 16 and fewer a workgroup in LDS (128 and 129 levels are either side of
-16 and 8), in memory (2049), and more rows than scalars are formed in line for."""
+16 and 8), in memory (2049 levels; more than 16384 columns of few levels, 98304
+of eight or more), and more rows than scalars are formed in line for."""
 import json
 
 import pytest
