@@ -20,7 +20,7 @@
 // and bilinear prolongation.  One V(1,1)-cycle from a zero guess is a fixed
 // linear operator, used as the right preconditioner of BiCGStab.  The
 // 15-point stencil has no (+-1,+-1) x-y couplings, so columns of one colour
-// are independent and a half sweep is one parallel launch.
+// are independent and update in parallel.
 #include <algorithm>
 #include <vector>
 

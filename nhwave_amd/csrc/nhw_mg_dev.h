@@ -634,12 +634,12 @@ __device__ __forceinline__ Pro<V> pro_at(int Mc, int Nc, int fx, int fy, int i, 
 //
 // Each colour's values pass between the half sweeps through LDS.
 //
-// Bound on large levels by the FP64 instruction rate and the three waves a
-// SIMD that 150 VGPRs leave, on small ones by the elimination's chain of
-// dependent operations.  Measured, FP64, a level's whole cycle: 1024 x 1024 x
-// 10 162 us (sweep by sweep 195), 512 x 512 54 (68), 64 x 64 22 in two
-// launches (34 in six); a V-cycle of the 1024 x 1024 x 10 hierarchy 304 us
-// (385).
+// Bound on large levels by waits that the three waves a SIMD left by 150 VGPRs
+// do not cover (1024 x 1024 x 10: 3.6 and 2.9 TB/s up and down, the VALU 40 to
+// 52 % busy), on small ones by the elimination's chain of dependent operations.
+// Measured, FP64, a level's whole cycle: 1024 x 1024 x 10 162 us (sweep by sweep
+// 195), 512 x 512 54 (68), 64 x 64 22 in two launches (34 in six); a V-cycle of
+// the 1024 x 1024 x 10 hierarchy 304 us (385).
 template <int TX, int TY>
 struct MgTile {
   static_assert(TX % 2 == 0 && TY % 2 == 0, "tiles start on even columns and whole coarse cells");

@@ -996,8 +996,8 @@ __global__ __launch_bounds__(256) void kb_geom_coarsen(BTab<R> T, int l) {
   ((R *)Cq.by)[h] = (R)(a[3] * w); ((R *)Cq.rd)[h] = (R)(a[4] * w);
 }
 
-// FP64 residual of the FP64 solution into the Krylov vectors (e = 0 in the
-// mixed form); partials (r,r), (b,b).  One thread walks one column.
+// FP64 residual of the FP64 solution into rh; partials (r,r), (b,b).  One
+// thread walks one column.
 template <class R>
 __global__ __launch_bounds__(256) void kb_mf_init(BTab<R> T, double *part) {
   const BPos b = bfind(T);
